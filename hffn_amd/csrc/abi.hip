@@ -662,6 +662,38 @@ int hffn_plan_gemv(int value_type, const void* up_planes, const int32_t* up_bina
     return HFFN_OK;
 }
 
+// -------------------------------------------------------------------------------- planes densified per call
+
+int hffn_prefill_workspace(int value_type, uint32_t n, uint32_t d_model, uint32_t d_ff, uint64_t* bytes) {
+    if (!bytes) return fail(HFFN_ERROR_ARGUMENT, "prefill_workspace: null result");
+    if (int status = check_shape(d_model, d_ff, n, (n + 3) / 4 * 4)) return status;
+    if (!valid_value_type(value_type)) return fail(HFFN_ERROR_ARGUMENT, "unknown value type %d", value_type);
+    if (d_ff % 8 != 0) return fail(HFFN_ERROR_ARGUMENT, "prefill: d_ff=%u must be a multiple of 8", d_ff);
+    *bytes = hffn::prefill_workspace_bytes(value_type, n, d_model, d_ff);
+    return HFFN_OK;
+}
+
+int hffn_forward_prefill(int value_type, const float* x, const int32_t* up_offsets, const int16_t* up_idx, const void* up_val,
+                         const float* b_up, const int32_t* out_offsets, const int16_t* out_hidden, const void* out_val,
+                         const float* b_down, void* workspace, uint64_t workspace_bytes, float* y, uint32_t d_model, uint32_t d_ff,
+                         uint32_t n, void* stream) {
+    uint64_t needed = 0;
+    if (int status = hffn_prefill_workspace(value_type, n, d_model, d_ff, &needed)) return status;
+    if (!x || !up_offsets || !up_idx || !up_val || !b_up || !out_offsets || !out_hidden || !out_val || !b_down || !workspace || !y)
+        return fail(HFFN_ERROR_ARGUMENT, "forward_prefill: null pointer");
+    for (const void* p : {static_cast<const void*>(x), static_cast<const void*>(b_up), static_cast<const void*>(b_down),
+                          static_cast<const void*>(y)})
+        if (reinterpret_cast<uintptr_t>(p) % 16 != 0)
+            return fail(HFFN_ERROR_ARGUMENT, "forward_prefill: x, y and the biases must be 16-byte aligned");
+    if (reinterpret_cast<uintptr_t>(workspace) % 256 != 0)
+        return fail(HFFN_ERROR_ARGUMENT, "forward_prefill: the workspace must be 256-byte aligned");
+    if (workspace_bytes < needed)
+        return fail(HFFN_ERROR_ARGUMENT, "forward_prefill: workspace of %llu bytes, %llu needed for n=%u",
+                    static_cast<unsigned long long>(workspace_bytes), static_cast<unsigned long long>(needed), n);
+    const hffn::PrefillCall call{x, up_offsets, up_idx, up_val, b_up, out_offsets, out_hidden, out_val, b_down, workspace, y, d_model, d_ff, n};
+    return launched(hffn::launch_prefill(value_type, call, static_cast<hipStream_t>(stream)), "forward_prefill");
+}
+
 // ----------------------------------------------------------------------------------------------------- training
 
 int hffn_forward_z(int up_mode, int down_mode, const float* x, const int32_t* up_offsets, const int16_t* up_idx, const float* up_val,

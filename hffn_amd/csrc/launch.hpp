@@ -95,6 +95,26 @@ hipError_t launch_mfma_up_planes(int vt, const void* planes, const int32_t* w_ex
 hipError_t launch_mfma_down(int vt, const void* planes, const int32_t* v_exp, const float* b_down, float* y, void* workspace,
                             uint32_t n, uint32_t d, uint32_t h, hipStream_t stream);
 
+// A whole forward on planes densified for the call (mfma.hip): layers without planes of their own, calls above the
+// decode sizes. d a multiple of 16, h of 8, distinct ascending indices per row; x token-major [n, d], 16-byte aligned,
+// b_up and b_down 16-byte aligned, the workspace (prefill_workspace_bytes) 256-byte aligned and of any content.
+struct PrefillCall {
+    const float* x;
+    const int32_t* up_off;
+    const int16_t* up_idx;
+    const void* up_val;
+    const float* b_up;
+    const int32_t* down_off;
+    const int16_t* down_idx;
+    const void* down_val;
+    const float* b_down;
+    void* workspace;
+    float* y;
+    uint32_t d, h, n;
+};
+uint64_t prefill_workspace_bytes(int vt, uint32_t n, uint32_t d, uint32_t h);
+hipError_t launch_prefill(int vt, const PrefillCall& call, hipStream_t stream);
+
 // Sampled products of the training backward on the streamed GEMM (mfma.hip): the dense G = A B^T over the tokens,
 // then the support's entries and the bias gradient (A [rows, ld], B [cols, ld] row-major, n real columns).
 // grad_dense_workspace_bytes is 0 for shapes the streamed GEMM does not take.

@@ -114,14 +114,15 @@ __device__ __forceinline__ size_t plane_at(uint32_t rows, uint32_t row, uint32_t
 // whose range is one chunk keeps its values in registers, longer ranges are read again (from L2).
 constexpr uint32_t kSplitBlockRows = 8;
 constexpr uint32_t kSplitChunk = 256;  // k per chunk: 4 steps of 64
-__global__ __launch_bounds__(kThreads) void split_rows_kernel(const float* __restrict__ x, uint32_t M, uint32_t rows_pad,
-                                                             uint32_t K, uint32_t ld, uint32_t k_real, _Float16* __restrict__ planes,
-                                                             int32_t* __restrict__ e) {
-    constexpr uint32_t kWaves = kThreads / kWave;
-    __shared__ uint32_t part[kWaves][kSplitBlockRows];
-    const uint32_t lane = threadIdx.x % kWave, wave = uniform(threadIdx.x / kWave);
+constexpr uint32_t kSplitWaves = kThreads / kWave;
+// The work of kThreads threads (tid) on row group `group`; part: their maxima in LDS. Every thread of the block calls it.
+__device__ __forceinline__ void split_rows(uint32_t (&part)[kSplitWaves][kSplitBlockRows], uint32_t tid, uint32_t group,
+                                           const float* __restrict__ x, uint32_t M, uint32_t rows_pad, uint32_t K, uint32_t ld,
+                                           uint32_t k_real, _Float16* __restrict__ planes, int32_t* __restrict__ e) {
+    constexpr uint32_t kWaves = kSplitWaves;
+    const uint32_t lane = tid % kWave, wave = uniform(tid / kWave);
     const uint32_t r = lane % kSplitBlockRows, piece = lane / kSplitBlockRows;
-    const uint32_t row = blockIdx.x * kSplitBlockRows + r;
+    const uint32_t row = group * kSplitBlockRows + r;
     const uint32_t span = K / kWaves, k_begin = wave * span, k_end = k_begin + span;
     const float* src = x + static_cast<size_t>(row) * ld;
     const bool real = row < M;
@@ -188,104 +189,184 @@ __global__ __launch_bounds__(kThreads) void split_rows_kernel(const float* __res
         }
     }
 }
+__global__ __launch_bounds__(kThreads) void split_rows_kernel(const float* __restrict__ x, uint32_t M, uint32_t rows_pad,
+                                                             uint32_t K, uint32_t ld, uint32_t k_real, _Float16* __restrict__ planes,
+                                                             int32_t* __restrict__ e) {
+    __shared__ uint32_t part[kSplitWaves][kSplitBlockRows];
+    split_rows(part, threadIdx.x, blockIdx.x, x, M, rows_pad, K, ld, k_real, planes, e);
+}
 
 // --------------------------------------------------------------------------------------------- densify
 // Row n of the dense matrix (a neuron of W_up, or an output of W_down^T) has its slots [off[n], off[n+1]) at columns
 // idx[] (distinct within a row; the host checks it); densifying writes the whole row of both planes (zeros outside
-// the support) and its binade. A block takes kDensRows consecutive rows and kDensChunk columns (blockIdx.y): the rows'
+// the support) and its binade. A block takes kDensRows consecutive rows and kDensChunk columns: the rows'
 // maxima (two waves per row, over all their slots), then their hi/lo parts in its columns assembled in LDS (zeroed
 // meanwhile, then each slot of the chunk in its column) and written out whole: for every 16-byte chunk run the block's rows are
 // kDensRows consecutive 16-byte pieces, one 128-byte line per (run, row group). The rows are padded by 16 bytes in
 // LDS so that the eight rows of a chunk fall in different banks; the tile (66 KB) leaves room for two blocks per CU.
 constexpr uint32_t kDensRows = 8, kDensChunk = 2048, kDensThreads = 1024, kDensPad = 8;
+// Slots [8 q, 8 q + 8) of the compact rows: one 16-byte load of their indices, one (float32: two) of their values. vec:
+// idx and val start on 16-byte boundaries.
 template <typename V>
-__global__ __launch_bounds__(kDensThreads) void densify_kernel(const int32_t* __restrict__ off, const int16_t* __restrict__ idx,
-                                                              const V* __restrict__ val, uint32_t rows, uint32_t k,
-                                                              _Float16* __restrict__ planes, int32_t* __restrict__ exps) {
-    const auto value = [&](int32_t s) { return widen(val[s]); };
+struct SlotPiece {
+    static constexpr int kVals = 2 * static_cast<int>(sizeof(V));
+    uint32_t ids[4], vals[kVals];
+    __device__ __forceinline__ void load(const int16_t* __restrict__ idx, const V* __restrict__ val, int32_t q, int32_t nnz, bool vec) {
+        const int32_t s = 8 * q;
+        if (vec && s + 8 <= nnz) {
+            const uint4 i4 = *reinterpret_cast<const uint4*>(idx + s);
+            ids[0] = i4.x; ids[1] = i4.y; ids[2] = i4.z; ids[3] = i4.w;
+#pragma unroll
+            for (int p = 0; p < kVals; p += 4) {
+                const uint4 v4 = reinterpret_cast<const uint4*>(val + s)[p / 4];
+                vals[p] = v4.x; vals[p + 1] = v4.y; vals[p + 2] = v4.z; vals[p + 3] = v4.w;
+            }
+            return;
+        }
+        // unaligned arrays, or the piece across the end of the arrays: slot by slot, those past nnz zero
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ids[i] = 0;
+#pragma unroll
+        for (int i = 0; i < kVals; ++i) vals[i] = 0;
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (s + u < nnz) {
+                ids[u / 2] |= static_cast<uint32_t>(static_cast<uint16_t>(idx[s + u])) << (16 * (u % 2));
+                if constexpr (sizeof(V) == 2) vals[u / 2] |= static_cast<uint32_t>(val[s + u]) << (16 * (u % 2));
+                else vals[u] = __float_as_uint(val[s + u]);
+            }
+    }
+    __device__ __forceinline__ uint32_t index(int u) const { return u % 2 ? ids[u / 2] >> 16 : ids[u / 2] & 0xffffu; }
+    __device__ __forceinline__ float value(int u) const {
+        if constexpr (sizeof(V) == 2) return __uint_as_float(u % 2 ? vals[u / 2] & 0xffff0000u : vals[u / 2] << 16);
+        else return __uint_as_float(vals[u]);
+    }
+};
+
+// The slots [begin, end) of one row on two waves (half h of them), in pieces of 8 on 8-slot boundaries, 64 pieces at a
+// time in turn (lane l of half h: pieces first + 128 q). The first piece of a lane is requested at construction and held;
+// those of rows of more than 1016 slots are read at each pass.
+template <typename V>
+struct RowSlots {
+    static constexpr int32_t kStride = 2 * kWave;
+    const int16_t* idx;
+    const V* val;
+    int32_t begin, end, first, last, nnz;
+    bool vec;
+    SlotPiece<V> held;
+    __device__ __forceinline__ RowSlots(const int16_t* __restrict__ i, const V* __restrict__ v, int32_t b, int32_t e, int32_t slots, bool aligned,
+                                        uint32_t half, uint32_t lane)
+        : idx(i), val(v), begin(b), end(e), first((b >> 3) + static_cast<int32_t>(half * kWave + lane)), last(e > b ? (e + 7) >> 3 : 0),
+          nnz(slots), vec(aligned) {
+        if (first < last) held.load(idx, val, first, nnz, vec);
+    }
+    // f(index, value, inside the row) of every slot of the lane's pieces
+    template <typename F>
+    __device__ __forceinline__ void each(const F& f) const {
+        if (first >= last) return;
+        piece(held, first, f);
+        for (int32_t q = first + kStride; q < last; q += kStride) {
+            SlotPiece<V> p;
+            p.load(idx, val, q, nnz, vec);
+            piece(p, q, f);
+        }
+    }
+    template <typename F>
+    __device__ __forceinline__ void piece(const SlotPiece<V>& p, int32_t q, const F& f) const {
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            f(p.index(u), p.value(u), static_cast<uint32_t>(8 * q + u - begin) < static_cast<uint32_t>(end - begin));
+    }
+};
+struct DensTile {
+    _Float16 tile[2][kDensRows][kDensChunk + kDensPad];
+    uint32_t row_max[2][kDensRows];
+};
+struct DensSide {
+    const int32_t* off;
+    const int16_t* idx;
+    const void* val;
+    uint32_t rows, rows_pad, k;  // real rows; rows and columns of the planes
+    bool vec;
+    _Float16* planes;
+    int32_t* exps;
+};
+// A side's blocks: (row group, column chunk), chunk-major.
+constexpr uint32_t dens_blocks(uint32_t rows_pad, uint32_t k) { return (rows_pad + kDensRows - 1) / kDensRows * ((k + kDensChunk - 1) / kDensChunk); }
+constexpr uint32_t kDensOccupancy = 8;  // waves per SIMD of two blocks: at most 64 VGPRs
+
+// PARTS 1 (bfloat16 planes of one call): the hi plane alone, the only one its GEMMs read. Rows `rows` .. rows_pad - 1 and
+// columns past the indices are zeros.
+template <typename V, uint32_t PARTS>
+__device__ __forceinline__ void densify(DensTile& lds, const DensSide& side, uint32_t block) {
     static_assert(kDensRows * 16 == 128, "a row group's pieces of one chunk run fill one 128-byte line");
-    __shared__ __attribute__((aligned(16))) _Float16 tile[2][kDensRows][kDensChunk + kDensPad];
-    __shared__ uint32_t row_max[2][kDensRows];
-    constexpr uint32_t kWaves = kDensThreads / kWave;
-    static_assert(kWaves == 2 * kDensRows, "two waves per row");
+    auto& tile = lds.tile;
+    auto& row_max = lds.row_max;
+    static_assert(kDensThreads / kWave == 2 * kDensRows, "two waves per row");
     const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = uniform(tid / kWave);
     const uint32_t row = wave % kDensRows, half = wave / kDensRows;  // wave-uniform
-    const uint32_t r0 = blockIdx.x * kDensRows, n = r0 + row;
-    const uint32_t c0 = blockIdx.y * kDensChunk;
-    const uint32_t width = min(kDensChunk, k - c0), pieces = width / 8;  // width: a multiple of 32
-    // the block's tile zeroed while the slots are in flight
-    for (uint32_t i = tid; i < 2 * kDensRows * pieces; i += kDensThreads) {
-        const uint32_t part = i / (kDensRows * pieces), rr = (i / pieces) % kDensRows, j = i % pieces;
-        *reinterpret_cast<uint4*>(&tile[part][rr][j * 8]) = make_uint4(0, 0, 0, 0);
-    }
-    // Waves w and w + kDensRows take row r0 + w, slots interleaved by 64 (lane l of half h: begin + 64 h + l + 128 q).
-    // A row of at most kHeld slots per lane is read once, into registers, for both its maximum and its scatter; a
-    // longer row is read twice, kBatch slots per lane in flight. The two halves' maxima meet in LDS.
-    constexpr int kHeld = 16, kBatch = 16, kStride = 2 * kWave;
-    const int32_t begin = n < rows ? off[n] : 0, end = n < rows ? off[n + 1] : 0;
-    const int32_t first = begin + static_cast<int32_t>(half * kWave + lane);
-    const bool held = end - begin <= kHeld * kStride;  // wave-uniform
-    uint32_t hc[kHeld];
-    float hw[kHeld];
+    const uint32_t groups = (side.rows_pad + kDensRows - 1) / kDensRows, chunk = block / groups;
+    const uint32_t r0 = block % groups * kDensRows, n = r0 + row, c0 = chunk * kDensChunk;
+    const uint32_t width = min(kDensChunk, side.k - c0), pieces = width / 8;  // width: a multiple of 32
+    // Waves w and w + kDensRows take row r0 + w. The two halves' maxima meet in LDS.
+    const bool real = n < side.rows;
+    RowSlots<V> slots(side.idx, static_cast<const V*>(side.val), real ? side.off[n] : 0, real ? side.off[n + 1] : 0, side.off[side.rows],
+                      side.vec, half, lane);
+    // the tile zeroed while the slots are in flight
+    for (uint32_t i = tid; i < PARTS * sizeof(tile[0]) / 16; i += kDensThreads) reinterpret_cast<uint4*>(tile)[i] = make_uint4(0, 0, 0, 0);
     uint32_t m = 0;
-    if (held) {
-#pragma unroll
-        for (int q = 0; q < kHeld; ++q) {
-            const int32_t s = first + q * kStride;
-            const bool in = s < end;
-            hc[q] = in ? static_cast<uint16_t>(idx[s]) : 0xFFFFFFFFu;
-            hw[q] = in ? value(s) : 0.0f;
-        }
-#pragma unroll
-        for (int q = 0; q < kHeld; ++q) m = max(m, abs_bits(hw[q]));
-    } else {
-        // a batch's loads all issued before the first is used: a slot past the row reads the row's last slot again
-        // (a value of the row: the maximum is unchanged)
-        for (int32_t s0 = first; s0 < end; s0 += kBatch * kStride) {
-            float w[kBatch];
-#pragma unroll
-            for (int q = 0; q < kBatch; ++q) w[q] = value(min(s0 + q * kStride, end - 1));
-#pragma unroll
-            for (int q = 0; q < kBatch; ++q) m = max(m, abs_bits(w[q]));
-        }
-    }
+    slots.each([&](uint32_t, float v, bool inside) { m = max(m, inside ? abs_bits(v) : 0u); });
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) m = max(m, static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), o, kWave)));
     if (lane == 0) row_max[half][row] = m;
     __syncthreads();  // the tile is zeroed, the halves' maxima are in
     const int e = binade_of_bits(max(row_max[0][row], row_max[1][row]));
-    const auto place = [&](uint32_t c, float w) {
-        if (c < c0 || c >= c0 + width) return;  // another column block's slot, or past the row
+    slots.each([&](uint32_t column, float v, bool inside) {
+        // a slot of another row or column block goes to the row's padding, which nothing reads: no branch per slot
+        const uint32_t c = column - c0, at = inside && c < width ? c : kDensChunk;
         _Float16 hi, lo;
-        split(ldexpf(w, -e), hi, lo);
-        tile[0][row][c - c0] = hi;
-        tile[1][row][c - c0] = lo;
-    };
-    if (held) {
-#pragma unroll
-        for (int q = 0; q < kHeld; ++q) place(hc[q], hw[q]);
-    } else {
-        for (int32_t s0 = first; s0 < end; s0 += kBatch * kStride) {
-            uint32_t c[kBatch];
-            float w[kBatch];
-#pragma unroll
-            for (int q = 0; q < kBatch; ++q) {  // past the row: its last slot again (placed again, the same cell and value)
-                const int32_t at = min(s0 + q * kStride, end - 1);
-                c[q] = static_cast<uint16_t>(idx[at]);
-                w[q] = value(at);
-            }
-#pragma unroll
-            for (int q = 0; q < kBatch; ++q) place(c[q], w[q]);
-        }
-    }
+        split(ldexpf(v, -e), hi, lo);
+        tile[0][row][at] = hi;
+        if constexpr (PARTS == 2) tile[1][row][at] = lo;
+    });
     __syncthreads();
-    for (uint32_t i = tid; i < 2 * pieces * kDensRows; i += kDensThreads) {
-        const uint32_t rr = i % kDensRows, j = (i / kDensRows) % pieces, part = i / (kDensRows * pieces);
-        if (r0 + rr < rows)
-            *reinterpret_cast<uint4*>(planes + plane_at(rows, r0 + rr, c0 + j * 8, part)) =
-                *reinterpret_cast<const uint4*>(&tile[part][rr][j * 8]);
-    }
-    if (blockIdx.y == 0 && half == 0 && lane == 0 && n < rows) exps[n] = e;
+    // thread t: row t % 8, pieces t / 8, t / 8 + 128, ... of every part (no division by the width: two per 16 bytes moved
+    // cost more than the moves)
+    const uint32_t rr = tid % kDensRows;
+    if (r0 + rr < side.rows_pad)
+        for (uint32_t j = tid / kDensRows; j < pieces; j += kDensThreads / kDensRows)
+#pragma unroll
+            for (uint32_t part = 0; part < PARTS; ++part)
+                *reinterpret_cast<uint4*>(side.planes + plane_at(side.rows_pad, r0 + rr, c0 + j * 8, part)) =
+                    *reinterpret_cast<const uint4*>(&tile[part][rr][j * 8]);
+    if (chunk == 0 && half == 0 && lane == 0 && n < side.rows_pad) side.exps[n] = e;
+}
+template <typename V>
+__global__ __launch_bounds__(kDensThreads, kDensOccupancy) void densify_kernel(DensSide side) {
+    __shared__ __attribute__((aligned(16))) DensTile lds;
+    densify<V, 2>(lds, side, blockIdx.x);
+}
+
+// What a call that densifies its own planes (launch_prefill) needs before its first GEMM, in one launch: the planes of
+// both sides from the compact rows and the input planes of x. Blocks 0 .. up_blocks - 1 densify W_up, the next
+// down_blocks W_down, the last split x, kSplitGroups groups of 8 rows a block. MI355X, at 128 / 2048 tokens: 9.9 / 7.4 us
+// on 512 x 2048 at 20 % (float32), 17.9 / 15.2 on 1024 x 4096 at 10 %, 38 / 46 on 2048 x 8192 at 20 % (bfloat16; 72 with
+// single slots a lane in place of 8, 2-byte loads). A block is a chain of four round trips (offsets, slots, LDS, stores).
+constexpr uint32_t kSplitGroups = kDensThreads / kThreads;
+template <typename V>
+__global__ __launch_bounds__(kDensThreads, kDensOccupancy) void prefill_prep_kernel(DensSide up, DensSide down, uint32_t up_blocks,
+                                                                                   uint32_t down_blocks, const float* __restrict__ x,
+                                                                                   uint32_t M, uint32_t rows_pad, uint32_t K, uint32_t ld,
+                                                                                   _Float16* __restrict__ planes, int32_t* __restrict__ e) {
+    constexpr uint32_t kParts = sizeof(V) == 2 ? 1 : 2;
+    __shared__ __attribute__((aligned(16))) DensTile lds;
+    if (blockIdx.x < up_blocks) return densify<V, kParts>(lds, up, blockIdx.x);
+    if (blockIdx.x < up_blocks + down_blocks) return densify<V, kParts>(lds, down, blockIdx.x - up_blocks);
+    using Parts = uint32_t[kSplitGroups][kSplitWaves][kSplitBlockRows];
+    Parts& parts = reinterpret_cast<Parts&>(lds);
+    const uint32_t g = uniform(threadIdx.x / kThreads);
+    split_rows(parts[g], threadIdx.x % kThreads, (blockIdx.x - up_blocks - down_blocks) * kSplitGroups + g, x, M, rows_pad, K, ld, ld,
+               planes, e);
 }
 
 // ------------------------------------------------------------------------------------------------ GEMM
@@ -648,11 +729,33 @@ __device__ __forceinline__ void block_barrier() {
     asm volatile("" ::: "memory");
 }
 
+// Waits until at most min(R, later) stages of L transfers each are in flight: the wave's oldest have landed.
+template <int R, int L>
+__device__ __forceinline__ void wait_stages(uint32_t later) {
+    if constexpr (R == 0) wait_loads<0>();
+    else if (later >= static_cast<uint32_t>(R)) wait_loads<R * L>();
+    else wait_stages<R - 1, L>(later);
+}
+
 // LIVE < BM (one row tile of up to LIVE tokens): only the first LIVE rows of A are transferred and multiplied; the
 // waves whose rows are all padding only transfer and meet at the barriers. The live rows get the same
 // products in the same order as with LIVE = BM, and the padding rows' accumulators stay zero, as zero A rows leave
 // them, so the results are bitwise those of the full tile.
-template <Epi EPI, bool LO_B, int LIVE>
+//
+// CHAIN > 0 (the calls whose planes are densified per call, which stand in for the compact store's paths): the MFMA
+// accumulators run over CHAIN k-tiles only, then are added to a second set of float32 sums (Down: brought from the
+// activation block's power of two to 1 on the way, exact, in place of the rescale) and start from zero again. One
+// chain of MFMAs over all of K loses 6.5e-7 of the result (2048 x 8192 at 20 %, bfloat16, 1999 tokens, against 64 bits),
+// three times as much as the tiles path it stands in for (2.05e-7); in chains of one activation block it keeps 2.0e-7, for
+// ~4 % of the GEMMs' time.
+//
+// BM < 256 (those calls too): row tiles of 128 (waves of 32 x 64) or 64 (32 x 32), where 256 rows by 128 columns leave
+// CUs idle or would have to be split over K, with the partials' round trip and another launch. A k-tile of such a tile
+// is multiplied faster than its transfer arrives, so the ring holds as many stages as LDS takes. 768 x 3072 (float32) at
+// 512 tokens: up projection 18.2 + 6.4 us in 3 splits of 256 rows and their activation pass, 17.6 us with 64 rows (no
+// split); down 18.7 -> 14.6 us.
+constexpr int dma_stages(int bm) { return bm == 64 ? 6 : bm == 128 ? 4 : kDmaStages; }
+template <Epi EPI, bool LO_B, int LIVE, int CHAIN, int BM = kDmaBM>
 __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
     const _Float16* __restrict__ a_planes,  // [K / 32][8][rows_pad][8]
     const int32_t* __restrict__ a_exp,      // Up: [rows_pad]; Down: [K / kActBlock, rows_pad] (act_exp_at)
@@ -664,19 +767,22 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
     int32_t* __restrict__ out_exp,          // Up: [Ncol / BN, rows_pad] activation block binades (act_exp_at)
     uint32_t M, uint32_t rows_pad, uint32_t Ncol, uint32_t K, uint32_t splits,
     uint32_t whole_n,                       // Down: column tiles below whole_n take all of K and write y into `out`
-    float* __restrict__ part) {             // Down, whole_n > 0: the other column tiles' partials [splits, M, Ncol - whole_n BN]
-    // 8 waves in 4 x 2, 64 x 64 outputs each (two waves per SIMD)
-    constexpr int W = kDmaWaves, MI = 2, NI = 2, BM = kDmaBM, BN = kDmaBN, S = kDmaStages;
-    constexpr uint32_t kT = 64 * W, kWaveRows = 32 * MI, kHalf = W / 2;
-    static_assert(kWaveRows * (W / 2) == BM, "the waves cover the block's rows");
-    static_assert(kHalf * kWave == BM, "the upper half of the waves holds a thread per block row");
+    float* __restrict__ part,               // Down, whole_n > 0: the other column tiles' partials [splits, M, Ncol - whole_n BN]
+    uint32_t cols) {                        // real columns (<= Ncol, a multiple of 4): biases and y end there
+    // 256 rows: 8 waves in 4 x 2, 64 x 64 outputs each (two waves per SIMD)
+    constexpr int W = kDmaWaves, MI = BM == kDmaBM ? 2 : 1, NI = BM == 64 ? 1 : 2, BN = kDmaBN, S = dma_stages(BM);
+    constexpr uint32_t kT = 64 * W, kWaveRows = 32 * MI, kWaveCols = 32 * NI, kWavesN = BN / kWaveCols;
+    static_assert(kWaveRows * (W / kWavesN) == BM, "the waves cover the block's rows");
+    static_assert(BM == kDmaBM || (CHAIN > 0 && LIVE == BM), "narrower row tiles: whole ones, in chains");
+    constexpr bool FOLD = CHAIN > 0;
+    static_assert(!FOLD || EPI != Epi::Down || CHAIN == static_cast<int>(kKtPerActBlock), "a down chain has one power of two per row");
     static_assert(LIVE == BM || LIVE == 128 || LIVE == 64, "live rows: the whole tile, its first half or first quarter");
     constexpr uint32_t kStage = kRuns * (BM + BN) * 8;  // halves per stage
     // Down: the activation binades of up to kDmaMaxActBlocks blocks sit in e_tab; with bfloat16 weights the B lo plane of
     // every ring slot (8 KB, never transferred) holds 32 blocks more, so that a tile can take all of a wide K
     constexpr uint32_t kLoRegion = kRuns * BM * 8 + kRuns / 2 * BN * 8, kLoRuns = kRuns / 2 * BN * 8 * 2 / BM;
-    constexpr uint32_t kMaxActBlocks = LO_B ? kDmaMaxActBlocks : kDmaMaxActBlocks + S * kLoRuns;
-    static_assert(kLoRuns == kDmaLoRuns, "the host's plan counts the ring's spare runs alike");
+    constexpr uint32_t kMaxActBlocks = LO_B || BM != kDmaBM ? kDmaMaxActBlocks : kDmaMaxActBlocks + S * kLoRuns;
+    static_assert(BM != kDmaBM || kLoRuns == kDmaLoRuns, "the host's plan counts the ring's spare runs alike");
     constexpr int kRowRuns = LIVE / 64;                  // 64-row runs of A transferred per (part, chunk)
     // runs of B transferred per k-tile: both planes, or the hi plane alone when the lo plane is not read (LO_B false)
     constexpr int kRunsB = LO_B ? kRuns : kRuns / 2;
@@ -693,16 +799,16 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
     // Down: the BM binades of the k range's activation block c (c < kMaxActBlocks): a row of e_tab, or a 256-byte run in
     // the unused B lo plane of ring slot (c - kDmaMaxActBlocks) / kLoRuns
     const auto etab = [&](uint32_t c) -> int8_t* {
-        if (LO_B || c < kDmaMaxActBlocks) return &e_tab[c][0];
+        if (LO_B || BM != kDmaBM || c < kDmaMaxActBlocks) return &e_tab[c][0];
         const uint32_t o = c - kDmaMaxActBlocks;
         return reinterpret_cast<int8_t*>(smem + (o / kLoRuns) * kStage + kLoRegion) + (o % kLoRuns) * BM;
     };
 
     const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = uniform(tid / kWave);
-    const uint32_t wm = wave / 2, wn = wave % 2;
+    const uint32_t wm = wave / kWavesN, wn = wave % kWavesN;
     // wave-uniform: this wave's rows hold tokens (a constant for a full tile)
     const bool live = LIVE == BM || wm * kWaveRows < static_cast<uint32_t>(LIVE);
-    const uint32_t tiles_m = rows_pad / BM, tiles_n = Ncol / BN;
+    const uint32_t tiles_m = (M + BM - 1) / BM, tiles_n = Ncol / BN;
     // the first tiles_m * whole_n blocks: column tiles 0 .. whole_n - 1 over all of K (one round of long blocks first);
     // the others: the remaining column tiles, K split `splits` ways (whole_n 0: every tile split alike)
     const uint32_t whole_blocks = tiles_m * whole_n;
@@ -712,7 +818,9 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
     const uint32_t nsplit = whole ? 1 : splits;
     const uint32_t m0 = tile.m * BM, n0 = tile.n * BN;
     const uint32_t ktiles = K / kBK;
-    const uint32_t k_begin = tile.split * ktiles / nsplit, k_end = (tile.split + 1) * ktiles / nsplit;
+    // K split on k-tiles (Down: on activation blocks)
+    constexpr uint32_t kUnit = EPI == Epi::Down ? kKtPerActBlock : 1;
+    const uint32_t k_begin = tile.split * (ktiles / kUnit) / nsplit * kUnit, k_end = (tile.split + 1) * (ktiles / kUnit) / nsplit * kUnit;
     const uint32_t kb0 = k_begin / kKtPerActBlock;
 
     // piece q of wave w's share of a stage: a run of 64 rows (1 KB) of A (pieces below kLoadsA), then of B; its
@@ -758,26 +866,27 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
         const uint32_t blocks = (k_end - k_begin) / kKtPerActBlock;  // at least one: K is split on activation blocks
         const int8_t* tab = act_exps(a_exp);
         for (uint32_t c = wave; c < blocks; c += W)
-            dma4(tab + act_exp_at(rows_pad, m0, kb0 + c), lane * 4, etab(c));
+            if (lane < BM / 4) dma4(tab + act_exp_at(rows_pad, m0, kb0 + c), lane * 4, etab(c));
     } else {
-        if (wave == 0) dma16(a_exp + m0, lane * 16, &e_row[0][0]);
+        if (wave == 0 && lane < BM / 4) dma16(a_exp + m0, lane * 16, &e_row[0][0]);
     }
 #pragma unroll
     for (int s = 0; s < S; ++s)
         if (static_cast<uint32_t>(s) < steps) issue(k_begin + s, s);
     // stage k_begin has landed (later stages may be in flight), and with it the binades; then the block meets
-    if (steps >= 3) wait_loads<2 * kLoads>();
-    else if (steps == 2) wait_loads<kLoads>();
-    else wait_loads<0>();
+    wait_stages<S - 1, kLoads>(steps - 1);
     block_barrier();
 
-    floatx16 acc[MI][NI];
+    floatx16 acc[MI][NI], sum[FOLD ? MI : 1][FOLD ? NI : 1];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < NI; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+            for (int r = 0; r < 16; ++r) {
+                acc[i][j][r] = 0.0f;
+                if constexpr (FOLD) sum[i][j][r] = 0.0f;
+            }
 
     // operand fragments of one 16-wide k step (chunk pair kk of a k-tile)
     struct Frags {
@@ -796,7 +905,7 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
         }
 #pragma unroll
         for (int j = 0; j < NI; ++j) {
-            const uint32_t r = wn * (BN / 2) + j * 32 + lane % 32;
+            const uint32_t r = wn * kWaveCols + j * 32 + lane % 32;
             f.bh[j] = *reinterpret_cast<const half8*>(s_b + (chunk * BN + r) * 8);
             if constexpr (LO_B) f.bl[j] = *reinterpret_cast<const half8*>(s_b + ((4 + chunk) * BN + r) * 8);
         }
@@ -850,8 +959,35 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
     // wave changes it (lane l checks the wave's row l; binades are multiples of kActBinadeStep, so changes are rare;
     // checked here rather than for all blocks after the prologue, which measured 0.5 % slower); accumulator registers
     // 4g .. 4g + 3 hold 4 consecutive rows, so one 4-byte read per block and group
+    // the chain that ends before k-tile kt, into the float32 sums
+    const auto fold = [&](uint32_t kt) {
+        if constexpr (FOLD) {
+            if (!live) return;
+            const uint32_t kb = (kt - 1) / kKtPerActBlock - kb0;
+#pragma unroll
+            for (int i = 0; i < MIL; ++i)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    uint32_t e = 0;
+                    if constexpr (EPI == Epi::Down)
+                        e = *reinterpret_cast<const uint32_t*>(etab(kb) + wave_row<kWaveRows>(wm, i, 4 * g, lane));
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) {
+                        const float f = EPI == Epi::Down ? ldexpf(1.0f, static_cast<int8_t>(e >> (8 * b))) : 1.0f;
+#pragma unroll
+                        for (int j = 0; j < NI; ++j) {
+                            const int r = 4 * g + b;
+                            sum[i][j][r] = EPI == Epi::Down ? fmaf(acc[i][j][r], f, sum[i][j][r]) : sum[i][j][r] + acc[i][j][r];
+                            acc[i][j][r] = 0.0f;
+                        }
+                    }
+                }
+        }
+    };
     const auto rescale = [&](uint32_t kt) {
-        if constexpr (EPI == Epi::Down) {
+        if constexpr (FOLD) {
+            if ((kt - k_begin) % CHAIN == 0 && kt != k_begin) fold(kt);
+        } else if constexpr (EPI == Epi::Down) {
             const uint32_t kb = kt / kKtPerActBlock - kb0;
             if (kt % kKtPerActBlock != 0 || kt == k_begin || !live) return;
             const uint32_t own = wm * kWaveRows + lane;
@@ -896,8 +1032,7 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
         load(f1, slot, 1);
         __builtin_amdgcn_sched_barrier(0);
         multiply(f0);
-        if (kt + 2 < k_end) wait_loads<kLoads>();  // stage kt + 1 has landed, kt + 2 may be in flight
-        else wait_loads<0>();
+        wait_stages<S - 2, kLoads>(k_end - kt - 2);  // stage kt + 1 has landed, the S - 2 after it may be in flight
         wait_loads<63>();  // the same LDS wait on every path, where the compiler's wait tracking sees it
         block_barrier();
         load(f0, (it + 1) % S, 0);
@@ -912,7 +1047,12 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
     __builtin_amdgcn_sched_barrier(0);
     multiply(f0);
     multiply(f1);
+    fold(k_end);
     __syncthreads();
+    const auto result = [&](int i, int j, int r) -> float {
+        if constexpr (FOLD) return sum[i][j][r];
+        else return acc[i][j][r];
+    };
 
     if constexpr (EPI == Epi::Up) {
         // v = gelu(z + b) once per element into an fp32 [BM][BN] tile in LDS; then thread t takes block row t: the
@@ -923,19 +1063,20 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
         float* tile_v = reinterpret_cast<float*>(smem);
 #pragma unroll
         for (int j = 0; j < NI; ++j) {
-            const uint32_t c = wn * (BN / 2) + j * 32 + lane % 32;
+            const uint32_t c = wn * kWaveCols + j * 32 + lane % 32;
             const int ce = b_exp[n0 + c];
-            const float cb = bias[n0 + c];
+            const float cb = n0 + c < cols ? bias[n0 + c] : 0.0f;  // a padding neuron: gelu(0) = 0
 #pragma unroll
             for (int i = 0; i < MI; ++i)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const uint32_t m = wave_row<kWaveRows>(wm, i, r, lane);
-                    tile_v[m * kLd + c] = gelu(ldexpf(acc[i][j][r], e_row[0][m] + ce) + cb);
+                    const float z = ldexpf(result(i, j, r), e_row[0][m] + ce) + cb;
+                    tile_v[m * kLd + c] = FOLD ? gelu_near(z) : gelu(z);
                 }
         }
         __syncthreads();
-        // H threads per block row (1 with 4 waves, 2 with 8: lanes h of a row are adjacent), each a BN / H-wide part
+        // H threads per block row (2 with 256 rows, 4 with fewer: lanes h of a row are adjacent), each a BN / H-wide part
         constexpr uint32_t H = kT / BM;
         const uint32_t row = tid / H, part = tid % H;
         const float* row_v = tile_v + row * kLd;
@@ -976,33 +1117,38 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
         const uint32_t kb_last = (k_end - 1) / kKtPerActBlock - kb0;
         // the last activation block's binades held in a ring slot (a wide k range), which the tile below overwrites,
         // are first copied to e_row (block-uniform condition)
-        const bool last_in_ring = EPI == Epi::Down && kb_last >= kDmaMaxActBlocks;
+        const bool last_in_ring = EPI == Epi::Down && !FOLD && kb_last >= kDmaMaxActBlocks;
         if (last_in_ring) {
             if (tid < BM) e_row[0][tid] = etab(kb_last)[tid];
             __syncthreads();
         }
 #pragma unroll
         for (int j = 0; j < NI; ++j) {
-            const uint32_t c = wn * (BN / 2) + j * 32 + lane % 32;
+            const uint32_t c = wn * kWaveCols + j * 32 + lane % 32;
             const int ce = b_exp[n0 + c];
 #pragma unroll
             for (int i = 0; i < MI; ++i)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const uint32_t m = wave_row<kWaveRows>(wm, i, r, lane);
-                    const int ea = EPI == Epi::Down && !last_in_ring ? static_cast<int>(e_tab[kb_last][m]) : e_row[0][m];
-                    tile_v[m * kLd + c] = ldexpf(acc[i][j][r], ea + ce);
+                    // (a folded down sum is in units of 1 already)
+                    const int ea = EPI != Epi::Down || last_in_ring ? e_row[0][m] : FOLD ? 0 : static_cast<int>(e_tab[kb_last][m]);
+                    tile_v[m * kLd + c] = ldexpf(result(i, j, r), ea + ce);
                 }
         }
         __syncthreads();
         // y (whole k range) or this split's partial: [splits, M, Ncol], or with whole_n > 0 [splits, M, Ncol - whole_n BN]
         // over the split column tiles only
-        const uint32_t ld = nsplit > 1 && whole_n > 0 ? Ncol - whole_n * BN : Ncol, c0 = n0 - (ld == Ncol ? 0 : whole_n * BN);
+        // (y: the real columns only; partials: the padded ones as well)
+        const bool apart = nsplit > 1 && whole_n > 0, is_y = EPI == Epi::Down && nsplit == 1;
+        const uint32_t ld = apart ? Ncol - whole_n * BN : is_y ? cols : Ncol, c0 = n0 - (apart ? whole_n * BN : 0);
         float* target = nsplit == 1 ? out : (whole_n > 0 ? part : out) + static_cast<size_t>(tile.split) * M * ld;
+        const uint32_t c_end = is_y ? cols - min(cols, n0) : BN;
         const bool add_bias = EPI == Epi::Down && nsplit == 1 && bias != nullptr;  // no bias: the training gx product
         for (uint32_t q = tid; q < BM * (BN / 4); q += kT) {
             const uint32_t m = q / (BN / 4), c = (q % (BN / 4)) * 4;
             if (m0 + m >= M) break;  // rows ascend with q
+            if (c >= c_end) continue;
             float4 v = *reinterpret_cast<const float4*>(tile_v + m * kLd + c);
             if (add_bias) {
                 const float4 b = *reinterpret_cast<const float4*>(bias + n0 + c);
@@ -1014,14 +1160,14 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
 }
 
 // y[m, c0 + c] = sum over splits (in split order) of partials[s, m, c] + bias[c0 + c] for the partials' width columns
-// (y rows of Ncol); 4 columns per thread.
+// below cols (y rows of cols); 4 columns per thread, kReduceRows rows x 256 columns per block.
+constexpr uint32_t kReduceRows = 4;
 __global__ __launch_bounds__(kThreads) void reduce_splits_kernel(const float* __restrict__ partials, const float* __restrict__ bias,
-                                                                float* __restrict__ y, uint32_t M, uint32_t Ncol, uint32_t splits,
-                                                                uint32_t width, uint32_t c0) {
-    const size_t quads = static_cast<size_t>(M) * width / 4;
-    const size_t i = static_cast<size_t>(blockIdx.x) * kThreads + threadIdx.x;
-    if (i >= quads) return;
-    const size_t m = i / (width / 4), c = c0 + (i % (width / 4)) * 4;
+                                                                float* __restrict__ y, uint32_t M, uint32_t splits, uint32_t width,
+                                                                uint32_t c0, uint32_t cols) {
+    const uint32_t m = blockIdx.x * kReduceRows + threadIdx.x / 64, quad = blockIdx.y * 64 + threadIdx.x % 64, c = c0 + quad * 4;
+    if (m >= M || quad * 4 >= width || c >= cols) return;
+    const size_t quads = static_cast<size_t>(M) * (width / 4), i = static_cast<size_t>(m) * (width / 4) + quad;
     const float4* p = reinterpret_cast<const float4*>(partials);
     float4 t = p[i];
     for (uint32_t s0 = 1; s0 < splits; s0 += 8) {  // 8 loads in flight, added in split order
@@ -1039,7 +1185,7 @@ __global__ __launch_bounds__(kThreads) void reduce_splits_kernel(const float* __
         const float4 b = *reinterpret_cast<const float4*>(bias + c);
         t.x += b.x; t.y += b.y; t.z += b.z; t.w += b.w;
     }
-    *reinterpret_cast<float4*>(y + m * Ncol + c) = t;
+    *reinterpret_cast<float4*>(y + static_cast<size_t>(m) * cols + c) = t;
 }
 
 // Activation planes from the up GEMM's k-split partial sums (Epi::UpSplit): v = gelu(sum over the splits, in split
@@ -1048,12 +1194,18 @@ __global__ __launch_bounds__(kThreads) void reduce_splits_kernel(const float* __
 // gemm_dma_kernel<Up> writes them. A wave takes 4 rows of one 128-neuron block: 16 lanes per row, 8 consecutive
 // neurons per lane (one 16-byte chunk per part); the block's maximum is a 16-lane xor butterfly.
 constexpr uint32_t kActRowsPerBlock = kThreads / 16;
+template <bool NEAR>  // gelu_near
 __global__ __launch_bounds__(kThreads) void act_planes_kernel(const float* __restrict__ partials, uint32_t splits,
                                                              const float* __restrict__ b_up, _Float16* __restrict__ planes,
-                                                             int8_t* __restrict__ exps, uint32_t M, uint32_t rows_pad, uint32_t H) {
+                                                             int8_t* __restrict__ exps, uint32_t M, uint32_t rows_pad, uint32_t H,
+                                                             uint32_t cols) {
     const uint32_t m = blockIdx.x * kActRowsPerBlock + threadIdx.x / 16, sub = threadIdx.x % 16;
     const uint32_t nb = blockIdx.y, n = nb * kActBlock + sub * 8;
-    const float4 b0 = *reinterpret_cast<const float4*>(b_up + n), b1 = *reinterpret_cast<const float4*>(b_up + n + 4);
+    float4 b0 = make_float4(0.f, 0.f, 0.f, 0.f), b1 = b0;
+    if (n < cols) {  // a multiple of 8: whole pieces
+        b0 = *reinterpret_cast<const float4*>(b_up + n);
+        b1 = *reinterpret_cast<const float4*>(b_up + n + 4);
+    }
     float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (m < M) {
         for (uint32_t s0 = 0; s0 < splits; s0 += 4) {  // 8 loads in flight, added in split order
@@ -1077,7 +1229,7 @@ __global__ __launch_bounds__(kThreads) void act_planes_kernel(const float* __res
     uint32_t largest = 0;
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
-        v[q] = gelu(v[q] + b[q]);
+        v[q] = NEAR ? gelu_near(v[q] + b[q]) : gelu(v[q] + b[q]);
         largest = max(largest, abs_bits(v[q]));
     }
 #pragma unroll
@@ -1401,14 +1553,39 @@ hipError_t launch_dma(const _Float16* a_planes, const int32_t* a_exp, const _Flo
     const dim3 grid(tiles_m * whole_n + tiles_m * (tiles_n - whole_n) * splits), block(64 * kDmaWaves);
     const uint32_t rows_pad = rows_padded(M), live = rows_live(M);
     if (live == 64)
-        hipLaunchKernelGGL((gemm_dma_kernel<EPI, LO_B, 64>), grid, block, 0, stream, a_planes, a_exp, b_planes, b_exp, bias, out,
-                           out_planes, out_exp, M, rows_pad, Ncol, K, splits, whole_n, part);
+        hipLaunchKernelGGL((gemm_dma_kernel<EPI, LO_B, 64, 0>), grid, block, 0, stream, a_planes, a_exp, b_planes, b_exp, bias, out,
+                           out_planes, out_exp, M, rows_pad, Ncol, K, splits, whole_n, part, Ncol);
     else if (live == 128)
-        hipLaunchKernelGGL((gemm_dma_kernel<EPI, LO_B, 128>), grid, block, 0, stream, a_planes, a_exp, b_planes, b_exp, bias, out,
-                           out_planes, out_exp, M, rows_pad, Ncol, K, splits, whole_n, part);
+        hipLaunchKernelGGL((gemm_dma_kernel<EPI, LO_B, 128, 0>), grid, block, 0, stream, a_planes, a_exp, b_planes, b_exp, bias, out,
+                           out_planes, out_exp, M, rows_pad, Ncol, K, splits, whole_n, part, Ncol);
     else
-        hipLaunchKernelGGL((gemm_dma_kernel<EPI, LO_B, kDmaBM>), grid, block, 0, stream, a_planes, a_exp, b_planes, b_exp, bias, out,
-                           out_planes, out_exp, M, rows_pad, Ncol, K, splits, whole_n, part);
+        hipLaunchKernelGGL((gemm_dma_kernel<EPI, LO_B, kDmaBM, 0>), grid, block, 0, stream, a_planes, a_exp, b_planes, b_exp, bias, out,
+                           out_planes, out_exp, M, rows_pad, Ncol, K, splits, whole_n, part, Ncol);
+    return hipGetLastError();
+}
+
+// The chained GEMMs: row tiles of bm (64, 128 or 256) tokens, K split `splits` ways.
+template <Epi EPI, bool LO_B, int CHAIN>
+hipError_t launch_chained(uint32_t bm, const _Float16* a_planes, const int32_t* a_exp, const _Float16* b_planes, const int32_t* b_exp,
+                          const float* bias, float* out, _Float16* out_planes, int32_t* out_exp, uint32_t M, uint32_t Ncol, uint32_t K,
+                          uint32_t splits, uint32_t cols, hipStream_t stream) {
+    const dim3 grid(ceil_div(M, bm) * (Ncol / kDmaBN) * splits);
+    const uint32_t rows_pad = rows_padded(M);
+#define HFFN_CHAINED(BM)                                                                                                          \
+    hipLaunchKernelGGL((gemm_dma_kernel<EPI, LO_B, BM, CHAIN, BM>), grid, dim3(64 * kDmaWaves), 0, stream, a_planes, a_exp, b_planes, \
+                       b_exp, bias, out, out_planes, out_exp, M, rows_pad, Ncol, K, splits, 0u, static_cast<float*>(nullptr), cols)
+    if (bm == 64) HFFN_CHAINED(64);
+    else if (bm == 128) HFFN_CHAINED(128);
+    else HFFN_CHAINED(256);
+#undef HFFN_CHAINED
+    return hipGetLastError();
+}
+
+// y = the split partials [splits, M, width] of columns c0 .. c0 + width - 1, added in split order, plus the bias.
+hipError_t launch_reduce_splits(const float* partials, const float* bias, float* y, uint32_t M, uint32_t splits, uint32_t width, uint32_t c0,
+                                uint32_t cols, hipStream_t stream) {
+    hipLaunchKernelGGL(reduce_splits_kernel, dim3(ceil_div(M, kReduceRows), ceil_div(width, 256)), dim3(kThreads), 0, stream, partials, bias, y,
+                       M, splits, width, c0, cols);
     return hipGetLastError();
 }
 
@@ -1423,11 +1600,8 @@ hipError_t dma_down(DownPlan plan, const _Float16* a_planes, const int32_t* a_ex
                          : launch_dma<Epi::Down, LO_B>(a_planes, a_exp, b_planes, b_exp, bias, partials, nullptr, nullptr, M, Ncol, K,
                                                        plan.splits, stream);
     if (status != hipSuccess) return status;
-    const uint32_t c0 = plan.whole_n * kDmaBN, width = Ncol - c0;
-    const size_t quads = static_cast<size_t>(M) * width / 4;
-    hipLaunchKernelGGL(reduce_splits_kernel, dim3(static_cast<uint32_t>((quads + kThreads - 1) / kThreads)), dim3(kThreads), 0, stream,
-                       partials, bias, y, M, Ncol, plan.splits, width, c0);
-    return hipGetLastError();
+    const uint32_t c0 = plan.whole_n * kDmaBN;
+    return launch_reduce_splits(partials, bias, y, M, plan.splits, Ncol - c0, c0, Ncol, stream);
 }
 
 // Workspace layout (int32 words unless stated; rows = M padded to kRowPad): split counters [down tiles of the
@@ -1543,15 +1717,18 @@ hipError_t launch_grad_dense(const float* row, const float* mat, const int32_t* 
 
 size_t mfma_workspace_bytes(uint32_t n, uint32_t d, uint32_t h) { return workspace_layout(n, d, h).bytes; }
 
+namespace {
+bool slots_aligned(const void* idx, const void* val) {
+    return reinterpret_cast<uintptr_t>(idx) % 16 == 0 && reinterpret_cast<uintptr_t>(val) % 16 == 0;
+}
+}  // namespace
+
 hipError_t launch_densify(int vt, const int32_t* off, const int16_t* idx, const void* val, uint32_t rows, uint32_t k,
                           void* planes, int32_t* exps, hipStream_t stream) {
-    const dim3 grid(ceil_div(rows, kDensRows), ceil_div(k, kDensChunk)), block(kDensThreads);
-    if (vt == kBF16)
-        hipLaunchKernelGGL((densify_kernel<uint16_t>), grid, block, 0, stream, off, idx, static_cast<const uint16_t*>(val), rows, k,
-                           static_cast<_Float16*>(planes), exps);
-    else
-        hipLaunchKernelGGL((densify_kernel<float>), grid, block, 0, stream, off, idx, static_cast<const float*>(val), rows, k,
-                           static_cast<_Float16*>(planes), exps);
+    const dim3 grid(dens_blocks(rows, k)), block(kDensThreads);
+    const DensSide side{off, idx, val, rows, rows, k, slots_aligned(idx, val), static_cast<_Float16*>(planes), exps};
+    if (vt == kBF16) hipLaunchKernelGGL((densify_kernel<uint16_t>), grid, block, 0, stream, side);
+    else hipLaunchKernelGGL((densify_kernel<float>), grid, block, 0, stream, side);
     return hipGetLastError();
 }
 
@@ -1586,8 +1763,8 @@ hipError_t launch_mfma_up_planes(int vt, const void* planes, const int32_t* w_ex
                         : launch_dma<Epi::UpSplit, true>(x_planes, words + w.x_binades, p, w_exp, nullptr, partials, nullptr, nullptr, n,
                                                          h, d, splits, stream);
         if (status != hipSuccess) return status;
-        hipLaunchKernelGGL(act_planes_kernel, dim3(rows_live(n) / kActRowsPerBlock, h / kActBlock), dim3(kThreads), 0, stream, partials,
-                           splits, b_up, act_planes, reinterpret_cast<int8_t*>(words + w.act_binades), n, rows_padded(n), h);
+        hipLaunchKernelGGL(act_planes_kernel<false>, dim3(rows_live(n) / kActRowsPerBlock, h / kActBlock), dim3(kThreads), 0, stream, partials,
+                           splits, b_up, act_planes, reinterpret_cast<int8_t*>(words + w.act_binades), n, rows_padded(n), h, h);
         return hipGetLastError();
     }
     if (dma_tiles(n, h) >= kDmaMinBlocks) {
@@ -1624,6 +1801,144 @@ hipError_t launch_mfma_down(int vt, const void* planes, const int32_t* v_exp, co
                                       words + w.counters, n, d, h, stream);
     return gemm<Epi::Down, true>(shape, act_planes, words + w.act_binades, p, v_exp, b_down, y, nullptr, nullptr, partials,
                                  words + w.counters, n, d, h, stream);
+}
+
+// ------------------------------------------------------------------------------ planes densified per call
+// A call above the decode sizes on a layer without planes of its own: the planes of both sides are densified from the
+// compact rows into the call's workspace (one launch, with the split of x), then the streamed GEMMs run on them as on a
+// layer's own. Widths are padded to multiples of 256 (zero rows and columns; biases and y end at the real ones). The
+// GEMMs run in chains of one activation block, the float32 up projection in half of one: its three MFMAs per step make
+// chains of 128 k as long as the sums over them (error against 64 bits, 1024 x 4096 shape at 2048 tokens: 2.48e-7 ->
+// 2.38e-7; the bfloat16 1.4B shape the other way, 2.16e-7 -> 2.23e-7). Calls above kPrefillPiece tokens run in pieces over the
+// same planes, which bounds the workspace.
+constexpr uint32_t kPrefillPiece = 16384;
+constexpr int kPrefillDownChain = kKtPerActBlock;
+constexpr uint32_t kPrefillDownBlocks = 16;  // activation blocks of a down split: longer sums lose more than the tiles path
+constexpr uint32_t pad256(uint32_t v) { return (v + 255) / 256 * 256; }
+
+// Row tile and k splits by estimated time: the blocks run in rounds of one per CU, each ktile_us per k-tile plus its
+// prologue and epilogue; a count above 1 adds its partials' round trip and a launch. `unit`: k-tiles a split may not
+// cut (1: the up projection). Constants measured on MI355X at 8-64 k-tiles and 40-2048 blocks.
+struct ChainTile {
+    uint32_t bm;
+    double ktile_us[2], up_us, down_us;  // a k-tile with float32, bfloat16 weights; prologue and epilogue
+};
+constexpr ChainTile kChainTiles[] = {{64, {0.45, 0.36}, 6.4, 4.5}, {128, {0.66, 0.56}, 8.5, 6.0}, {256, {1.36, 0.97}, 9.0, 8.0}};
+constexpr uint32_t kPrefillMaxSplits = 24;
+struct ChainPlan {
+    uint32_t bm, splits;
+};
+ChainPlan chain_plan(uint32_t m, uint32_t ncol, uint32_t k, bool bf16, uint32_t unit, uint32_t min_splits) {
+    const uint32_t units = k / kBK / unit;
+    ChainPlan best{0, 0};
+    double best_us = 0.0;
+    for (const ChainTile& tile : kChainTiles)
+        for (uint32_t splits = min_splits; splits <= min(units, kPrefillMaxSplits); ++splits) {
+            const uint32_t rounds = ceil_div(ceil_div(m, tile.bm) * (ncol / kDmaBN) * splits, kCus);
+            double us = rounds * (ceil_div(units, splits) * unit * tile.ktile_us[bf16] + (unit == 1 ? tile.up_us : tile.down_us));
+            if (splits > 1) us += 8.0 * splits * m * ncol / kPartialBytesPerUs + kReduceUs;
+            if (best.bm == 0 || us < best_us) best = {tile.bm, splits}, best_us = us;
+        }
+    return best;
+}
+struct PrefillPlan {
+    ChainPlan up, down;
+};
+// m: the real tokens; planned for the end of their block of kRowPad (128 below it), so that a workspace sized for n
+// serves every smaller call
+uint32_t prefill_class(uint32_t m) { return m <= 128 ? 128 : rows_padded(m); }
+PrefillPlan prefill_plan(uint32_t m, uint32_t d, uint32_t h, bool bf16) {
+    static_assert(kPrefillDownBlocks <= kDmaMaxActBlocks, "a split's binades fit LDS");
+    const uint32_t rows = prefill_class(m);
+    return {chain_plan(rows, h, d, bf16, 1, 1), chain_plan(rows, d, h, bf16, kKtPerActBlock, ceil_div(h / kActBlock, kPrefillDownBlocks))};
+}
+
+struct PrefillLayout {
+    uint32_t d, h;  // padded widths
+    size_t up_planes, up_exp, down_planes, down_exp, x_exp, act_exp, x_planes, act_planes, partials, bytes;
+};
+// Byte offsets (256-byte aligned) for calls of up to n tokens; the partials hold the largest of any smaller call's.
+PrefillLayout prefill_layout(bool bf16, uint32_t n, uint32_t d, uint32_t h) {
+    PrefillLayout l{};
+    l.d = pad256(d);
+    l.h = pad256(h);
+    n = min(n, kPrefillPiece);
+    const size_t rows = rows_padded(n);
+    size_t at = 0;
+    const auto take = [&at](size_t bytes) {
+        const size_t from = at;
+        at = align256(at + bytes);
+        return from;
+    };
+    l.up_planes = take(dense_plane_halves(l.h, l.d) * 2);
+    l.up_exp = take(static_cast<size_t>(l.h) * 4);
+    l.down_planes = take(dense_plane_halves(l.d, l.h) * 2);
+    l.down_exp = take(static_cast<size_t>(l.d) * 4);
+    l.x_exp = take(rows * 4);
+    l.act_exp = take(rows * (l.h / kActBlock));
+    l.x_planes = take(dense_plane_halves(rows, l.d) * 2);
+    l.act_planes = take(dense_plane_halves(rows, l.h) * 2);
+    size_t most = 0;
+    for (uint32_t m = 128; m <= max(rows, size_t{128}); m += m == 128 ? 128 : kRowPad) {
+        const PrefillPlan plan = prefill_plan(m, l.d, l.h, bf16);
+        if (plan.up.splits > 1) most = max(most, static_cast<size_t>(plan.up.splits) * min(m, n) * l.h);
+        if (plan.down.splits > 1) most = max(most, static_cast<size_t>(plan.down.splits) * min(m, n) * l.d);
+    }
+    l.partials = take(most * 4);
+    l.bytes = at;
+    return l;
+}
+
+uint64_t prefill_workspace_bytes(int vt, uint32_t n, uint32_t d, uint32_t h) { return prefill_layout(vt == kBF16, n, d, h).bytes; }
+
+namespace {
+template <typename V>
+hipError_t prefill(const PrefillCall& c, hipStream_t stream) {
+    constexpr bool kLoB = sizeof(V) == 4;
+    constexpr int kUpChain = kLoB ? kKtPerActBlock / 2 : kKtPerActBlock;
+    const PrefillLayout l = prefill_layout(!kLoB, c.n, c.d, c.h);
+    char* w = static_cast<char*>(c.workspace);
+    const auto halves = [&](size_t at) { return reinterpret_cast<_Float16*>(w + at); };
+    const auto words = [&](size_t at) { return reinterpret_cast<int32_t*>(w + at); };
+    float* partials = reinterpret_cast<float*>(w + l.partials);
+    const DensSide up{c.up_off, c.up_idx, c.up_val, c.h, l.h, l.d, slots_aligned(c.up_idx, c.up_val), halves(l.up_planes), words(l.up_exp)};
+    const DensSide down{c.down_off, c.down_idx, c.down_val, c.d, l.d, l.h, slots_aligned(c.down_idx, c.down_val), halves(l.down_planes), words(l.down_exp)};
+    for (uint32_t t0 = 0; t0 < c.n; t0 += kPrefillPiece) {
+        const uint32_t n = min(kPrefillPiece, c.n - t0), rows = rows_padded(n), split_blocks = rows_live(n) / kSplitBlockRows / kSplitGroups;
+        const uint32_t up_blocks = t0 == 0 ? dens_blocks(l.h, l.d) : 0, down_blocks = t0 == 0 ? dens_blocks(l.d, l.h) : 0;
+        const float* x = c.x + static_cast<size_t>(t0) * c.d;
+        float* y = c.y + static_cast<size_t>(t0) * c.d;
+        hipLaunchKernelGGL(prefill_prep_kernel<V>, dim3(up_blocks + down_blocks + split_blocks), dim3(kDensThreads), 0, stream, up, down,
+                           up_blocks, down_blocks, x, n, rows, l.d, c.d, halves(l.x_planes), words(l.x_exp));
+        if (hipError_t status = hipGetLastError(); status != hipSuccess) return status;
+        const PrefillPlan plan = prefill_plan(n, l.d, l.h, !kLoB);
+        const bool split = plan.up.splits > 1;
+        hipError_t status =
+            split ? launch_chained<Epi::UpSplit, kLoB, kUpChain>(plan.up.bm, halves(l.x_planes), words(l.x_exp), up.planes, up.exps, nullptr,
+                                                                 partials, nullptr, nullptr, n, l.h, l.d, plan.up.splits, l.h, stream)
+                  : launch_chained<Epi::Up, kLoB, kUpChain>(plan.up.bm, halves(l.x_planes), words(l.x_exp), up.planes, up.exps, c.b_up,
+                                                            nullptr, halves(l.act_planes), words(l.act_exp), n, l.h, l.d, 1, c.h, stream);
+        if (status != hipSuccess) return status;
+        if (split) {
+            hipLaunchKernelGGL(act_planes_kernel<true>, dim3(rows_live(n) / kActRowsPerBlock, l.h / kActBlock), dim3(kThreads), 0, stream,
+                               partials, plan.up.splits, c.b_up, halves(l.act_planes), reinterpret_cast<int8_t*>(w + l.act_exp), n, rows,
+                               l.h, c.h);
+            if (status = hipGetLastError(); status != hipSuccess) return status;
+        }
+        const bool parts = plan.down.splits > 1;
+        status = launch_chained<Epi::Down, kLoB, kPrefillDownChain>(plan.down.bm, halves(l.act_planes), words(l.act_exp), down.planes,
+                                                                    down.exps, c.b_down, parts ? partials : y, nullptr, nullptr, n, l.d, l.h,
+                                                                    plan.down.splits, c.d, stream);
+        if (status == hipSuccess && parts)
+            status = launch_reduce_splits(partials, c.b_down, y, n, plan.down.splits, l.d, 0, c.d, stream);
+        if (status != hipSuccess) return status;
+    }
+    return hipSuccess;
+}
+}  // namespace
+
+hipError_t launch_prefill(int vt, const PrefillCall& call, hipStream_t stream) {
+    return vt == kBF16 ? prefill<uint16_t>(call, stream) : prefill<float>(call, stream);
 }
 
 size_t train_mfma_workspace_bytes(uint32_t n, uint32_t d, uint32_t h) { return workspace_layout(n, d, h, true).bytes; }

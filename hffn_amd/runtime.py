@@ -13,6 +13,8 @@ Kernel shapes (the build's own policy, ``up_mode``/``down_mode``):
   rows through a table of row bounds (default) or from a tiled copy (``tiled=True``: the compact slots regrouped at
   load by 16-row tile and 512-wide sub-chunk of K, interleaved 16-bit fields), densified per block in LDS and
   multiplied on 16x16x32 MFMAs.
+* planes of the call (``transient``) - both sides densified into the workspace, then split-fp16 MFMA GEMMs in short
+  chains; N > 64 on layers without resident planes, where estimated faster than the two compact-store paths above 64.
 * ``rows``  - lanes over tokens (1, 2 or 4 per lane), slots walked in order; large N on layers without the MFMA path.
 * ``mfma``  - tile-densified split-fp16 MFMA GEMMs over dense planes (up and down together) on high-density layers
   (density at least ``MFMA_MIN_DENSITY``, ``d_model`` and ``d_ff`` multiples of 256), above 64 tokens.
@@ -78,6 +80,17 @@ TILES_TIE = 1.05  # the tiles path wins estimates within 5 % of the lane-per-slo
 # (each slot reads its input row of every token from L2), fitted to forced-pair timings of the 70M/20 %, 410M/50 % and
 # 1.4B/20 % bf16 layers at 65-2048 tokens; against it the tiles path in pieces of 64 tokens (one tiles_us each).
 ROWS_CALL_US, ROWS_SLOT_US = 30.0, 0.148e-6
+# Calls above 64 tokens on planes densified for the call (hffn_forward_prefill), in place of either: PREFILL_CALL_US per
+# call, PREFILL_PLANE_US per densified weight and plane (float32: two), PREFILL_MAC_US per weight, padded token and MFMA
+# product (3 float32, 2 bfloat16), PREFILL_ROW_US per token and width. Fitted to 35 timings of nine layers (256 x 1024 to
+# 2560 x 10240, 10-30 % density, both value types) at 65-3000 tokens, each within 15 %. Against it the lane-per-token
+# kernels are priced at ROWS_SHARE of rows_us (which the same layers' timings stay below by about that), and at least at
+# their walk: ROWS_WALK_US plus ROWS_WALK_SLOT_US per slot of the longest row of either side (one wave walks a row).
+# Measured, µs (compact store's kernels, planes of the call): 512 x 2048 at 20 % float32, 128 tokens: 36.6, 30.3; 768 x
+# 3072 at 10 %, 128 and 512 tokens: 34.8, 39.9 and 55.8, 48.4; 1024 x 4096 at 10 % with outputs of up to 4096 slots, 128
+# tokens: 186, 46; 2048 x 8192 at 20 % bfloat16, 128 and 1999 tokens: 98, 80 and 1415, 318.
+PREFILL_CALL_US, PREFILL_PLANE_US, PREFILL_MAC_US, PREFILL_ROW_US = 22.5, 2.5e-6, 3.05e-9, 1.45e-6
+ROWS_SHARE, ROWS_WALK_US, ROWS_WALK_SLOT_US = 0.9, 10.0, 0.045
 MAX_TOKENS = 1 << 18      # runtime/gpu/nvidia/common/kernels/hffn_cuda/runtime.py:26
 # The reference's policy constants (runtime.py:24-25), with this policy's meaning: COOP_MAX_TOKENS, the largest N the
 # policy may run on the cooperative (lane-per-slot, wave-reduced) kernels; BLOCK_MAX_WIDTH, the widest d_ff up to which
@@ -148,6 +161,14 @@ def pieces_us(n: int, shape: StoreShape) -> float:
     """Estimated µs of N tokens on the tiles path, in calls of up to ``TILES_MAX_TOKENS`` tokens."""
     whole, rest = divmod(n, TILES_MAX_TOKENS)
     return whole * tiles_us(TILES_MAX_TOKENS, shape) + (tiles_us(rest, shape) if rest else 0.0)
+
+
+def prefill_us(n: int, d_model: int, d_ff: int, bf16: bool) -> float:
+    """Estimated µs of a call of more than 64 tokens on planes densified for the call."""
+    d, h = -(-d_model // 256) * 256, -(-d_ff // 256) * 256  # the planes' padded widths
+    rows = 128 if n <= 128 else -(-n // 256) * 256
+    return (PREFILL_CALL_US + PREFILL_PLANE_US * d * h * (1 if bf16 else 2) + PREFILL_MAC_US * d * h * rows * (2 if bf16 else 3)
+            + PREFILL_ROW_US * rows * (d + h))
 
 
 def decode_mode(n: int, shape: StoreShape, edges: bool, tiles: bool) -> str | None:
@@ -335,6 +356,11 @@ class HFFNRuntime:
             words = (_lib.query_bytes(self._lib.hffn_gemv_workspace, self.d_model, self.d_ff) + 3) // 4
             self._gemv_work = torch.empty(words, device=self.device)  # the decode GEMVs' k-split partial sums
         self._policy: dict[int, tuple[str, str]] = {}  # N -> the policy's (up, down)
+        self._transient_allowed = dense is not False and self._tiles is not None
+        longest = [torch.stack([tensors[name].diff().max() for tensors in self._tensors]).max() for name in ("up_offsets", "out_offsets")]
+        self._longest = sum(torch.stack(longest).tolist())  # slots of the longest row of either side
+        self._transient: dict[int, bool] = {}  # N -> whether the policy densifies planes for the call
+        self._prefill_work: torch.Tensor | None = None
         self.forced_up: str | None = None
         self.forced_down: str | None = None
         self.calls: Counter = Counter()
@@ -471,15 +497,22 @@ class HFFNRuntime:
             words = (_lib.query_bytes(self._lib.hffn_mfma_workspace, n, self.d_model, self.d_ff) + 3) // 4
         # zero-filled once: the split-K counters it holds start at zero and every call leaves them at zero
         self._mfma_work = torch.zeros(words, dtype=torch.int32, device=self.device)
+        self._transient.clear()
+        self._prefill_work = None
+        if any(self._prefers_transient(m) for m in {n, *(1 << b for b in range(7, n.bit_length()))}):
+            words = _lib.query_bytes(self._lib.hffn_prefill_workspace, self._args[0][0], n, self.d_model, self.d_ff) // 4
+            self._prefill_work = torch.empty(words, dtype=torch.int32, device=self.device)
         self._work = (self._x_t.data_ptr(), self._act.data_ptr(), self._y_t.data_ptr(), self._y.data_ptr())
 
     def workspace_bytes(self) -> int:
         return 4 * (self._x_t.numel() + self._act.numel() + self._y_t.numel() + self._y.numel() + self._mfma_work.numel() +
-                    self._gemv_work.numel() + self._tiles_work.numel())
+                    self._gemv_work.numel() + self._tiles_work.numel() +
+                    (self._prefill_work.numel() if self._prefill_work is not None else 0))
 
     def modes(self, n: int) -> tuple[str, str]:
-        """The (up, down) shapes a call of N tokens takes (forced ones first). The policy's choice depends on N and the
-        layers only, so it is worked out once per N (the library queries behind it are ctypes calls)."""
+        """The (up, down) shapes over the resident stores a call of N tokens takes (forced ones first). The policy's choice
+        depends on N and the layers only, so it is worked out once per N (the library queries behind it are ctypes
+        calls). An unforced call above 64 tokens may run on planes densified for the call instead (``transient``)."""
         chosen = self._policy.get(n) if self.forced_up is None and self.forced_down is None else None
         if chosen is None:
             chosen = self._modes(n)
@@ -487,21 +520,53 @@ class HFFNRuntime:
                 self._policy[n] = chosen
         return chosen
 
+    def _policy_mode(self, n: int) -> str | None:
+        """The pair (``tiles`` or ``mfma``) the policy runs N tokens on, or None: the lane-per-slot or -token kernels."""
+        if n <= TILES_MAX_TOKENS:
+            mode = decode_mode(n, self._store, edges_supported(self.d_model, n), self._tiles is not None)
+            return mode if mode == "tiles" else None
+        if self._planes is not None and self.density >= MFMA_MIN_DENSITY and mfma_streamed(n, self.d_model, self.d_ff):
+            return "mfma"
+        if self._tiles is not None and pieces_us(n, self._store) < rows_us(n, self._store):
+            return "tiles"
+        return None
+
     def _modes(self, n: int) -> tuple[str, str]:
         edges = edges_supported(self.d_model, n)
         if self.forced_up is None and self.forced_down is None:
-            if n <= TILES_MAX_TOKENS:
-                mode = decode_mode(n, self._store, edges, self._tiles is not None)
-                if mode == "tiles":
-                    return mode, mode
-            elif self._planes is not None and self.density >= MFMA_MIN_DENSITY and mfma_streamed(n, self.d_model, self.d_ff):
-                return "mfma", "mfma"
-            elif self._tiles is not None and pieces_us(n, self._store) < rows_us(n, self._store):
-                return "tiles", "tiles"
+            mode = self._policy_mode(n)
+            if mode is not None:
+                return mode, mode
         up = self.forced_up or up_mode(n, self.d_model)
         if up == "edges" and not edges:
             up = "rows"
         return up, self.forced_down or down_mode(n, self.d_ff)
+
+    def _prefers_transient(self, n: int) -> bool:
+        """Whether the policy runs N tokens on planes densified for the call: above 64 tokens, where neither resident
+        planes take the call nor the compact store's own kernels are estimated faster."""
+        if not self._transient_allowed or n <= TILES_MAX_TOKENS:
+            return False
+        up = self._policy_mode(n)
+        if up == "tiles":
+            other = pieces_us(n, self._store)
+        elif up is None:
+            other = max(ROWS_SHARE * rows_us(n, self._store), ROWS_WALK_US + ROWS_WALK_SLOT_US * self._longest)
+        else:
+            return False
+        return prefill_us(n, self.d_model, self.d_ff, self._args[0][0] == _lib.VALUE_BF16) < other
+
+    def transient(self, n: int) -> bool:
+        """Whether a call of N tokens runs on planes densified for the call (``hffn_forward_prefill``) in place of the
+        compact store's path that ``modes`` names: unforced calls above 64 tokens of layers without resident planes
+        (``dense=False`` excludes them as well), where that is estimated faster. The planes live in the runtime's
+        workspace, one layer's at a time; ``calls`` counts the call under the path that ``modes`` names."""
+        if self.forced_up is not None or self.forced_down is not None:
+            return False
+        chosen = self._transient.get(n)
+        if chosen is None:
+            chosen = self._transient[n] = n <= self._tokens and self._prefill_work is not None and self._prefers_transient(n)
+        return chosen
 
     def forward(self, index: int, x: torch.Tensor) -> torch.Tensor:
         """y[N, d_model] of layer ``index`` for x[N, d_model] (contiguous float32 on the device).
@@ -548,6 +613,12 @@ class HFFNRuntime:
         value_type, *model = self._args[index]
         x_t, act, y_t, y = self._work
         stream = torch.cuda.current_stream(self.device).cuda_stream
+        if self.transient(n):
+            x = _aligned(x)  # read 16 bytes at a time
+            _lib.check(self._lib.hffn_forward_prefill(value_type, x.data_ptr(), *model, self._prefill_work.data_ptr(),
+                                                      4 * self._prefill_work.numel(), y, self.d_model, self.d_ff, n, stream),
+                       f"forward ({up}, {down}) on planes of the call")
+            return
         if up == "tiles":
             x = _aligned(x)  # read 16 bytes at a time
             self._fresh_tiles(index)

@@ -27,7 +27,7 @@
 extern "C" {
 #endif
 
-#define HFFN_ABI_VERSION 18
+#define HFFN_ABI_VERSION 19
 
 #define HFFN_OK 0
 #define HFFN_ERROR_ARGUMENT (-1) /* invalid shape, mode, pointer or workspace */
@@ -271,6 +271,18 @@ int hffn_plan_tiles_compact(int value_type, const int16_t* up_idx, const void* u
                             const int16_t* out_hidden, const void* out_val, const int32_t* down_table, const float* b_down, float* act,
                             void* workspace, uint64_t workspace_bytes, float* y, uint32_t d_model, uint32_t d_ff, uint64_t nnz_up,
                             uint64_t nnz_down, uint32_t n, uint64_t* plan);
+
+/* A whole forward above the decode sizes on a layer without planes of its own: both sides' planes are densified from
+ * the compact rows into the call's workspace (hffn_prefill_workspace bytes for calls of up to n tokens, any content,
+ * 256-byte aligned), and the projections run on them as split-fp16 MFMA products, their float32 sums in chains of 128
+ * k. d_model a multiple of 16, d_ff of 8, distinct ascending indices per row; x, y and the biases 16-byte aligned.
+ * Widths need not be multiples of 256 (the planes are padded). Calls above 16384 tokens run in pieces of that size
+ * over the same planes. No counterpart (the reference's large-N kernels are gathers, kernels.py:87-191). */
+int hffn_prefill_workspace(int value_type, uint32_t n, uint32_t d_model, uint32_t d_ff, uint64_t* bytes);
+int hffn_forward_prefill(int value_type, const float* x, const int32_t* up_offsets, const int16_t* up_idx, const void* up_val,
+                         const float* b_up, const int32_t* out_offsets, const int16_t* out_hidden, const void* out_val,
+                         const float* b_down, void* workspace, uint64_t workspace_bytes, float* y, uint32_t d_model, uint32_t d_ff,
+                         uint32_t n, void* stream);
 
 /* ------------------------------------------------------------------------------------------------ training (fp32)
  * Layouts: act, z, gz hidden-major [d_ff, ld]; x_t, gy_t, gx_t feature-major [d_model, ld]; x, y, gx token-major

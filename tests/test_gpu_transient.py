@@ -1,0 +1,147 @@
+"""Calls on planes densified for the call (``hffn_forward_prefill``, the policy's ``transient`` calls above 64 tokens)
+against the float64 oracle: widths that are and are not multiples of 256, both value types, neurons without slots,
+rows longer than the densify kernel holds in registers, the edges of its token tiles (64, 128, 256), a call of several
+pieces, arrays off their 16-byte boundaries, and the planned and captured forms of the call.
+
+Tolerance: a relative error (2-norm) of 6e-7. Every operand is hi + lo in fp16 (2^-23 of the entry at most), the sums run
+in chains of at most 24 products and at most 32 chains, each rounded to float32: about sqrt(24 + 32) 2^-24 = 4.5e-7
+per projection at worst, 2e-7 measured for both."""
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from hffn_amd import _lib, synth
+from hffn_amd.ffn import hip_layer
+from hffn_amd.prepared_runtime import PreparedRuntime
+from hffn_amd.runtime import HFFNLayer, HFFNRuntime
+from oracle import reference
+
+pytestmark = pytest.mark.gpu
+RELATIVE = 6e-7
+
+
+def _side(rng, h, d, density, full):
+    degrees = rng.integers(0, max(2, int(2 * density * d)), h)
+    degrees[::11] = 0
+    degrees[full] = d  # neurons of every slot: one output (down) or neuron (up) row of full length
+    offsets = np.zeros(h + 1, np.int32)
+    offsets[1:] = np.cumsum(degrees)
+    index = np.concatenate([np.sort(rng.choice(d, k, replace=False)) for k in degrees] or [[]]).astype(np.int16)
+    return offsets, index, (rng.standard_normal(index.size) * 0.02).astype(np.float32)
+
+
+def _layer(d, h, density, bf16, seed=3):
+    rng = np.random.default_rng([seed, d, h])
+    up, down = _side(rng, h, d, density, [1]), _side(rng, h, d, density, [2, h - 1])
+    if bf16:  # values the bfloat16 store holds exactly
+        up, down = ((o, i, torch.from_numpy(v).bfloat16().float().numpy()) for o, i, v in (up, down))
+    b_up, b_down = ((rng.standard_normal(k) * 0.01).astype(np.float32) for k in (h, d))
+    return synth.CompactLayer(d, h, synth._groups(h), *up, b_up, *down, b_down)
+
+
+def _device_layer(layer, bf16, device):
+    t = lambda a: torch.from_numpy(a).to(device)  # noqa: E731
+    value = lambda a: t(a).bfloat16() if bf16 else t(a)  # noqa: E731
+    return HFFNLayer.from_hidden_major(layer.d_model, layer.d_ff, t(layer.b_up), t(layer.up_offsets), t(layer.up_idx),
+                                       value(layer.up_val), t(layer.b_down), t(layer.down_offsets), t(layer.down_idx),
+                                       value(layer.down_val))
+
+
+def _prefill(runtime, x, shift=0):
+    """hffn_forward_prefill on a workspace of NaNs, guard words behind y and the workspace; ``shift``: slots by which
+    copies of the index and value arrays start off their boundaries."""
+    lib, n = _lib.load(), x.shape[0]
+    tensors, keep = runtime._tensors[0], []
+
+    def at(name):
+        tensor = tensors[name]
+        if shift and name in ("up_idx", "up_val", "out_hidden", "out_val"):
+            moved = torch.zeros(tensor.numel() + shift, dtype=tensor.dtype, device=x.device)
+            moved[shift:] = tensor
+            keep.append(moved)
+            tensor = moved[shift:]
+        return tensor.data_ptr()
+
+    need = _lib.query_bytes(lib.hffn_prefill_workspace, runtime._args[0][0], n, runtime.d_model, runtime.d_ff)
+    work = torch.full((need // 4 + 64,), float("nan"), device=x.device)
+    y = torch.full((n + 1, runtime.d_model), -7.0, device=x.device)
+    arrays = [at(name) for name in ("up_offsets", "up_idx", "up_val", "b_up", "out_offsets", "out_hidden", "out_val", "b_down")]
+    _lib.check(lib.hffn_forward_prefill(runtime._args[0][0], x.data_ptr(), *arrays, work.data_ptr(), need, y.data_ptr(),
+                                        runtime.d_model, runtime.d_ff, n, torch.cuda.current_stream().cuda_stream), "prefill")
+    torch.cuda.synchronize()
+    assert bool((y[n] == -7.0).all()) and bool(torch.isnan(work[need // 4:]).all())
+    return y[:n]
+
+
+def _relative(y, expected):
+    return float(np.linalg.norm(y.double().cpu().numpy() - expected) / np.linalg.norm(expected))
+
+
+@pytest.mark.parametrize("d,h,density,bf16,tokens", [
+    (16, 8, 0.5, False, (1, 65)), (256, 1024, 0.2, False, (65, 129, 16384 + 70)), (400, 1608, 0.3, False, (64, 128, 257)),
+    (400, 1608, 0.3, True, (65, 300)), (768, 3072, 0.05, False, (128, 512)), (1104, 4424, 0.2, True, (70, 256, 513)),
+    (272, 9000, 0.1, False, (100,)), (2048, 8192, 0.1, True, (1030,))])
+def test_prefill_matches_the_oracle(d, h, density, bf16, tokens, device):
+    layer = _layer(d, h, density, bf16)
+    runtime = HFFNRuntime([_device_layer(layer, bf16, device)], device, dense=False)
+    weights = reference.dense_weights(layer)
+    for n in tokens:
+        x = np.random.default_rng([5, n]).standard_normal((n, d)).astype(np.float32)
+        x[n // 2] *= 1e-3  # tokens of other scales, and one of zeros
+        x[-1] = 0.0
+        expected = reference.forward_dense(layer, x, weights)
+        xd = torch.from_numpy(x).to(device)
+        y = _prefill(runtime, xd)
+        assert _relative(y, expected) <= RELATIVE, n
+        if n <= 300:
+            assert torch.equal(_prefill(runtime, xd, shift=3), y), n  # off the boundaries: the same planes, the same bits
+
+
+def test_policy_plans_and_capture(device):
+    """An unforced call above 64 tokens takes the planes of the call where estimated faster, eager, prepared and
+    captured with the same bits; forced pairs, dense=False and unsorted rows keep the compact store's kernels."""
+    d, h, n = 400, 1608, 300
+    layer = _layer(d, h, 0.3, False)
+    compact = hip_layer(layer)
+    runtime, prepared = HFFNRuntime([compact], device), PreparedRuntime([compact], device)
+    x = torch.from_numpy(np.random.default_rng(9).standard_normal((n, d)).astype(np.float32)).to(device)
+    y = runtime.forward(0, x).clone()
+    assert runtime.transient(n) and not runtime.transient(64) and sum(runtime.calls.values()) == 1
+    assert torch.equal(y, _prefill(runtime, x)) and torch.equal(prepared.forward(0, x), y) and torch.equal(prepared.forward(0, x), y)
+    assert _relative(y, reference.forward(layer, x.cpu().numpy())) <= RELATIVE
+    graph, out = torch.cuda.CUDAGraph(), torch.empty_like(y)
+    with torch.cuda.graph(graph):
+        out.copy_(runtime.forward(0, x))
+    for k in range(3):
+        x.mul_(0.5)
+        expected = prepared.forward(0, x).clone()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, expected), k
+    small = x[:70].contiguous()
+    runtime.force("rows", "rows")
+    assert not runtime.transient(n)
+    rows = runtime.forward(0, small).clone()
+    runtime.force(None, None)
+    assert float((runtime.forward(0, small) - rows).abs().max()) <= 1e-5
+    never = HFFNRuntime([compact], device, dense=False)
+    never.forward(0, x)
+    assert not never.transient(n) and never._prefill_work is None
+
+
+def test_prefill_refusals(device):
+    lib, size = _lib.load(), ctypes.c_uint64(0)
+    p, odd = 256, 264  # never dereferenced: the calls are refused before any launch
+    assert lib.hffn_prefill_workspace(0, 100, 400, 1608, ctypes.byref(size)) == _lib.OK
+    for arguments, message in (((0, odd, *[p] * 9, size.value, p, 400, 1608, 100), "aligned"),
+                               ((0, *[p] * 9, odd, size.value, p, 400, 1608, 100), "aligned"),
+                               ((0, *[p] * 10, size.value - 1, p, 400, 1608, 100), "workspace"),
+                               ((0, *[p] * 10, size.value, p, 400, 1604, 100), "multiple of 8"),
+                               ((0, *[p] * 10, size.value, p, 408, 1608, 100), "multiple of 16"),
+                               ((7, *[p] * 10, size.value, p, 400, 1608, 100), "value type"),
+                               ((0, *[p] * 5, None, *[p] * 4, size.value, p, 400, 1608, 100), "null")):
+        assert lib.hffn_forward_prefill(*arguments, None) == -1 and message in lib.hffn_last_error().decode(), message
