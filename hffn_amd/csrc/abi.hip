@@ -785,6 +785,57 @@ int hffn_backward_mfma(const float* gy, const float* z, const void* down_t_plane
                     "backward_mfma");
 }
 
+int hffn_train_planes_workspace(uint32_t n, uint32_t d_model, uint32_t d_ff, uint64_t* bytes) {
+    if (!bytes) return fail(HFFN_ERROR_ARGUMENT, "train_planes_workspace: null result");
+    if (int status = check_mfma(HFFN_VALUE_F32, d_model, d_ff, n)) return status;
+    *bytes = hffn::train_planes_workspace_bytes(n, d_model, d_ff);
+    return HFFN_OK;
+}
+
+namespace {
+int check_train_planes(const char* what, uint32_t d_model, uint32_t d_ff, uint32_t n, uint32_t ld, const void* workspace,
+                       uint64_t workspace_bytes, std::initializer_list<const void*> floats, std::initializer_list<const void*> others) {
+    uint64_t needed = 0;
+    if (int status = hffn_train_planes_workspace(n, d_model, d_ff, &needed)) return status;
+    if (ld < n || ld % 4 != 0) return fail(HFFN_ERROR_ARGUMENT, "%s: ld=%u must be a multiple of 4 and at least n=%u", what, ld, n);
+    for (const void* p : floats)
+        if (!p || reinterpret_cast<uintptr_t>(p) % 16 != 0) return fail(HFFN_ERROR_ARGUMENT, "%s: null or not 16-byte aligned float buffer", what);
+    for (const void* p : others)
+        if (!p) return fail(HFFN_ERROR_ARGUMENT, "%s: null pointer", what);
+    if (!workspace || reinterpret_cast<uintptr_t>(workspace) % 256 != 0)
+        return fail(HFFN_ERROR_ARGUMENT, "%s: the workspace must be 256-byte aligned", what);
+    if (workspace_bytes < needed)
+        return fail(HFFN_ERROR_ARGUMENT, "%s: workspace of %llu bytes, %llu needed", what, static_cast<unsigned long long>(workspace_bytes),
+                    static_cast<unsigned long long>(needed));
+    return HFFN_OK;
+}
+}  // namespace
+
+int hffn_forward_planes_z(const float* x, const int32_t* up_offsets, const int16_t* up_idx, const float* up_val, const float* b_up,
+                          const int32_t* out_offsets, const int16_t* out_hidden, const float* out_val, const float* b_down,
+                          void* workspace, uint64_t workspace_bytes, float* x_t, float* act, float* z, float* y, uint32_t d_model,
+                          uint32_t d_ff, uint32_t n, uint32_t ld, void* stream) {
+    if (int status = check_train_planes("forward_planes_z", d_model, d_ff, n, ld, workspace, workspace_bytes, {x, b_up, b_down, x_t, act, z, y},
+                                        {up_offsets, up_idx, up_val, out_offsets, out_hidden, out_val}))
+        return status;
+    const hffn::PrefillCall call{x, up_offsets, up_idx, up_val, b_up, out_offsets, out_hidden, out_val, b_down, workspace, y, d_model, d_ff, n};
+    return launched(hffn::launch_train_planes_forward(call, x_t, act, z, ld, static_cast<hipStream_t>(stream)), "forward_planes_z");
+}
+
+int hffn_backward_planes(const float* gy, const float* z, const int32_t* hid_offsets, const int16_t* hid_output, const int32_t* hid_pos,
+                         const float* out_val, const int32_t* in_offsets, const int16_t* in_hidden, const int32_t* in_pos,
+                         const float* up_val, float* hid_val, float* in_val, void* workspace, uint64_t workspace_bytes, float* gy_t,
+                         float* gz, float* gx, uint32_t d_model, uint32_t d_ff, uint32_t nnz_up, uint32_t nnz_down, uint32_t n,
+                         uint32_t ld, void* stream) {
+    if (int status = check_train_planes("backward_planes", d_model, d_ff, n, ld, workspace, workspace_bytes,
+                                        {gy, z, gy_t, gz, gx, hid_val, in_val},
+                                        {hid_offsets, hid_output, hid_pos, out_val, in_offsets, in_hidden, in_pos, up_val}))
+        return status;
+    const hffn::TrainBackward call{gy, z, hid_offsets, hid_output, hid_pos, out_val, in_offsets, in_hidden, in_pos, up_val,
+                                   hid_val, in_val, workspace, gy_t, gz, gx, d_model, d_ff, nnz_up, nnz_down, n, ld};
+    return launched(hffn::launch_train_planes_backward(call, static_cast<hipStream_t>(stream)), "backward_planes");
+}
+
 int hffn_grad_sddmm(const float* row, const float* mat, const int32_t* offsets, const int16_t* index, float* g, float* gb,
                     uint32_t rows, uint32_t n, uint32_t ld, uint32_t stride, void* stream) {
     if (int status = check_shape(16, rows, n, ld)) return status;
@@ -827,11 +878,8 @@ int hffn_grad_x(const float* gz, const int32_t* in_offsets, const int16_t* in_hi
                                                 nnz_up, s),
                         "grad_x (edges)");
     }
-    if (int status = launched(hffn::launch_down_rows(HFFN_VALUE_F32, gz, in_offsets, in_hidden, in_val, nullptr, gx_t, d_model, n,
-                                                     ld, s),
-                              "grad_x"))
-        return status;
-    return launched(hffn::launch_transpose(gx_t, gx, d_model, n, ld, d_model, s), "grad_x transpose");
+    // each output's lanes write gx token-major: no transpose after
+    return launched(hffn::launch_down_rows(HFFN_VALUE_F32, gz, in_offsets, in_hidden, in_val, nullptr, gx, d_model, n, ld, s, true), "grad_x");
 }
 
 int hffn_reduce_tiles(const float* ws, uint32_t stride, uint32_t tiles, uint32_t c1, uint32_t c2, uint32_t c3, float* g_down,
@@ -848,15 +896,44 @@ int hffn_adamw(float* p, const float* g, float* m, float* v, uint32_t count, flo
                float beta2, float one_minus_beta2, float step_size, float bias2_sqrt, float eps, void* stream) {
     if (count == 0) return HFFN_OK;
     if (!p || !g || !m || !v) return fail(HFFN_ERROR_ARGUMENT, "adamw: null pointer");
-    return launched(hffn::launch_adamw(p, g, m, v, count, lr_decay, beta1, one_minus_beta1, beta2, one_minus_beta2, step_size, bias2_sqrt,
-                                       eps, static_cast<hipStream_t>(stream)),
+    const hffn::AdamArray array{p, g, m, v, count};
+    return launched(hffn::launch_adamw(&array, 1, {lr_decay, beta1, one_minus_beta1, beta2, one_minus_beta2, step_size, bias2_sqrt, eps},
+                                       static_cast<hipStream_t>(stream)),
                     "adamw");
+}
+
+int hffn_adamw_arrays(uint32_t arrays, float* const* p, const float* const* g, float* const* m, float* const* v, const uint32_t* counts,
+                      float lr_decay, float beta1, float one_minus_beta1, float beta2, float one_minus_beta2, float step_size,
+                      float bias2_sqrt, float eps, void* stream) {
+    if (arrays == 0 || arrays > hffn::kAdamArrays) return fail(HFFN_ERROR_ARGUMENT, "adamw_arrays: %u arrays outside [1, %u]", arrays, hffn::kAdamArrays);
+    if (!p || !g || !m || !v || !counts) return fail(HFFN_ERROR_ARGUMENT, "adamw_arrays: null pointer");
+    hffn::AdamArray list[hffn::kAdamArrays];
+    uint32_t used = 0;
+    for (uint32_t k = 0; k < arrays; ++k) {
+        if (counts[k] == 0) continue;
+        if (!p[k] || !g[k] || !m[k] || !v[k]) return fail(HFFN_ERROR_ARGUMENT, "adamw_arrays: null pointer");
+        list[used++] = {p[k], g[k], m[k], v[k], counts[k]};
+    }
+    return launched(hffn::launch_adamw(list, used, {lr_decay, beta1, one_minus_beta1, beta2, one_minus_beta2, step_size, bias2_sqrt, eps},
+                                       static_cast<hipStream_t>(stream)),
+                    "adamw_arrays");
 }
 
 int hffn_gather_values(const float* src, const int32_t* pos, float* dst, uint32_t count, void* stream) {
     if (count == 0) return HFFN_OK;
     if (!src || !pos || !dst) return fail(HFFN_ERROR_ARGUMENT, "gather_values: null pointer");
     return launched(hffn::launch_gather_values(src, pos, dst, count, static_cast<hipStream_t>(stream)), "gather_values");
+}
+
+int hffn_backward_prepare(const float* gy, float* gy_t, const float* out_val, const int32_t* hid_pos, float* hid_val, const float* up_val,
+                          const int32_t* in_pos, float* in_val, uint32_t d_model, uint32_t nnz_up, uint32_t nnz_down, uint32_t n,
+                          uint32_t ld, void* stream) {
+    if (int status = check_shape(d_model, 1, n, ld)) return status;
+    if (!gy || !gy_t || (nnz_down && (!out_val || !hid_pos || !hid_val)) || (nnz_up && (!up_val || !in_pos || !in_val)))
+        return fail(HFFN_ERROR_ARGUMENT, "backward_prepare: null pointer");
+    return launched(hffn::launch_backward_prepare(gy, gy_t, n, d_model, ld, out_val, hid_pos, hid_val, nnz_down, up_val, in_pos, in_val, nnz_up,
+                                                  static_cast<hipStream_t>(stream)),
+                    "backward_prepare");
 }
 
 int hffn_read_probe(const void* data, uint64_t bytes, uint32_t* sink, uint32_t sink_words, uint32_t blocks, void* stream) {

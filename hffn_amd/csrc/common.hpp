@@ -112,6 +112,58 @@ __device__ __forceinline__ void load_vec(const float* p, float (&out)[N]) {
     }
 }
 
+// out[c, r] = in[r, c] of the tile of kTransRows x kTransCols at (r0, c0), by the kTransThreads threads t, through LDS
+// (padded by one float per row). Every thread of the block calls it (one barrier). A full tile whose rows start on
+// 16-byte boundaries on both sides (vectors: strides multiples of 4 floats, aligned pointers) moves float4s: thread t
+// reads 16 bytes of input rows t / 16 and t / 16 + 16 (16 threads per 256-byte row run) and writes 16 bytes of output rows
+// t / 8 and t / 8 + 32 (4 input rows each), every load issued before the first LDS write; any other tile moves floats.
+constexpr uint32_t kTransRows = 32, kTransCols = 64, kTransThreads = 256;
+typedef float TransposeTile[kTransRows][kTransCols + 1];
+inline bool transpose_vectors(const void* in, const void* out, uint32_t in_ld, uint32_t out_ld) {
+    return in_ld % 4 == 0 && out_ld % 4 == 0 && reinterpret_cast<uintptr_t>(in) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
+}
+__device__ __forceinline__ void transpose_tile(TransposeTile& tile, uint32_t t, uint32_t r0, uint32_t c0, const float* __restrict__ in,
+                                               float* __restrict__ out, uint32_t rows, uint32_t cols, uint32_t in_ld, uint32_t out_ld,
+                                               bool vectors) {
+    static_assert(kTransRows * kTransCols / 4 == 2 * kTransThreads, "two float4 per thread each way");
+    const bool whole = vectors && r0 + kTransRows <= rows && c0 + kTransCols <= cols;
+    if (whole) {
+        float4 v[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const uint32_t r = t / 16 + 16 * j, c = (t % 16) * 4;
+            v[j] = *reinterpret_cast<const float4*>(in + static_cast<size_t>(r0 + r) * in_ld + c0 + c);
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const uint32_t r = t / 16 + 16 * j, c = (t % 16) * 4;
+            tile[r][c] = v[j].x;
+            tile[r][c + 1] = v[j].y;
+            tile[r][c + 2] = v[j].z;
+            tile[r][c + 3] = v[j].w;
+        }
+    } else {
+        for (uint32_t k = t; k < kTransRows * kTransCols; k += kTransThreads) {
+            const uint32_t r = k / kTransCols, c = k % kTransCols;
+            if (r0 + r < rows && c0 + c < cols) tile[r][c] = in[static_cast<size_t>(r0 + r) * in_ld + c0 + c];
+        }
+    }
+    __syncthreads();
+    if (whole) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const uint32_t c = t / 8 + 32 * j, r = (t % 8) * 4;
+            const float4 w = make_float4(tile[r][c], tile[r + 1][c], tile[r + 2][c], tile[r + 3][c]);
+            *reinterpret_cast<float4*>(out + static_cast<size_t>(c0 + c) * out_ld + r0 + r) = w;
+        }
+        return;
+    }
+    for (uint32_t k = t; k < kTransRows * kTransCols; k += kTransThreads) {
+        const uint32_t c = k / kTransRows, r = k % kTransRows;
+        if (c0 + c < cols && r0 + r < rows) out[static_cast<size_t>(c0 + c) * out_ld + r0 + r] = tile[r][c];
+    }
+}
+
 // s_waitcnt vmcnt(N) lgkmcnt(0): at most N vector-memory loads of this wave still in flight, its LDS accesses done.
 template <int N>
 __device__ __forceinline__ void wait_loads() {

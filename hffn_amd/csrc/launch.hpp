@@ -66,10 +66,23 @@ hipError_t launch_grad_sddmm(const float* row, const float* mat, const int32_t* 
                              uint32_t rows, uint32_t n, uint32_t ld, uint32_t stride, hipStream_t stream);
 hipError_t launch_reduce_tiles(const float* ws, uint32_t stride, uint32_t tiles, uint32_t c1, uint32_t c2, uint32_t c3,
                                float* g_down, float* gb_down, float* g_up, float* gb_up, hipStream_t stream);
-hipError_t launch_adamw(float* p, const float* g, float* m, float* v, uint32_t count, float lr_decay, float beta1,
-                        float one_minus_beta1, float beta2, float one_minus_beta2, float step_size, float bias2_sqrt, float eps,
-                        hipStream_t stream);
+// AdamW on up to kAdamArrays arrays in one launch.
+constexpr uint32_t kAdamArrays = 4;
+struct AdamArray {
+    float* p;
+    const float* g;
+    float *m, *v;
+    uint32_t count;
+};
+struct AdamScalars {
+    float lr_decay, beta1, one_minus_beta1, beta2, one_minus_beta2, step_size, bias2_sqrt, eps;
+};
+hipError_t launch_adamw(const AdamArray* arrays, uint32_t count, const AdamScalars& scalars, hipStream_t stream);
 hipError_t launch_gather_values(const float* src, const int32_t* pos, float* dst, uint32_t count, hipStream_t stream);
+// gy [n, d] -> gy_t [d, ld]; hid_val[i] = out_val[hid_pos[i]]; in_val[i] = up_val[in_pos[i]]: one launch.
+hipError_t launch_backward_prepare(const float* gy, float* gy_t, uint32_t n, uint32_t d, uint32_t ld, const float* out_val,
+                                   const int32_t* hid_pos, float* hid_val, uint32_t nnz_down, const float* up_val, const int32_t* in_pos,
+                                   float* in_val, uint32_t nnz_up, hipStream_t stream);
 
 // Output-major transpose of the hidden-major down store (stable in slot order).
 uint32_t output_major_chunks(uint32_t nnz);
@@ -133,6 +146,28 @@ hipError_t launch_train_forward(const float* x, const void* up_planes, const int
 hipError_t launch_train_backward(const float* gy, const float* z, const void* down_t_planes, const int32_t* down_t_exp,
                                  const void* up_t_planes, const int32_t* up_t_exp, void* workspace, float* gz, float* gx, uint32_t n,
                                  uint32_t d, uint32_t h, uint32_t ld, hipStream_t stream);
+
+// The same on planes densified per call from the compact rows (d and h multiples of 256, any n): the forward of
+// PrefillCall (float32) that also writes x_t, act and z; the backward that also writes gy_t, its sides densified from the
+// transposed supports, their values read in place by position. Workspace: train_planes_workspace_bytes, any content.
+struct TrainBackward {
+    const float *gy, *z;
+    const int32_t* hid_off;
+    const int16_t* hid_output;
+    const int32_t* hid_pos;
+    const float* out_val;
+    const int32_t* in_off;
+    const int16_t* in_hidden;
+    const int32_t* in_pos;
+    const float* up_val;
+    float *hid_val, *in_val;  // the values in the transposed orders, where a side gathers them first
+    void* workspace;
+    float *gy_t, *gz, *gx;
+    uint32_t d, h, nnz_up, nnz_down, n, ld;
+};
+uint64_t train_planes_workspace_bytes(uint32_t n, uint32_t d, uint32_t h);
+hipError_t launch_train_planes_forward(const PrefillCall& call, float* x_t, float* act, float* z, uint32_t ld, hipStream_t stream);
+hipError_t launch_train_planes_backward(const TrainBackward& call, hipStream_t stream);
 
 // Decode-sized projections over the same planes (gemv.hip): act token-major [n, h] (16-byte aligned), y token-major
 // [n, d]; `work` (gemv_workspace_bytes) holds the k-split partial sums.

@@ -100,6 +100,11 @@ __device__ __forceinline__ void split(float v, _Float16& hi, _Float16& lo) {
     lo = static_cast<_Float16>(v - static_cast<float>(hi));
 }
 
+// Whether column k of a B plane lies in an odd chain of 2^bits columns (the chained GEMMs; kNoChains: never).
+constexpr uint32_t kNoChains = 31;
+constexpr uint32_t chain_bits(uint32_t ktiles) { return ktiles == 1 ? 5 : 1 + chain_bits(ktiles / 2); }  // 32 k per k-tile
+__device__ __forceinline__ bool chain_odd(uint32_t k, uint32_t bits) { return (k >> bits) & 1u; }
+
 // Index of element (row, k) of part p (0 hi, 1 lo) in planes of `rows` rows.
 __device__ __forceinline__ size_t plane_at(uint32_t rows, uint32_t row, uint32_t k, uint32_t p) {
     return ((static_cast<size_t>(k / kBK) * kRuns + p * 4 + (k % kBK) / 8) * rows + row) * 8 + k % 8;
@@ -118,7 +123,7 @@ constexpr uint32_t kSplitWaves = kThreads / kWave;
 // The work of kThreads threads (tid) on row group `group`; part: their maxima in LDS. Every thread of the block calls it.
 __device__ __forceinline__ void split_rows(uint32_t (&part)[kSplitWaves][kSplitBlockRows], uint32_t tid, uint32_t group,
                                            const float* __restrict__ x, uint32_t M, uint32_t rows_pad, uint32_t K, uint32_t ld,
-                                           uint32_t k_real, _Float16* __restrict__ planes, int32_t* __restrict__ e) {
+                                           uint32_t k_real, uint32_t bits, _Float16* __restrict__ planes, int32_t* __restrict__ e) {
     constexpr uint32_t kWaves = kSplitWaves;
     const uint32_t lane = tid % kWave, wave = uniform(tid / kWave);
     const uint32_t r = lane % kSplitBlockRows, piece = lane / kSplitBlockRows;
@@ -176,14 +181,15 @@ __device__ __forceinline__ void split_rows(uint32_t (&part)[kSplitWaves][kSplitB
         for (int i = 0; i < 4; ++i) {
             if (k0 + 64 * i >= k_end) break;
             half8 h, l;
+            const uint32_t k = k0 + 64 * i + 8 * piece;
+            const float by = chain_odd(k, bits) ? -scale : scale;
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
                 _Float16 hh, ll;
-                split(v[i][q] * scale, hh, ll);
+                split(v[i][q] * by, hh, ll);
                 h[q] = hh;
                 l[q] = ll;
             }
-            const uint32_t k = k0 + 64 * i + 8 * piece;
             *reinterpret_cast<half8*>(planes + plane_at(rows_pad, row, k, 0)) = h;
             *reinterpret_cast<half8*>(planes + plane_at(rows_pad, row, k, 1)) = l;
         }
@@ -193,7 +199,18 @@ __global__ __launch_bounds__(kThreads) void split_rows_kernel(const float* __res
                                                              uint32_t K, uint32_t ld, uint32_t k_real, _Float16* __restrict__ planes,
                                                              int32_t* __restrict__ e) {
     __shared__ uint32_t part[kSplitWaves][kSplitBlockRows];
-    split_rows(part, threadIdx.x, blockIdx.x, x, M, rows_pad, K, ld, k_real, planes, e);
+    split_rows(part, threadIdx.x, blockIdx.x, x, M, rows_pad, K, ld, k_real, kNoChains, planes, e);
+}
+
+// Two matrices of the same columns in one launch (the operands of a sampled product).
+__global__ __launch_bounds__(kThreads) void split_pair_kernel(const float* __restrict__ a, uint32_t a_rows, _Float16* __restrict__ a_planes,
+                                                             int32_t* __restrict__ a_e, const float* __restrict__ b, uint32_t b_rows,
+                                                             _Float16* __restrict__ b_planes, int32_t* __restrict__ b_e, uint32_t K,
+                                                             uint32_t ld, uint32_t k_real, uint32_t b_bits) {
+    __shared__ uint32_t part[kSplitWaves][kSplitBlockRows];
+    const uint32_t a_blocks = a_rows / kSplitBlockRows;
+    if (blockIdx.x < a_blocks) split_rows(part, threadIdx.x, blockIdx.x, a, a_rows, a_rows, K, ld, k_real, kNoChains, a_planes, a_e);
+    else split_rows(part, threadIdx.x, blockIdx.x - a_blocks, b, b_rows, b_rows, K, ld, k_real, b_bits, b_planes, b_e);
 }
 
 // --------------------------------------------------------------------------------------------- densify
@@ -211,11 +228,22 @@ template <typename V>
 struct SlotPiece {
     static constexpr int kVals = 2 * static_cast<int>(sizeof(V));
     uint32_t ids[4], vals[kVals];
-    __device__ __forceinline__ void load(const int16_t* __restrict__ idx, const V* __restrict__ val, int32_t q, int32_t nnz, bool vec) {
+    // pos (float32, null for none): slot s holds val[pos[s]], one more load of the 8 positions, then 8 gathered values
+    __device__ __forceinline__ void load(const int16_t* __restrict__ idx, const V* __restrict__ val, const int32_t* __restrict__ pos,
+                                         int32_t q, int32_t nnz, bool vec) {
         const int32_t s = 8 * q;
         if (vec && s + 8 <= nnz) {
             const uint4 i4 = *reinterpret_cast<const uint4*>(idx + s);
             ids[0] = i4.x; ids[1] = i4.y; ids[2] = i4.z; ids[3] = i4.w;
+            if constexpr (sizeof(V) == 4) {
+                if (pos != nullptr) {
+                    const int4 a = *reinterpret_cast<const int4*>(pos + s), b = *reinterpret_cast<const int4*>(pos + s + 4);
+                    const int32_t at[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) vals[u] = __float_as_uint(val[at[u]]);
+                    return;
+                }
+            }
 #pragma unroll
             for (int p = 0; p < kVals; p += 4) {
                 const uint4 v4 = reinterpret_cast<const uint4*>(val + s)[p / 4];
@@ -233,7 +261,7 @@ struct SlotPiece {
             if (s + u < nnz) {
                 ids[u / 2] |= static_cast<uint32_t>(static_cast<uint16_t>(idx[s + u])) << (16 * (u % 2));
                 if constexpr (sizeof(V) == 2) vals[u / 2] |= static_cast<uint32_t>(val[s + u]) << (16 * (u % 2));
-                else vals[u] = __float_as_uint(val[s + u]);
+                else vals[u] = __float_as_uint(val[pos != nullptr ? pos[s + u] : s + u]);
             }
     }
     __device__ __forceinline__ uint32_t index(int u) const { return u % 2 ? ids[u / 2] >> 16 : ids[u / 2] & 0xffffu; }
@@ -251,14 +279,15 @@ struct RowSlots {
     static constexpr int32_t kStride = 2 * kWave;
     const int16_t* idx;
     const V* val;
+    const int32_t* pos;
     int32_t begin, end, first, last, nnz;
     bool vec;
     SlotPiece<V> held;
-    __device__ __forceinline__ RowSlots(const int16_t* __restrict__ i, const V* __restrict__ v, int32_t b, int32_t e, int32_t slots, bool aligned,
-                                        uint32_t half, uint32_t lane)
-        : idx(i), val(v), begin(b), end(e), first((b >> 3) + static_cast<int32_t>(half * kWave + lane)), last(e > b ? (e + 7) >> 3 : 0),
+    __device__ __forceinline__ RowSlots(const int16_t* __restrict__ i, const V* __restrict__ v, const int32_t* __restrict__ positions, int32_t b,
+                                        int32_t e, int32_t slots, bool aligned, uint32_t half, uint32_t lane)
+        : idx(i), val(v), pos(positions), begin(b), end(e), first((b >> 3) + static_cast<int32_t>(half * kWave + lane)), last(e > b ? (e + 7) >> 3 : 0),
           nnz(slots), vec(aligned) {
-        if (first < last) held.load(idx, val, first, nnz, vec);
+        if (first < last) held.load(idx, val, pos, first, nnz, vec);
     }
     // f(index, value, inside the row) of every slot of the lane's pieces
     template <typename F>
@@ -267,7 +296,7 @@ struct RowSlots {
         piece(held, first, f);
         for (int32_t q = first + kStride; q < last; q += kStride) {
             SlotPiece<V> p;
-            p.load(idx, val, q, nnz, vec);
+            p.load(idx, val, pos, q, nnz, vec);
             piece(p, q, f);
         }
     }
@@ -286,7 +315,9 @@ struct DensSide {
     const int32_t* off;
     const int16_t* idx;
     const void* val;
+    const int32_t* pos;          // null, or (float32) the slots' places in val
     uint32_t rows, rows_pad, k;  // real rows; rows and columns of the planes
+    uint32_t bits;               // chain_odd
     bool vec;
     _Float16* planes;
     int32_t* exps;
@@ -310,7 +341,7 @@ __device__ __forceinline__ void densify(DensTile& lds, const DensSide& side, uin
     const uint32_t width = min(kDensChunk, side.k - c0), pieces = width / 8;  // width: a multiple of 32
     // Waves w and w + kDensRows take row r0 + w. The two halves' maxima meet in LDS.
     const bool real = n < side.rows;
-    RowSlots<V> slots(side.idx, static_cast<const V*>(side.val), real ? side.off[n] : 0, real ? side.off[n + 1] : 0, side.off[side.rows],
+    RowSlots<V> slots(side.idx, static_cast<const V*>(side.val), side.pos, real ? side.off[n] : 0, real ? side.off[n + 1] : 0, side.off[side.rows],
                       side.vec, half, lane);
     // the tile zeroed while the slots are in flight
     for (uint32_t i = tid; i < PARTS * sizeof(tile[0]) / 16; i += kDensThreads) reinterpret_cast<uint4*>(tile)[i] = make_uint4(0, 0, 0, 0);
@@ -325,7 +356,7 @@ __device__ __forceinline__ void densify(DensTile& lds, const DensSide& side, uin
         // a slot of another row or column block goes to the row's padding, which nothing reads: no branch per slot
         const uint32_t c = column - c0, at = inside && c < width ? c : kDensChunk;
         _Float16 hi, lo;
-        split(ldexpf(v, -e), hi, lo);
+        split(ldexpf(chain_odd(column, side.bits) ? -v : v, -e), hi, lo);
         tile[0][row][at] = hi;
         if constexpr (PARTS == 2) tile[1][row][at] = lo;
     });
@@ -349,24 +380,35 @@ __global__ __launch_bounds__(kDensThreads, kDensOccupancy) void densify_kernel(D
 
 // What a call that densifies its own planes (launch_prefill) needs before its first GEMM, in one launch: the planes of
 // both sides from the compact rows and the input planes of x. Blocks 0 .. up_blocks - 1 densify W_up, the next
-// down_blocks W_down, the last split x, kSplitGroups groups of 8 rows a block. MI355X, at 128 / 2048 tokens: 9.9 / 7.4 us
+// down_blocks W_down, the next split_blocks split x, kSplitGroups groups of 8 rows a block (training: the others transpose
+// it). MI355X, at 128 / 2048 tokens: 9.9 / 7.4 us
 // on 512 x 2048 at 20 % (float32), 17.9 / 15.2 on 1024 x 4096 at 10 %, 38 / 46 on 2048 x 8192 at 20 % (bfloat16; 72 with
 // single slots a lane in place of 8, 2-byte loads). A block is a chain of four round trips (offsets, slots, LDS, stores).
 constexpr uint32_t kSplitGroups = kDensThreads / kThreads;
 template <typename V>
 __global__ __launch_bounds__(kDensThreads, kDensOccupancy) void prefill_prep_kernel(DensSide up, DensSide down, uint32_t up_blocks,
-                                                                                   uint32_t down_blocks, const float* __restrict__ x,
-                                                                                   uint32_t M, uint32_t rows_pad, uint32_t K, uint32_t ld,
-                                                                                   _Float16* __restrict__ planes, int32_t* __restrict__ e) {
+                                                                                   uint32_t down_blocks, uint32_t split_blocks,
+                                                                                   const float* __restrict__ x, uint32_t M,
+                                                                                   uint32_t rows_pad, uint32_t K, uint32_t ld,
+                                                                                   _Float16* __restrict__ planes, int32_t* __restrict__ e,
+                                                                                   float* __restrict__ x_t, uint32_t t_ld, uint32_t tiles_c,
+                                                                                   bool vectors) {
     constexpr uint32_t kParts = sizeof(V) == 2 ? 1 : 2;
     __shared__ __attribute__((aligned(16))) DensTile lds;
     if (blockIdx.x < up_blocks) return densify<V, kParts>(lds, up, blockIdx.x);
     if (blockIdx.x < up_blocks + down_blocks) return densify<V, kParts>(lds, down, blockIdx.x - up_blocks);
     using Parts = uint32_t[kSplitGroups][kSplitWaves][kSplitBlockRows];
     Parts& parts = reinterpret_cast<Parts&>(lds);
-    const uint32_t g = uniform(threadIdx.x / kThreads);
-    split_rows(parts[g], threadIdx.x % kThreads, (blockIdx.x - up_blocks - down_blocks) * kSplitGroups + g, x, M, rows_pad, K, ld, ld,
-               planes, e);
+    const uint32_t g = uniform(threadIdx.x / kThreads), block = blockIdx.x - up_blocks - down_blocks;
+    if (block < split_blocks) {
+        split_rows(parts[g], threadIdx.x % kThreads, block * kSplitGroups + g, x, M, rows_pad, K, ld, ld, kNoChains, planes, e);
+        return;
+    }
+    // training: x [M, ld] transposed too, a tile per group (a tile past the rows moves nothing)
+    static_assert(kThreads == kTransThreads && sizeof(TransposeTile) * kSplitGroups <= sizeof(DensTile), "a tile per group of threads");
+    const uint32_t tile = (block - split_blocks) * kSplitGroups + g;
+    transpose_tile(reinterpret_cast<TransposeTile*>(&lds)[g], threadIdx.x % kThreads, tile / tiles_c * kTransRows, tile % tiles_c * kTransCols, x,
+                   x_t, M, ld, ld, t_ld, vectors);
 }
 
 // ------------------------------------------------------------------------------------------------ GEMM
@@ -749,6 +791,10 @@ __device__ __forceinline__ void wait_stages(uint32_t later) {
 // three times as much as the tiles path it stands in for (2.05e-7); in chains of one activation block it keeps 2.0e-7, for
 // ~4 % of the GEMMs' time.
 //
+// The MFMAs' own sums are biased downwards (mean error -1.3e-8 of an output's deviation, whatever its sign), which a sum
+// over many tokens adds up: the b_up gradient of 2048 tokens lost 6.5e-7 where gathers lose 2.5e-7. So the B planes of
+// these calls hold -w in every odd chain's columns (chain_odd), whose sums are subtracted: the bias cancels.
+//
 // BM < 256 (those calls too): row tiles of 128 (waves of 32 x 64) or 64 (32 x 32), where 256 rows by 128 columns leave
 // CUs idle or would have to be split over K, with the partials' round trip and another launch. A k-tile of such a tile
 // is multiplied faster than its transfer arrives, so the ring holds as many stages as LDS takes. 768 x 3072 (float32) at
@@ -963,6 +1009,7 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
     const auto fold = [&](uint32_t kt) {
         if constexpr (FOLD) {
             if (!live) return;
+            const float sign = ((kt - 1) / CHAIN) & 1u ? -1.0f : 1.0f;  // odd chains: the B planes hold -w
             const uint32_t kb = (kt - 1) / kKtPerActBlock - kb0;
 #pragma unroll
             for (int i = 0; i < MIL; ++i)
@@ -973,11 +1020,11 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
                         e = *reinterpret_cast<const uint32_t*>(etab(kb) + wave_row<kWaveRows>(wm, i, 4 * g, lane));
 #pragma unroll
                     for (int b = 0; b < 4; ++b) {
-                        const float f = EPI == Epi::Down ? ldexpf(1.0f, static_cast<int8_t>(e >> (8 * b))) : 1.0f;
+                        const float f = EPI == Epi::Down ? ldexpf(sign, static_cast<int8_t>(e >> (8 * b))) : sign;
 #pragma unroll
                         for (int j = 0; j < NI; ++j) {
                             const int r = 4 * g + b;
-                            sum[i][j][r] = EPI == Epi::Down ? fmaf(acc[i][j][r], f, sum[i][j][r]) : sum[i][j][r] + acc[i][j][r];
+                            sum[i][j][r] = fmaf(acc[i][j][r], f, sum[i][j][r]);
                             acc[i][j][r] = 0.0f;
                         }
                     }
@@ -986,7 +1033,7 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
     };
     const auto rescale = [&](uint32_t kt) {
         if constexpr (FOLD) {
-            if ((kt - k_begin) % CHAIN == 0 && kt != k_begin) fold(kt);
+            if (kt % CHAIN == 0 && kt != k_begin) fold(kt);
         } else if constexpr (EPI == Epi::Down) {
             const uint32_t kb = kt / kKtPerActBlock - kb0;
             if (kt % kKtPerActBlock != 0 || kt == k_begin || !live) return;
@@ -1254,26 +1301,31 @@ __global__ __launch_bounds__(kThreads) void act_planes_kernel(const float* __res
 //            binades (read by the down GEMM);
 //   GradZ:   gz = sum * gelu'(z), z read hidden-major: gz hidden-major and as planes with block binades (read by the gx
 //            GEMM).
-// Blocks and threads as act_planes_kernel (16 tokens x one 128-neuron block; 16 threads per token, 8 neurons each). The
-// hidden-major rows go through LDS tiles [128 neurons][16 tokens]: thread i takes neuron i / 4 and tokens 4 (i % 4) ..
-// + 3, 16 bytes at a time (ld and the block's first token are multiples of 4, so a vector that starts below ld ends
-// below it); only tokens below M are written.
+// Threads as act_planes_kernel (16 per token, 8 neurons each), 32 tokens x one 128-neuron block. The hidden-major rows go
+// through LDS tiles [128 neurons][32 tokens]: thread i takes neuron i / 8 and tokens 4 (i % 8) .. + 3, 16 bytes at a time
+// (ld and the block's first token are multiples of 4, so a vector that starts below ld ends below it), a 128-byte line per
+// neuron; only tokens below M are written. Bound by memory (4 bytes a split read, 12
+// or 16 read or written per entry): MI355X, 2048 tokens x 4096 neurons, Forward / GradZ: 49 / 39 us in blocks of 16 tokens
+// (half lines, 4-byte stores), 27.6 / 26.3 us now.
+constexpr uint32_t kTrainRows = 32, kTrainThreads = kTrainRows * 16;
 enum class TrainPost { Forward, GradZ };
 template <TrainPost MODE>
-__global__ __launch_bounds__(kThreads) void train_planes_kernel(const float* __restrict__ partials, uint32_t splits,
+__global__ __launch_bounds__(kTrainThreads) void train_planes_kernel(const float* __restrict__ partials, uint32_t splits,
                                                                const float* __restrict__ b_up, const float* __restrict__ z_in,
                                                                float* __restrict__ out_a, float* __restrict__ out_b,
                                                                _Float16* __restrict__ planes, int8_t* __restrict__ exps, uint32_t M,
                                                                uint32_t rows_pad, uint32_t H, uint32_t ld) {
-    constexpr uint32_t R = kActRowsPerBlock;
-    static_assert(R == 16 && kActBlock * 4 % kThreads == 0, "16 tokens a block; the tile rows divide over the threads");
+    constexpr uint32_t R = kTrainRows, kQuads = R / 4;
+    static_assert(kActBlock * kQuads % kTrainThreads == 0, "the tile rows divide over the threads");
     __shared__ float ta[kActBlock][R + 1], tb[kActBlock][R + 1];  // Forward: z, act; GradZ: z, gz
+    __shared__ float scales[R];
     const uint32_t ml = threadIdx.x / 16, sub = threadIdx.x % 16;
     const uint32_t m0 = blockIdx.x * R, m = m0 + ml;
     const uint32_t nb = blockIdx.y, n0 = nb * kActBlock, n = n0 + sub * 8;
     if constexpr (MODE == TrainPost::GradZ) {
-        for (uint32_t i = threadIdx.x; i < kActBlock * 4; i += kThreads) {
-            const uint32_t r = i / 4, c = (i % 4) * 4;
+#pragma unroll
+        for (uint32_t i = threadIdx.x; i < kActBlock * kQuads; i += kTrainThreads) {
+            const uint32_t r = i / kQuads, c = (i % kQuads) * 4;
             float4 q = make_float4(0.f, 0.f, 0.f, 0.f);
             if (m0 + c < ld) q = *reinterpret_cast<const float4*>(z_in + static_cast<size_t>(n0 + r) * ld + m0 + c);
             ta[r][c] = q.x, ta[r][c + 1] = q.y, ta[r][c + 2] = q.z, ta[r][c + 3] = q.w;
@@ -1321,32 +1373,44 @@ __global__ __launch_bounds__(kThreads) void train_planes_kernel(const float* __r
     }
 #pragma unroll
     for (int off = 8; off >= 1; off >>= 1) largest = max(largest, static_cast<uint32_t>(__shfl_xor(static_cast<int>(largest), off, kWave)));
-    const int e = act_binade(largest);
-    if (sub == 0) exps[act_exp_at(rows_pad, m, nb)] = static_cast<int8_t>(e);
-    const float scale = ldexpf(1.0f, -e);
-    half8 hi, lo;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-        _Float16 hh, ll;
-        split(v[q] * scale, hh, ll);
-        hi[q] = hh;
-        lo[q] = ll;
+    if (sub == 0) {
+        const int e = act_binade(largest);
+        exps[act_exp_at(rows_pad, m, nb)] = static_cast<int8_t>(e);
+        scales[ml] = ldexpf(1.0f, -e);
     }
-    *reinterpret_cast<half8*>(planes + plane_at(rows_pad, m, n, 0)) = hi;
-    *reinterpret_cast<half8*>(planes + plane_at(rows_pad, m, n, 1)) = lo;
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < kActBlock * 4; i += kThreads) {
-        const uint32_t r = i / 4, c = (i % 4) * 4;
-        const size_t at = static_cast<size_t>(n0 + r) * ld + m0 + c;
+    {  // the planes from the tile, token by token: 32 tokens' 16 bytes of a chunk follow one another
+        const uint32_t t = threadIdx.x % R, chunk = threadIdx.x / R;
+        const float scale = scales[t];
+        half8 hi, lo;
 #pragma unroll
-        for (uint32_t q = 0; q < 4; ++q) {
-            if (m0 + c + q >= M) break;
-            if constexpr (MODE == TrainPost::Forward) {
-                out_a[at + q] = ta[r][c + q];
-                out_b[at + q] = tb[r][c + q];
+        for (int q = 0; q < 8; ++q) {
+            _Float16 hh, ll;
+            split(tb[chunk * 8 + q][t] * scale, hh, ll);
+            hi[q] = hh;
+            lo[q] = ll;
+        }
+        *reinterpret_cast<half8*>(planes + plane_at(rows_pad, m0 + t, n0 + chunk * 8, 0)) = hi;
+        *reinterpret_cast<half8*>(planes + plane_at(rows_pad, m0 + t, n0 + chunk * 8, 1)) = lo;
+    }
+#pragma unroll
+    for (uint32_t i = threadIdx.x; i < kActBlock * kQuads; i += kTrainThreads) {
+        const uint32_t r = i / kQuads, c = (i % kQuads) * 4;
+        const size_t at = static_cast<size_t>(n0 + r) * ld + m0 + c;
+        const auto row = [&](float* __restrict__ to, const float (&from)[R + 1]) {
+            if (m0 + c + 4 <= M) {
+                *reinterpret_cast<float4*>(to + at) = make_float4(from[c], from[c + 1], from[c + 2], from[c + 3]);
             } else {
-                out_a[at + q] = tb[r][c + q];
+#pragma unroll
+                for (uint32_t q = 0; q < 3; ++q)
+                    if (m0 + c + q < M) to[at + q] = from[c + q];
             }
+        };
+        if constexpr (MODE == TrainPost::Forward) {
+            row(out_a, ta[r]);
+            row(out_b, tb[r]);
+        } else {
+            row(out_a, tb[r]);
         }
     }
 }
@@ -1658,62 +1722,15 @@ Workspace workspace_layout(uint32_t m, uint32_t d, uint32_t h, bool training = f
 
 }  // namespace
 
+namespace {
+size_t align256(size_t v) { return (v + 255) / 256 * 256; }
+}  // namespace
+
 size_t dense_plane_halves(uint32_t rows, uint32_t k) { return static_cast<size_t>(rows) * k * 2; }
 
 bool mfma_shape_supported(uint32_t d, uint32_t h) { return d % 256 == 0 && h % 256 == 0; }
 
 bool mfma_streamed(uint32_t n, uint32_t d, uint32_t h) { return dma_up_splits(n, h, d) != 0 && dma_down_splits(n, d, h) != 0; }
-
-// Workspace of the dense sampled product (bytes, 256-aligned parts): the planes of A [rows, k_pad] and B [cols,
-// k_pad] (tokens padded to a multiple of 256, split_rows' k granularity), their row binades and the GEMM's partials.
-namespace {
-struct GradDenseLayout {
-    size_t a_planes, b_planes, a_exp, b_exp, partials, bytes;
-    uint32_t k_pad, splits;
-};
-size_t align256(size_t v) { return (v + 255) / 256 * 256; }
-GradDenseLayout grad_dense_layout(uint32_t rows, uint32_t cols, uint32_t n) {
-    GradDenseLayout l{};
-    l.k_pad = ceil_div(n, 256) * 256;
-    l.splits = dma_up_splits(rows, cols, l.k_pad);
-    l.a_planes = 0;
-    l.b_planes = align256(l.a_planes + dense_plane_halves(rows, l.k_pad) * 2);
-    l.a_exp = align256(l.b_planes + dense_plane_halves(cols, l.k_pad) * 2);
-    l.b_exp = align256(l.a_exp + static_cast<size_t>(rows) * 4);
-    l.partials = align256(l.b_exp + static_cast<size_t>(cols) * 4);
-    l.bytes = l.partials + static_cast<size_t>(l.splits) * rows * cols * 4;
-    return l;
-}
-}  // namespace
-
-size_t grad_dense_workspace_bytes(uint32_t rows, uint32_t cols, uint32_t n) {
-    if (rows % kRowPad != 0 || cols % kDmaBN != 0) return 0;
-    const GradDenseLayout l = grad_dense_layout(rows, cols, n);
-    return l.splits == 0 ? 0 : l.bytes;
-}
-
-hipError_t launch_grad_dense(const float* row, const float* mat, const int32_t* off, const int16_t* idx, float* g, float* gb,
-                             uint32_t rows, uint32_t cols, uint32_t n, uint32_t ld, void* workspace, hipStream_t stream) {
-    const GradDenseLayout l = grad_dense_layout(rows, cols, n);
-    char* w = static_cast<char*>(workspace);
-    auto* a_planes = reinterpret_cast<_Float16*>(w + l.a_planes);
-    auto* b_planes = reinterpret_cast<_Float16*>(w + l.b_planes);
-    auto* a_exp = reinterpret_cast<int32_t*>(w + l.a_exp);
-    auto* b_exp = reinterpret_cast<int32_t*>(w + l.b_exp);
-    auto* partials = reinterpret_cast<float*>(w + l.partials);
-    hipLaunchKernelGGL(split_rows_kernel, dim3(rows / kSplitBlockRows), dim3(kThreads), 0, stream, row, rows, rows, l.k_pad, ld, n,
-                       a_planes, a_exp);
-    hipLaunchKernelGGL(split_rows_kernel, dim3(cols / kSplitBlockRows), dim3(kThreads), 0, stream, mat, cols, cols, l.k_pad, ld, n,
-                       b_planes, b_exp);
-    if (hipError_t status = hipGetLastError(); status != hipSuccess) return status;
-    if (hipError_t status = launch_dma<Epi::UpSplit, true>(a_planes, a_exp, b_planes, b_exp, nullptr, partials, nullptr, nullptr, rows,
-                                                           cols, l.k_pad, l.splits, stream);
-        status != hipSuccess)
-        return status;
-    hipLaunchKernelGGL(gather_dense_kernel, dim3(ceil_div(rows, kThreads / kWave)), dim3(kThreads), 0, stream, partials, l.splits, row,
-                       ld, n, off, idx, g, gb, rows, cols);
-    return hipGetLastError();
-}
 
 size_t mfma_workspace_bytes(uint32_t n, uint32_t d, uint32_t h) { return workspace_layout(n, d, h).bytes; }
 
@@ -1726,7 +1743,7 @@ bool slots_aligned(const void* idx, const void* val) {
 hipError_t launch_densify(int vt, const int32_t* off, const int16_t* idx, const void* val, uint32_t rows, uint32_t k,
                           void* planes, int32_t* exps, hipStream_t stream) {
     const dim3 grid(dens_blocks(rows, k)), block(kDensThreads);
-    const DensSide side{off, idx, val, rows, rows, k, slots_aligned(idx, val), static_cast<_Float16*>(planes), exps};
+    const DensSide side{off, idx, val, nullptr, rows, rows, k, kNoChains, slots_aligned(idx, val), static_cast<_Float16*>(planes), exps};
     if (vt == kBF16) hipLaunchKernelGGL((densify_kernel<uint16_t>), grid, block, 0, stream, side);
     else hipLaunchKernelGGL((densify_kernel<float>), grid, block, 0, stream, side);
     return hipGetLastError();
@@ -1812,7 +1829,7 @@ hipError_t launch_mfma_down(int vt, const void* planes, const int32_t* v_exp, co
 // 2.38e-7; the bfloat16 1.4B shape the other way, 2.16e-7 -> 2.23e-7). Calls above kPrefillPiece tokens run in pieces over the
 // same planes, which bounds the workspace.
 constexpr uint32_t kPrefillPiece = 16384;
-constexpr int kPrefillDownChain = kKtPerActBlock;
+constexpr int kPrefillDownChain = kKtPerActBlock, kUpChainF32 = kKtPerActBlock / 2, kUpChainBf16 = kKtPerActBlock;
 constexpr uint32_t kPrefillDownBlocks = 16;  // activation blocks of a down split: longer sums lose more than the tiles path
 constexpr uint32_t pad256(uint32_t v) { return (v + 255) / 256 * 256; }
 
@@ -1858,11 +1875,12 @@ struct PrefillLayout {
     size_t up_planes, up_exp, down_planes, down_exp, x_exp, act_exp, x_planes, act_planes, partials, bytes;
 };
 // Byte offsets (256-byte aligned) for calls of up to n tokens; the partials hold the largest of any smaller call's.
-PrefillLayout prefill_layout(bool bf16, uint32_t n, uint32_t d, uint32_t h) {
+// training: not in pieces, and the up projection's sums always go through the partials.
+PrefillLayout plan_layout(bool bf16, bool training, uint32_t n, uint32_t d, uint32_t h) {
     PrefillLayout l{};
     l.d = pad256(d);
     l.h = pad256(h);
-    n = min(n, kPrefillPiece);
+    if (!training) n = min(n, kPrefillPiece);
     const size_t rows = rows_padded(n);
     size_t at = 0;
     const auto take = [&at](size_t bytes) {
@@ -1881,7 +1899,7 @@ PrefillLayout prefill_layout(bool bf16, uint32_t n, uint32_t d, uint32_t h) {
     size_t most = 0;
     for (uint32_t m = 128; m <= max(rows, size_t{128}); m += m == 128 ? 128 : kRowPad) {
         const PrefillPlan plan = prefill_plan(m, l.d, l.h, bf16);
-        if (plan.up.splits > 1) most = max(most, static_cast<size_t>(plan.up.splits) * min(m, n) * l.h);
+        if (training || plan.up.splits > 1) most = max(most, static_cast<size_t>(plan.up.splits) * min(m, n) * l.h);
         if (plan.down.splits > 1) most = max(most, static_cast<size_t>(plan.down.splits) * min(m, n) * l.d);
     }
     l.partials = take(most * 4);
@@ -1889,27 +1907,44 @@ PrefillLayout prefill_layout(bool bf16, uint32_t n, uint32_t d, uint32_t h) {
     return l;
 }
 
-uint64_t prefill_workspace_bytes(int vt, uint32_t n, uint32_t d, uint32_t h) { return prefill_layout(vt == kBF16, n, d, h).bytes; }
+// The last layouts of the thread by their arguments (each plans every row count up to n: ~10 us of host time at 2048).
+PrefillLayout prefill_layout(bool bf16, bool training, uint32_t n, uint32_t d, uint32_t h) {
+    struct Entry {
+        bool bf16, training;
+        uint32_t n, d, h;
+        PrefillLayout layout;
+    };
+    thread_local Entry entries[8] = {};
+    thread_local uint32_t next = 0;
+    for (const Entry& e : entries)
+        if (e.n == n && e.d == d && e.h == h && e.bf16 == bf16 && e.training == training) return e.layout;
+    Entry& e = entries[next++ % 8];
+    e = {bf16, training, n, d, h, plan_layout(bf16, training, n, d, h)};
+    return e.layout;
+}
+
+uint64_t prefill_workspace_bytes(int vt, uint32_t n, uint32_t d, uint32_t h) { return prefill_layout(vt == kBF16, false, n, d, h).bytes; }
 
 namespace {
 template <typename V>
 hipError_t prefill(const PrefillCall& c, hipStream_t stream) {
     constexpr bool kLoB = sizeof(V) == 4;
-    constexpr int kUpChain = kLoB ? kKtPerActBlock / 2 : kKtPerActBlock;
-    const PrefillLayout l = prefill_layout(!kLoB, c.n, c.d, c.h);
+    constexpr int kUpChain = kLoB ? kUpChainF32 : kUpChainBf16;
+    const PrefillLayout l = prefill_layout(!kLoB, false, c.n, c.d, c.h);
     char* w = static_cast<char*>(c.workspace);
     const auto halves = [&](size_t at) { return reinterpret_cast<_Float16*>(w + at); };
     const auto words = [&](size_t at) { return reinterpret_cast<int32_t*>(w + at); };
     float* partials = reinterpret_cast<float*>(w + l.partials);
-    const DensSide up{c.up_off, c.up_idx, c.up_val, c.h, l.h, l.d, slots_aligned(c.up_idx, c.up_val), halves(l.up_planes), words(l.up_exp)};
-    const DensSide down{c.down_off, c.down_idx, c.down_val, c.d, l.d, l.h, slots_aligned(c.down_idx, c.down_val), halves(l.down_planes), words(l.down_exp)};
+    const DensSide up{c.up_off, c.up_idx, c.up_val, nullptr, c.h, l.h, l.d, chain_bits(kUpChain), slots_aligned(c.up_idx, c.up_val), halves(l.up_planes), words(l.up_exp)};
+    const DensSide down{c.down_off, c.down_idx, c.down_val, nullptr, c.d, l.d, l.h, chain_bits(kPrefillDownChain), slots_aligned(c.down_idx, c.down_val), halves(l.down_planes), words(l.down_exp)};
     for (uint32_t t0 = 0; t0 < c.n; t0 += kPrefillPiece) {
         const uint32_t n = min(kPrefillPiece, c.n - t0), rows = rows_padded(n), split_blocks = rows_live(n) / kSplitBlockRows / kSplitGroups;
         const uint32_t up_blocks = t0 == 0 ? dens_blocks(l.h, l.d) : 0, down_blocks = t0 == 0 ? dens_blocks(l.d, l.h) : 0;
         const float* x = c.x + static_cast<size_t>(t0) * c.d;
         float* y = c.y + static_cast<size_t>(t0) * c.d;
         hipLaunchKernelGGL(prefill_prep_kernel<V>, dim3(up_blocks + down_blocks + split_blocks), dim3(kDensThreads), 0, stream, up, down,
-                           up_blocks, down_blocks, x, n, rows, l.d, c.d, halves(l.x_planes), words(l.x_exp));
+                           up_blocks, down_blocks, split_blocks, x, n, rows, l.d, c.d, halves(l.x_planes), words(l.x_exp),
+                           static_cast<float*>(nullptr), 0u, 1u, false);
         if (hipError_t status = hipGetLastError(); status != hipSuccess) return status;
         const PrefillPlan plan = prefill_plan(n, l.d, l.h, !kLoB);
         const bool split = plan.up.splits > 1;
@@ -1941,6 +1976,56 @@ hipError_t launch_prefill(int vt, const PrefillCall& call, hipStream_t stream) {
     return vt == kBF16 ? prefill<uint16_t>(call, stream) : prefill<float>(call, stream);
 }
 
+// Workspace of the dense sampled product (bytes, 256-aligned parts): the planes of A [rows, k_pad] and B [cols,
+// k_pad] (tokens padded to a multiple of 256, split_rows' k granularity), their row binades and the GEMM's partials. The GEMM
+// takes the chained tiles: 2048 tokens on 1024 x 4096 are 128 tiles of 256 rows, half of the CUs, and 256 of 128 rows.
+namespace {
+struct GradDenseLayout {
+    size_t a_planes, b_planes, a_exp, b_exp, partials, bytes;
+    uint32_t k_pad;
+    ChainPlan plan;
+};
+GradDenseLayout grad_dense_layout(uint32_t rows, uint32_t cols, uint32_t n) {
+    GradDenseLayout l{};
+    l.k_pad = ceil_div(n, 256) * 256;
+    l.plan = chain_plan(rows, cols, l.k_pad, false, 1, 1);
+    l.a_planes = 0;
+    l.b_planes = align256(l.a_planes + dense_plane_halves(rows, l.k_pad) * 2);
+    l.a_exp = align256(l.b_planes + dense_plane_halves(cols, l.k_pad) * 2);
+    l.b_exp = align256(l.a_exp + static_cast<size_t>(rows) * 4);
+    l.partials = align256(l.b_exp + static_cast<size_t>(cols) * 4);
+    l.bytes = l.partials + static_cast<size_t>(l.plan.splits) * rows * cols * 4;
+    return l;
+}
+}  // namespace
+
+size_t grad_dense_workspace_bytes(uint32_t rows, uint32_t cols, uint32_t n) {
+    if (rows % kRowPad != 0 || cols % kDmaBN != 0) return 0;
+    // (few tiles: the gather is the better one)
+    return dma_up_splits(rows, cols, ceil_div(n, 256) * 256) == 0 ? 0 : grad_dense_layout(rows, cols, n).bytes;
+}
+
+hipError_t launch_grad_dense(const float* row, const float* mat, const int32_t* off, const int16_t* idx, float* g, float* gb,
+                             uint32_t rows, uint32_t cols, uint32_t n, uint32_t ld, void* workspace, hipStream_t stream) {
+    const GradDenseLayout l = grad_dense_layout(rows, cols, n);
+    char* w = static_cast<char*>(workspace);
+    auto* a_planes = reinterpret_cast<_Float16*>(w + l.a_planes);
+    auto* b_planes = reinterpret_cast<_Float16*>(w + l.b_planes);
+    auto* a_exp = reinterpret_cast<int32_t*>(w + l.a_exp);
+    auto* b_exp = reinterpret_cast<int32_t*>(w + l.b_exp);
+    auto* partials = reinterpret_cast<float*>(w + l.partials);
+    hipLaunchKernelGGL(split_pair_kernel, dim3((rows + cols) / kSplitBlockRows), dim3(kThreads), 0, stream, row, rows, a_planes, a_exp, mat, cols,
+                       b_planes, b_exp, l.k_pad, ld, n, chain_bits(kUpChainF32));
+    if (hipError_t status = hipGetLastError(); status != hipSuccess) return status;
+    if (hipError_t status = launch_chained<Epi::UpSplit, true, kUpChainF32>(l.plan.bm, a_planes, a_exp, b_planes, b_exp, nullptr, partials,
+                                                                            nullptr, nullptr, rows, cols, l.k_pad, l.plan.splits, cols, stream);
+        status != hipSuccess)
+        return status;
+    hipLaunchKernelGGL(gather_dense_kernel, dim3(ceil_div(rows, kThreads / kWave)), dim3(kThreads), 0, stream, partials, l.plan.splits, row,
+                       ld, n, off, idx, g, gb, rows, cols);
+    return hipGetLastError();
+}
+
 size_t train_mfma_workspace_bytes(uint32_t n, uint32_t d, uint32_t h) { return workspace_layout(n, d, h, true).bytes; }
 
 // Training forward on the planes (fp32 weights): x split into planes, the up projection as a split product (partials
@@ -1965,11 +2050,101 @@ hipError_t launch_train_forward(const float* x, const void* up_planes, const int
                                                            nullptr, partials, nullptr, nullptr, n, h, d, splits, stream);
         status != hipSuccess)
         return status;
-    hipLaunchKernelGGL(train_planes_kernel<TrainPost::Forward>, dim3(rows_live(n) / kActRowsPerBlock, h / kActBlock), dim3(kThreads), 0,
+    hipLaunchKernelGGL(train_planes_kernel<TrainPost::Forward>, dim3(rows_live(n) / kTrainRows, h / kActBlock), dim3(kTrainThreads), 0,
                        stream, partials, splits, b_up, nullptr, z, act, act_planes, reinterpret_cast<int8_t*>(words + w.act_binades), n,
                        rows_padded(n), h, ld);
     if (hipError_t status = hipGetLastError(); status != hipSuccess) return status;
     return launch_mfma_down(kF32, down_planes, down_exp, b_down, y, workspace, n, d, h, stream);
+}
+
+// Training on planes densified per call, in the workspace of the training layout (train_planes_workspace_bytes): the
+// chained GEMMs, as launch_prefill. `in` is x or gy; the sides are W_up and W_down, or W_down^T and W_up^T.
+namespace {
+struct TrainWork {
+    PrefillLayout l;
+    _Float16 *in_planes, *mid_planes;
+    int32_t *in_exp, *mid_exp;
+    float* partials;
+    DensSide first, second;  // [h rows, d k] and [d rows, h k]
+};
+TrainWork train_work(void* workspace, uint32_t n, uint32_t d, uint32_t h) {
+    const PrefillLayout l = prefill_layout(false, true, n, d, h);
+    char* w = static_cast<char*>(workspace);
+    const auto halves = [&](size_t at) { return reinterpret_cast<_Float16*>(w + at); };
+    const auto words = [&](size_t at) { return reinterpret_cast<int32_t*>(w + at); };
+    TrainWork t{l, halves(l.x_planes), halves(l.act_planes), words(l.x_exp), words(l.act_exp), reinterpret_cast<float*>(w + l.partials), {}, {}};
+    t.first = {nullptr, nullptr, nullptr, nullptr, h, l.h, l.d, chain_bits(kUpChainF32), true, halves(l.up_planes), words(l.up_exp)};
+    t.second = {nullptr, nullptr, nullptr, nullptr, d, l.d, l.h, chain_bits(kPrefillDownChain), true, halves(l.down_planes), words(l.down_exp)};
+    return t;
+}
+void set_slots(DensSide& side, const int32_t* off, const int16_t* idx, const float* val, const int32_t* pos) {
+    side.off = off, side.idx = idx, side.val = val, side.pos = pos;
+    side.vec = slots_aligned(idx, pos != nullptr ? static_cast<const void*>(pos) : val);
+}
+// Whether densifying reads a side's values by position as it goes, or from a copy gathered first: a block of each column
+// chunk reads its rows' slots, twice where a wave does not hold them, and a gathered 4-byte read costs a cache line. 1024 x
+// 4096 at 512 and 2048 tokens: up_t at 50 % (2 chunks of rows of 2048 slots, 8.4 M reads) 68 us in place, 14.6 + 12 us
+// gathered first; at 10 % (0.84 M reads) in place costs the launch 4 us, gathering first 4.8 and a launch.
+bool gathers_in_place(const DensSide& side, uint32_t nnz) {
+    const uint32_t reads = ceil_div(side.k, kDensChunk) * (nnz / side.rows > 1016 ? 2 : 1);
+    return reads == 1 || static_cast<uint64_t>(reads) * nnz <= 1u << 20;
+}
+hipError_t train_prep(const TrainWork& t, const float* in, float* in_t, uint32_t n, uint32_t d, uint32_t ld, hipStream_t stream) {
+    const uint32_t up_blocks = dens_blocks(t.l.h, t.l.d), down_blocks = dens_blocks(t.l.d, t.l.h);
+    const uint32_t split_blocks = rows_live(n) / kSplitBlockRows / kSplitGroups, tiles_c = d / kTransCols;
+    hipLaunchKernelGGL(prefill_prep_kernel<float>,
+                       dim3(up_blocks + down_blocks + split_blocks + ceil_div(tiles_c * ceil_div(n, kTransRows), kSplitGroups)), dim3(kDensThreads),
+                       0, stream, t.first, t.second, up_blocks, down_blocks, split_blocks, in, n, rows_padded(n), t.l.d, d, t.in_planes, t.in_exp,
+                       in_t, ld, tiles_c, transpose_vectors(in, in_t, d, ld));
+    return hipGetLastError();
+}
+// partials = in [n, d] first^T, then the epilogue MODE (train_planes_kernel); out = mid [n, h] second^T (+ bias)
+template <TrainPost MODE>
+hipError_t train_products(const TrainWork& t, const float* b_up, const float* z_in, float* out_a, float* out_b, const float* bias, float* out,
+                          uint32_t n, uint32_t d, uint32_t h, uint32_t ld, hipStream_t stream) {
+    const PrefillPlan plan = prefill_plan(n, t.l.d, t.l.h, false);
+    if (hipError_t status = launch_chained<Epi::UpSplit, true, kUpChainF32>(plan.up.bm, t.in_planes, t.in_exp, t.first.planes, t.first.exps,
+                                                                            nullptr, t.partials, nullptr, nullptr, n, h, d, plan.up.splits, h,
+                                                                            stream);
+        status != hipSuccess)
+        return status;
+    hipLaunchKernelGGL(train_planes_kernel<MODE>, dim3(rows_live(n) / kTrainRows, h / kActBlock), dim3(kTrainThreads), 0, stream, t.partials,
+                       plan.up.splits, b_up, z_in, out_a, out_b, t.mid_planes, reinterpret_cast<int8_t*>(t.mid_exp), n, rows_padded(n), h, ld);
+    if (hipError_t status = hipGetLastError(); status != hipSuccess) return status;
+    const bool parts = plan.down.splits > 1;
+    if (hipError_t status = launch_chained<Epi::Down, true, kPrefillDownChain>(plan.down.bm, t.mid_planes, t.mid_exp, t.second.planes,
+                                                                               t.second.exps, bias, parts ? t.partials : out, nullptr, nullptr,
+                                                                               n, d, h, plan.down.splits, d, stream);
+        status != hipSuccess || !parts)
+        return status;
+    return launch_reduce_splits(t.partials, bias, out, n, plan.down.splits, d, 0, d, stream);
+}
+}  // namespace
+
+uint64_t train_planes_workspace_bytes(uint32_t n, uint32_t d, uint32_t h) { return prefill_layout(false, true, n, d, h).bytes; }
+
+hipError_t launch_train_planes_forward(const PrefillCall& c, float* x_t, float* act, float* z, uint32_t ld, hipStream_t stream) {
+    TrainWork t = train_work(c.workspace, c.n, c.d, c.h);
+    set_slots(t.first, c.up_off, c.up_idx, static_cast<const float*>(c.up_val), nullptr);
+    set_slots(t.second, c.down_off, c.down_idx, static_cast<const float*>(c.down_val), nullptr);
+    if (hipError_t status = train_prep(t, c.x, x_t, c.n, c.d, ld, stream); status != hipSuccess) return status;
+    return train_products<TrainPost::Forward>(t, c.b_up, nullptr, z, act, c.b_down, c.y, c.n, c.d, c.h, ld, stream);
+}
+
+hipError_t launch_train_planes_backward(const TrainBackward& c, hipStream_t stream) {
+    TrainWork t = train_work(c.workspace, c.n, c.d, c.h);
+    const auto side = [&](DensSide& to, const int32_t* off, const int16_t* idx, const int32_t* pos, const float* val, float* values, uint32_t nnz) {
+        if (gathers_in_place(to, nnz)) {
+            set_slots(to, off, idx, val, pos);
+            return hipSuccess;
+        }
+        set_slots(to, off, idx, values, nullptr);
+        return launch_gather_values(val, pos, values, nnz, stream);
+    };
+    if (hipError_t status = side(t.first, c.hid_off, c.hid_output, c.hid_pos, c.out_val, c.hid_val, c.nnz_down); status != hipSuccess) return status;
+    if (hipError_t status = side(t.second, c.in_off, c.in_hidden, c.in_pos, c.up_val, c.in_val, c.nnz_up); status != hipSuccess) return status;
+    if (hipError_t status = train_prep(t, c.gy, c.gy_t, c.n, c.d, c.ld, stream); status != hipSuccess) return status;
+    return train_products<TrainPost::GradZ>(t, nullptr, c.z, c.gz, nullptr, nullptr, c.gx, c.n, c.d, c.h, c.ld, stream);
 }
 
 // Training backward products on the planes: gy split into planes; gz = (gy W_down) * gelu'(z) as a split product over
@@ -1992,7 +2167,7 @@ hipError_t launch_train_backward(const float* gy, const float* z, const void* do
                                                            down_t_exp, nullptr, partials, nullptr, nullptr, n, h, d, splits, stream);
         status != hipSuccess)
         return status;
-    hipLaunchKernelGGL(train_planes_kernel<TrainPost::GradZ>, dim3(rows_live(n) / kActRowsPerBlock, h / kActBlock), dim3(kThreads), 0,
+    hipLaunchKernelGGL(train_planes_kernel<TrainPost::GradZ>, dim3(rows_live(n) / kTrainRows, h / kActBlock), dim3(kTrainThreads), 0,
                        stream, partials, splits, nullptr, z, gz, nullptr, gz_planes, reinterpret_cast<int8_t*>(words + w.act_binades), n,
                        rows_padded(n), h, ld);
     if (hipError_t status = hipGetLastError(); status != hipSuccess) return status;

@@ -20,11 +20,13 @@ partials ``[tiles, columns]`` of the gather sampled products, and the workspace 
 The step: ``hffn_forward_z`` (the runtime's gather forward writing ``z``); the sampled products ``g_down``/``gb_down``
 and ``g_up``/``gb_up`` as gathers over 256-token tiles (``hffn_grad_sddmm``, tiles added in order by
 ``hffn_reduce_tiles``) or, from ``GRAD_DENSE_MIN_TOKENS`` tokens on dense enough layers, as split-fp16 MFMA products
-sampled at the support (``hffn_grad_dense``); ``gz`` by ``hffn_grad_hidden``; ``gx`` by ``hffn_grad_x``; AdamW per
-array by ``hffn_adamw``. After an update the runtime's densified planes of that layer are rebuilt before their next use.
-On layers whose runtime holds densified planes, from ``TRAIN_MFMA_MIN_TOKENS`` tokens (``train_mode``), the forward
-with z (``hffn_forward_mfma_z``) and gz, gx (``hffn_backward_mfma``) run as split-fp16 MFMA products instead, the
-backward over planes of W_down^T and W_up^T densified at every backward from the values in the transposed orders.
+sampled at the support (``hffn_grad_dense``); ``gz`` by ``hffn_grad_hidden``; ``gx`` by ``hffn_grad_x``; AdamW in
+one launch (``hffn_adamw_arrays``). After an update the runtime's densified planes of that layer are rebuilt before their next use.
+From ``TRAIN_MFMA_MIN_TOKENS`` tokens (``train_mode``) the forward with z, gz and gx run as split-fp16 MFMA products
+instead: the forward on the runtime's densified planes where it holds them (``hffn_forward_mfma_z``), else, where
+estimated faster than the gathers, on planes densified for the call (``hffn_forward_planes_z``); the backward always on
+planes of W_down^T and W_up^T densified for the call, the values read from the compact arrays by position
+(``hffn_backward_planes``), so that the values in the transposed orders are gathered by the gather backward only.
 """
 from __future__ import annotations
 
@@ -36,7 +38,8 @@ from dataclasses import dataclass
 import torch
 
 from . import _lib
-from .runtime import MAX_TOKENS, PAIR_MODES, HFFNRuntime, _aligned, down_mode, edges_supported, leading_dim, mfma_streamed, up_mode
+from .runtime import (MAX_TOKENS, PAIR_MODES, ROWS_SHARE, ROWS_WALK_SLOT_US, ROWS_WALK_US, HFFNRuntime, _aligned, down_mode,
+                      edges_supported, leading_dim, mfma_streamed, prefill_us, rows_us, up_mode)
 
 PARAMETERS = ("up_val", "b_up", "out_val", "b_down")
 SUPPORTS = ("in_offsets", "in_pos", "in_hidden", "hid_offsets", "hid_pos", "hid_output")
@@ -85,7 +88,7 @@ class _LayerState:
     supports: dict
     values: dict          # in_val, hid_val: the compact values in the transposed orders
     columns: tuple        # g_down [0, c1), gb_down [c1, c2), g_up [c2, c3), gb_up [c3, width) of the partials
-    planes_t: dict | None = None  # planes of W_down^T and W_up^T (the MFMA backward), allocated by reserve
+    adamw: tuple          # hffn_adamw_arrays' arrays: values, gradients, first and second moments, counts
 
 
 class HFFNTrainRuntime:
@@ -102,7 +105,10 @@ class HFFNTrainRuntime:
         self.calls: Counter = Counter()        # (up, down) of the forwards that kept z
         self.forced_grad: str | None = None    # diagnostic: the sampled products' formulation, else the policy's
         self.forced_train: str | None = None   # diagnostic: the forward with z, gz and gx on gathers or planes
-        self._mfma_work: torch.Tensor | None = None
+        self._mfma_work: torch.Tensor | None = None    # forward on the runtime's planes
+        self._planes_work: torch.Tensor | None = None  # planes densified per call
+        self._planes_shapes = bool(self._lib.hffn_mfma_supported(self.d_model, self.d_ff))
+        self._modes: dict = {}                  # (what, N, forced) -> mode
         self._tokens = 0                        # N the dense buffers hold
         self._tiles = 1                         # token tiles the partials hold (none allocated for 1)
         self._partials: torch.Tensor | None = None
@@ -129,11 +135,15 @@ class HFFNTrainRuntime:
         c1 = arrays["out_val"].numel()
         c2 = c1 + self.d_model
         c3 = c2 + arrays["up_val"].numel()
-        return _LayerState(grads={name: torch.zeros_like(arrays[name]) for name in PARAMETERS},
-                           moments={name: (torch.zeros_like(arrays[name]), torch.zeros_like(arrays[name])) for name in PARAMETERS},
-                           supports=supports,
+        grads = {name: torch.zeros_like(arrays[name]) for name in PARAMETERS}
+        moments = {name: (torch.zeros_like(arrays[name]), torch.zeros_like(arrays[name])) for name in PARAMETERS}
+        pointers = ctypes.c_void_p * len(PARAMETERS)
+        of = lambda tensors: pointers(*(tensors(name).data_ptr() for name in PARAMETERS))  # noqa: E731
+        adamw = (of(arrays.__getitem__), of(grads.__getitem__), of(lambda name: moments[name][0]), of(lambda name: moments[name][1]),
+                 (ctypes.c_uint32 * len(PARAMETERS))(*(arrays[name].numel() for name in PARAMETERS)))
+        return _LayerState(grads=grads, moments=moments, supports=supports,
                            values={"in_val": torch.empty_like(arrays["up_val"]), "hid_val": torch.empty_like(arrays["out_val"])},
-                           columns=(c1, c2, c3, c3 + self.d_ff))
+                           columns=(c1, c2, c3, c3 + self.d_ff), adamw=adamw)
 
     # -- buffers ---------------------------------------------------------------------------------------------------
     def reserve(self, n: int) -> None:
@@ -159,23 +169,29 @@ class HFFNTrainRuntime:
     def _mfma_possible(self, n: int) -> bool:
         return self.runtime.mfma_available and mfma_streamed(n, self.d_model, self.d_ff)
 
+    def _planes_possible(self, n: int) -> bool:
+        """Whether the forward with z may run on planes densified for the call at N."""
+        return self._planes_shapes and self.runtime._transient_allowed and not self.runtime.mfma_available
+
+    def _planes_preferred(self, n: int) -> bool:
+        """Whether the forward with z is estimated faster on planes densified for the call than on the lane-per-token
+        gathers (the backward's gz and gx are the same products)."""
+        gather = max(ROWS_SHARE * rows_us(n, self.runtime._store), ROWS_WALK_US + ROWS_WALK_SLOT_US * self.runtime._longest)
+        return self._planes_possible(n) and prefill_us(n, self.d_model, self.d_ff, False) < gather
+
     def _grow_mfma(self, n: int) -> None:
-        """The MFMA workspace at N and every layer's transposed planes, when the planes products may run at N."""
-        if not self._mfma_possible(n):
+        """The workspaces of the MFMA products at N, when they may run at N."""
+        if self.train_mode(n) != "mfma":
             return
-        need = _lib.query_bytes(self._lib.hffn_train_mfma_workspace, n, self.d_model, self.d_ff)
-        if self._mfma_work is None or need > self._mfma_work.numel():
-            self._mfma_work = torch.zeros(need, dtype=torch.uint8, device=self.runtime.device)
-            self.growths += 1
-        for state in self._layers:
-            if state.planes_t is None:
-                device, planes = self.runtime.device, {}
-                for side, rows, k in (("down_t", self.d_ff, self.d_model), ("up_t", self.d_model, self.d_ff)):
-                    size = _lib.query_bytes(self._lib.hffn_dense_planes_bytes, rows, k)
-                    planes[side] = torch.empty(size // 2, dtype=torch.float16, device=device)
-                    planes[f"{side}_binades"] = torch.empty(rows, dtype=torch.int32, device=device)
-                state.planes_t = planes
+        if self._mfma_possible(n):
+            need = _lib.query_bytes(self._lib.hffn_train_mfma_workspace, n, self.d_model, self.d_ff)
+            if self._mfma_work is None or need > self._mfma_work.numel():
+                self._mfma_work = torch.zeros(need, dtype=torch.uint8, device=self.runtime.device)
                 self.growths += 1
+        need = _lib.query_bytes(self._lib.hffn_train_planes_workspace, n, self.d_model, self.d_ff)
+        if self._planes_work is None or need > self._planes_work.numel():
+            self._planes_work = torch.empty(need, dtype=torch.uint8, device=self.runtime.device)
+            self.growths += 1
 
     def _grow_partials(self, n: int) -> None:
         tiles = grad_tiles(n)
@@ -216,23 +232,30 @@ class HFFNTrainRuntime:
             if self.forced_grad == "dense" and not self._dense_bytes_at(n):
                 raise ValueError(f"the dense sampled products do not run at N={n} on {self.d_model} x {self.d_ff}")
             return self.forced_grad
-        dense = n >= GRAD_DENSE_MIN_TOKENS and self.runtime.density >= GRAD_DENSE_MIN_DENSITY and self._dense_bytes_at(n) > 0
-        return "dense" if dense else "gather"
+        mode = self._modes.get(("grad", n))
+        if mode is None:
+            dense = n >= GRAD_DENSE_MIN_TOKENS and self.runtime.density >= GRAD_DENSE_MIN_DENSITY and self._dense_bytes_at(n) > 0
+            mode = self._modes["grad", n] = "dense" if dense else "gather"
+        return mode
 
     def train_mode(self, n: int) -> str:
         """``mfma`` (the forward with z, gz and gx as split-fp16 MFMA products over densified planes) from
-        ``TRAIN_MFMA_MIN_TOKENS`` tokens when the runtime holds planes, runs its policy (no forced pair) and the streamed
-        GEMM takes N, else ``gather``; ``forced_train`` overrides the choice."""
-        possible = self._mfma_possible(n)
+        ``TRAIN_MFMA_MIN_TOKENS`` tokens when the runtime runs its policy (no forced pair) and either holds planes and the
+        streamed GEMM takes N, or holds none and planes densified for the call are estimated faster; else ``gather``.
+        ``forced_train`` overrides the choice."""
         if self.forced_train is not None:
             if self.forced_train not in TRAIN_MODES:
                 raise ValueError(f"training mode is one of {TRAIN_MODES}, not {self.forced_train!r}")
-            if self.forced_train == "mfma" and not possible:
+            if self.forced_train == "mfma" and not (self._mfma_possible(n) or self._planes_possible(n)):
                 raise ValueError(f"the planes products do not run at N={n} on {self.d_model} x {self.d_ff} (no planes, or "
                                  "a shape the streamed GEMM refuses)")
             return self.forced_train
-        policy = self.runtime.forced_up is None and self.runtime.forced_down is None
-        return "mfma" if possible and policy and n >= TRAIN_MFMA_MIN_TOKENS else "gather"
+        if n < TRAIN_MFMA_MIN_TOKENS or self.runtime.forced_up is not None or self.runtime.forced_down is not None:
+            return "gather"
+        mode = self._modes.get(("train", n))
+        if mode is None:
+            mode = self._modes["train", n] = "mfma" if self._mfma_possible(n) or self._planes_preferred(n) else "gather"
+        return mode
 
     def _runtime_planes(self, index: int) -> dict:
         """The runtime's planes of layer ``index``, rebuilt first if an update made them stale."""
@@ -276,7 +299,14 @@ class HFFNTrainRuntime:
             raise ValueError(f"z must be a contiguous float32 device tensor of at least {self.d_ff * ld} entries")
         self.reserve(n)
         x_t, act, y_t, y = runtime._work
-        if self.train_mode(n) == "mfma":
+        if self.train_mode(n) == "mfma" and not runtime.mfma_available:
+            x = _aligned(x)
+            _, *model = runtime._args[index]
+            _lib.check(self._lib.hffn_forward_planes_z(x.data_ptr(), *model, self._planes_work.data_ptr(), self._planes_work.numel(), x_t,
+                                                       act, z.data_ptr(), y, self.d_model, self.d_ff, n, ld, _stream(runtime.device)),
+                       "forward with z (planes of the call)")
+            self.calls["mfma", "mfma"] += 1
+        elif self.train_mode(n) == "mfma":
             planes, tensors, x = self._runtime_planes(index), runtime._tensors[index], _aligned(x)
             _lib.check(self._lib.hffn_forward_mfma_z(x.data_ptr(), planes["up"].data_ptr(), planes["up_binades"].data_ptr(),
                                                      tensors["b_up"].data_ptr(), planes["down"].data_ptr(),
@@ -310,25 +340,20 @@ class HFFNTrainRuntime:
         arrays, state = runtime._tensors[index], self._layers[index]
         supports, values, grads = state.supports, state.values, state.grads
         x_t, act, _, _ = runtime._work
-        _lib.check(lib.hffn_transpose(gy.data_ptr(), self._gy_t.data_ptr(), n, d, d, ld, stream), "gy feature-major")
-        for source, position, target in (("out_val", "hid_pos", "hid_val"), ("up_val", "in_pos", "in_val")):
-            _lib.check(lib.hffn_gather_values(arrays[source].data_ptr(), supports[position].data_ptr(), values[target].data_ptr(),
-                                              values[target].numel(), stream), f"{target} refresh")
         planes_mode = self.train_mode(n) == "mfma"
-        if planes_mode:  # gz and gx on the planes of W_down^T and W_up^T, densified from the values just gathered
-            planes_t = state.planes_t
-            for side, rows, k, (offsets, owner, vals) in (("down_t", h, d, ("hid_offsets", "hid_output", "hid_val")),
-                                                          ("up_t", d, h, ("in_offsets", "in_hidden", "in_val"))):
-                source = values[vals]
-                _lib.check(lib.hffn_densify(_lib.VALUE_F32, supports[offsets].data_ptr(), supports[owner].data_ptr(),
-                                            source.data_ptr(), rows, k, planes_t[side].data_ptr(),
-                                            planes_t[f"{side}_binades"].data_ptr(), stream), f"densify {side}")
-            gy_in = _aligned(gy)
-            _lib.check(lib.hffn_backward_mfma(gy_in.data_ptr(), z_ptr, planes_t["down_t"].data_ptr(),
-                                              planes_t["down_t_binades"].data_ptr(), planes_t["up_t"].data_ptr(),
-                                              planes_t["up_t_binades"].data_ptr(), self._mfma_work.data_ptr(),
-                                              self._mfma_work.numel(), self._gz.data_ptr(), self._gx.data_ptr(), d, h, n, ld, stream),
-                       "gz, gx (mfma)")
+        if planes_mode:  # gz and gx on the planes of W_down^T and W_up^T, densified from the values by position; gy_t with them
+            gy_in, at = _aligned(gy), lambda name: supports[name].data_ptr()  # noqa: E731
+            _lib.check(lib.hffn_backward_planes(gy_in.data_ptr(), z_ptr, at("hid_offsets"), at("hid_output"), at("hid_pos"),
+                                                arrays["out_val"].data_ptr(), at("in_offsets"), at("in_hidden"), at("in_pos"),
+                                                arrays["up_val"].data_ptr(), values["hid_val"].data_ptr(), values["in_val"].data_ptr(),
+                                                self._planes_work.data_ptr(), self._planes_work.numel(), self._gy_t.data_ptr(),
+                                                self._gz.data_ptr(), self._gx.data_ptr(), d, h, *runtime._nnz[index], n, ld, stream),
+                       "gz, gx (planes of the call)")
+        else:
+            _lib.check(lib.hffn_backward_prepare(gy.data_ptr(), self._gy_t.data_ptr(), arrays["out_val"].data_ptr(),
+                                                 supports["hid_pos"].data_ptr(), values["hid_val"].data_ptr(), arrays["up_val"].data_ptr(),
+                                                 supports["in_pos"].data_ptr(), values["in_val"].data_ptr(), d, *runtime._nnz[index], n, ld,
+                                                 stream), "gy feature-major, values in the transposed orders")
         dense = self.grad_mode(n) == "dense"
         if dense:
             self._grow_dense(n)
@@ -375,12 +400,9 @@ class HFFNTrainRuntime:
         beta1, beta2 = self.betas
         scalars = (self.lr * self.weight_decay, beta1, 1.0 - beta1, beta2, 1.0 - beta2, self.lr / (1.0 - beta1 ** k),
                    math.sqrt(1.0 - beta2 ** k), self.eps)
-        arrays, state = self.runtime._tensors[index], self._layers[index]
-        stream = _stream(self.runtime.device)
-        for name in PARAMETERS:
-            first, second = state.moments[name]
-            _lib.check(self._lib.hffn_adamw(arrays[name].data_ptr(), state.grads[name].data_ptr(), first.data_ptr(),
-                                            second.data_ptr(), arrays[name].numel(), *scalars, stream), f"AdamW of {name}")
+        values, grads, first, second, counts = self._layers[index].adamw
+        _lib.check(self._lib.hffn_adamw_arrays(len(PARAMETERS), values, grads, first, second, counts, *scalars, _stream(self.runtime.device)),
+                   "AdamW")
         self.runtime.invalidate_planes(index)
 
     def step(self, index: int, x: torch.Tensor, gy: torch.Tensor) -> torch.Tensor:
@@ -424,6 +446,7 @@ class HFFNTrainRuntime:
                 + size(state.supports.values()) + size(state.values.values()),
                 "workspace": self.runtime.workspace_bytes() + size((self._z, self._gz, self._gy_t, self._gx_t, self._gx))
                 + (self._dense_work.numel() if self._dense_work is not None else 0)
-                + (self._mfma_work.numel() if self._mfma_work is not None else 0),
-                "planes_t": size(state.planes_t.values()) if state.planes_t is not None else 0,
+                + (self._mfma_work.numel() if self._mfma_work is not None else 0)
+                + (self._planes_work.numel() if self._planes_work is not None else 0),
+                "planes_t": 0,  # the transposed planes live in the workspace, one layer's at a time
                 "partials": size((self._partials,)) if self._partials is not None else 0}

@@ -329,6 +329,28 @@ int hffn_backward_mfma(const float* gy, const float* z, const void* down_t_plane
                        const int32_t* up_t_binades, void* workspace, uint64_t workspace_bytes, float* gz, float* gx, uint32_t d_model,
                        uint32_t d_ff, uint32_t n, uint32_t ld, void* stream);
 
+/* The same products on planes densified for the call (widths multiples of 256, any n, no resident planes; float32 sums
+ * in chains of at most 128 k): hffn_forward_planes_z from the compact rows; hffn_backward_planes, which also writes gy_t
+ * (gy transposed, [d_model, ld]), from the transposed supports, whose slot s holds out_val[hid_pos[s]] or
+ * up_val[in_pos[s]] (hid_val and in_val: buffers of nnz_down and nnz_up floats for them). The workspace (hffn_train_planes_workspace bytes, any content) is 256-byte aligned, float buffers
+ * 16-byte aligned. */
+int hffn_train_planes_workspace(uint32_t n, uint32_t d_model, uint32_t d_ff, uint64_t* bytes);
+int hffn_forward_planes_z(const float* x, const int32_t* up_offsets, const int16_t* up_idx, const float* up_val, const float* b_up,
+                          const int32_t* out_offsets, const int16_t* out_hidden, const float* out_val, const float* b_down,
+                          void* workspace, uint64_t workspace_bytes, float* x_t, float* act, float* z, float* y, uint32_t d_model,
+                          uint32_t d_ff, uint32_t n, uint32_t ld, void* stream);
+int hffn_backward_planes(const float* gy, const float* z, const int32_t* hid_offsets, const int16_t* hid_output, const int32_t* hid_pos,
+                         const float* out_val, const int32_t* in_offsets, const int16_t* in_hidden, const int32_t* in_pos,
+                         const float* up_val, float* hid_val, float* in_val, void* workspace, uint64_t workspace_bytes, float* gy_t,
+                         float* gz, float* gx, uint32_t d_model, uint32_t d_ff, uint32_t nnz_up, uint32_t nnz_down, uint32_t n,
+                         uint32_t ld, void* stream);
+
+/* What the gather backward needs first, in one launch: gy_t [d_model, ld] = gy transposed, hid_val[i] = out_val[hid_pos[i]]
+ * and in_val[i] = up_val[in_pos[i]] (the values in the transposed orders). */
+int hffn_backward_prepare(const float* gy, float* gy_t, const float* out_val, const int32_t* hid_pos, float* hid_val, const float* up_val,
+                          const int32_t* in_pos, float* in_val, uint32_t d_model, uint32_t nnz_up, uint32_t nnz_down, uint32_t n,
+                          uint32_t ld, void* stream);
+
 /* Sampled product over an owner-row support: for each owner o < rows, token tile k and slot q of o,
  * g[k*stride + q] = sum_t row[o, t] mat[index[q], t] and gb[k*stride + o] = sum_t row[o, t] (t over tile k, below n);
  * row, mat 16-byte aligned [*, ld]; stride is ignored for n <= 256 (the results are the gradients). With
@@ -359,6 +381,10 @@ int hffn_reduce_tiles(const float* ws, uint32_t stride, uint32_t tiles, uint32_t
  * p -= step_size m / (sqrt(v) / bias2_sqrt + eps). Replaces adamw (kernels_train.py:233-247). */
 int hffn_adamw(float* p, const float* g, float* m, float* v, uint32_t count, float lr_decay, float beta1, float one_minus_beta1,
                float beta2, float one_minus_beta2, float step_size, float bias2_sqrt, float eps, void* stream);
+/* The same on 1-4 arrays in one launch (host arrays of device pointers and counts, read during the call). */
+int hffn_adamw_arrays(uint32_t arrays, float* const* p, const float* const* g, float* const* m, float* const* v, const uint32_t* counts,
+                      float lr_decay, float beta1, float one_minus_beta1, float beta2, float one_minus_beta2, float step_size,
+                      float bias2_sqrt, float eps, void* stream);
 
 /* dst[j] = src[pos[j]]: the values of a transposed support refreshed from the compact array they index (the
  * reference reads them through the positions inside its kernels, kernels_train.py:142-150, 204-215). */
