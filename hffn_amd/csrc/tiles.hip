@@ -136,12 +136,14 @@ __global__ __launch_bounds__(kThreads) void tiles_kernel(const float* __restrict
     constexpr uint32_t kWaveSums = TR * TT * kTokenTile * kRows;
     constexpr uint32_t kTileBytes = P * kPlane * 2, kSumBytes = kWaves / 2 * kWaveSums * 4;
     static_assert(kTileBytes <= kTileBudget, "block shape beyond the LDS budget");
-    __shared__ __align__(16) unsigned char lds[kTileBytes > kSumBytes ? kTileBytes : kSumBytes];
+    constexpr uint32_t kSpare = kTileBytes / 2;  // a cell nothing reads, behind the tile
+    __shared__ __align__(16) unsigned char lds[kTileBytes + 16 > kSumBytes ? kTileBytes + 16 : kSumBytes];
     uint16_t* tile = reinterpret_cast<uint16_t*>(lds);  // [plane][row][W], swizzled runs
     float* sums = reinterpret_cast<float*>(lds);        // [wave % 8][tr][tt][token][row], after the products
 
     const uint32_t lane = threadIdx.x % kWave, wave = uniform(threadIdx.x / kWave);
     const uint32_t r = lane % 16, c = lane / 16;
+    const uint32_t token0 = blockIdx.z * TT * kTokenTile;  // the block's first token
     const uint32_t chunk = blockIdx.y, tile0 = blockIdx.x * TR, tiles = (rows + kRows - 1) / kRows;
     const uint32_t kb = chunk * W, width = min(W, K - kb), kbase = kb % kSuper;
     const uint32_t j0 = chunk * S, j1 = min(j0 + S, subchunks);
@@ -192,7 +194,7 @@ __global__ __launch_bounds__(kThreads) void tiles_kernel(const float* __restrict
         live = 0;
 #pragma unroll
         for (int q = 0; q < S; ++q) {
-            const uint32_t kk = (wave * S + q) * kStep + c * 8, t = tt * kTokenTile + r;
+            const uint32_t kk = (wave * S + q) * kStep + c * 8, t = token0 + tt * kTokenTile + r;
             const bool inside = t < n && kk < width;
             live |= static_cast<uint32_t>(inside) << q;
             load_vec<8>(in + (inside ? static_cast<size_t>(t) * K + kb + kk : 0), xv[q]);
@@ -267,17 +269,17 @@ __global__ __launch_bounds__(kThreads) void tiles_kernel(const float* __restrict
             const uint32_t rr = tr * kRows + wave;
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
-                const int32_t slot = 8 * q + u;
-                if (slot >= s0[tr] && slot < s1[tr]) {
-                    const uint32_t at = tile_at<W>(rr, field(part[0], u) - kb);
-                    if constexpr (P == 1) {
-                        tile[at] = static_cast<uint16_t>(field(part[1], u));
-                    } else {
-                        const float sv = ldexpf(piece_value(part, u), -row_e[tr]);
-                        const _Float16 hi = static_cast<_Float16>(sv);
-                        tile[at] = __builtin_bit_cast(uint16_t, hi);
-                        tile[kPlane + at] = __builtin_bit_cast(uint16_t, static_cast<_Float16>(sv - static_cast<float>(hi)));
-                    }
+                const bool inside = static_cast<uint32_t>(8 * q + u - s0[tr]) < static_cast<uint32_t>(s1[tr] - s0[tr]);
+                const uint32_t at = tile_at<W>(rr, field(part[0], u) - kb);
+                if constexpr (P == 1) {
+                    // a slot of a neighbouring row or chunk goes to the spare cell: no branch per slot (the 1.4B layer's call
+                    // at 16 tokens 20.15 -> 19.35 us; with the split below instead of a copy the branch is the faster form)
+                    tile[inside ? at : kSpare] = static_cast<uint16_t>(field(part[1], u));
+                } else if (inside) {
+                    const float sv = ldexpf(piece_value(part, u), -row_e[tr]);
+                    const _Float16 hi = static_cast<_Float16>(sv);
+                    tile[at] = __builtin_bit_cast(uint16_t, hi);
+                    tile[kPlane + at] = __builtin_bit_cast(uint16_t, static_cast<_Float16>(sv - static_cast<float>(hi)));
                 }
             }
         };
@@ -338,9 +340,7 @@ __global__ __launch_bounds__(kThreads) void tiles_kernel(const float* __restrict
     floatx4 acc[TT][TR];
     // the A operands of step q of the current tile: fp16 hi/lo, or the three bfloat16 parts of each input
     auto split = [&](int q, int ex, uint32_t (&aq)[3][4]) {
-        float v[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = (live >> q) & 1u ? xv[q][i] : 0.0f;
+        const float (&v)[8] = xv[q];  // dead ones zeroed (settle)
         if constexpr (P == 2) {
             half8 xh, xl;
 #pragma unroll
@@ -356,20 +356,16 @@ __global__ __launch_bounds__(kThreads) void tiles_kernel(const float* __restrict
         } else {
 #pragma unroll
             for (int i = 0; i < 8; i += 2) {
-                uint32_t part[3][2];
+                uint32_t part[3][2];  // the upper half of each word is the bfloat16
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
-                    const float x0 = v[i + h];
-                    const uint32_t b1 = __float_as_uint(x0) & 0xffff0000u;
-                    const float rest = x0 - __uint_as_float(b1);
-                    const uint32_t b2 = __float_as_uint(rest) & 0xffff0000u;
-                    const uint32_t b3 = __float_as_uint(rest - __uint_as_float(b2));  // <= 8 significant bits left
-                    part[0][h] = b1 >> 16;
-                    part[1][h] = b2 >> 16;
-                    part[2][h] = b3 >> 16;
+                    part[0][h] = __float_as_uint(v[i + h]);
+                    const float rest = v[i + h] - __uint_as_float(part[0][h] & 0xffff0000u);
+                    part[1][h] = __float_as_uint(rest);
+                    part[2][h] = __float_as_uint(rest - __uint_as_float(part[1][h] & 0xffff0000u));  // <= 8 significant bits left
                 }
 #pragma unroll
-                for (int j = 0; j < 3; ++j) aq[j][i / 2] = part[j][0] | (part[j][1] << 16);
+                for (int j = 0; j < 3; ++j) aq[j][i / 2] = __builtin_amdgcn_perm(part[j][1], part[j][0], 0x07060302u);
             }
         }
     };
@@ -397,13 +393,21 @@ __global__ __launch_bounds__(kThreads) void tiles_kernel(const float* __restrict
     for (int tt = 0; tt < TT; ++tt) {
 #pragma unroll
         for (int tr = 0; tr < TR; ++tr) acc[tt][tr] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-        int ex = 0;  // float32: the token's power of two over the wave's k (lanes r, r + 16, r + 32, r + 48 hold it)
-        if constexpr (P == 2) {
-            uint32_t m = 0;
+        // settle: zero the inputs outside the call (a wave whose inputs are all inside, the usual one, skips it)
+        if (__builtin_amdgcn_ballot_w64(live != (1u << S) - 1) != 0) {
 #pragma unroll
             for (int q = 0; q < S; ++q)
 #pragma unroll
-                for (int i = 0; i < 8; ++i) m = max(m, ((live >> q) & 1u ? __float_as_uint(xv[q][i]) : 0u) & 0x7fffffffu);
+                for (int i = 0; i < 8; ++i) xv[q][i] = (live >> q) & 1u ? xv[q][i] : 0.0f;
+        }
+        int ex = 0;  // float32: the token's power of two over the wave's k (lanes r, r + 16, r + 32, r + 48 hold it)
+        if constexpr (P == 2) {
+            float most = 0.0f;  // (a NaN is passed over here; it reaches the token's outputs through its products)
+#pragma unroll
+            for (int q = 0; q < S; ++q)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) most = fmaxf(most, fabsf(xv[q][i]));
+            uint32_t m = __float_as_uint(most);
             m = max(m, static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), 16, kWave)));
             m = max(m, static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), 32, kWave)));
             ex = binade_of(m);
@@ -436,42 +440,41 @@ __global__ __launch_bounds__(kThreads) void tiles_kernel(const float* __restrict
     }
     __syncthreads();  // the tile is read: its LDS now holds the waves' sums
 
-    // 4. the 16 waves' sums in a fixed order (wave w + 8 into wave w, then waves 0..7), the row's power of two, then the
-    // output or this chunk's partial
-    float* mine = sums + (wave % (kWaves / 2)) * kWaveSums;
+    // 4. the 16 waves' sums in a fixed order (wave w + 8 onto wave w, then waves 0..7), the row's power of two, then the
+    // output or this chunk's partial. Where LDS holds all 16 waves' sums they meet at one barrier; else waves 8..15 go
+    // first (the same order).
+    constexpr bool kAll = 2 * kSumBytes <= sizeof(lds);
     auto cell = [](int tr, int tt, uint32_t token, uint32_t row) { return ((tr * TT + tt) * kTokenTile + token) * kRows + row; };
-    if (wave >= kWaves / 2) {
+    auto each = [&](auto&& f) {
 #pragma unroll
         for (int tr = 0; tr < TR; ++tr)
 #pragma unroll
             for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) mine[cell(tr, tt, 4 * c + i, r)] = acc[tt][tr][i];
-    }
-    __syncthreads();
-    if (wave < kWaves / 2) {
-#pragma unroll
-        for (int tr = 0; tr < TR; ++tr)
-#pragma unroll
-            for (int tt = 0; tt < TT; ++tt)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    float* at = mine + cell(tr, tt, 4 * c + i, r);
-                    *at = acc[tt][tr][i] + *at;
-                }
+                for (int i = 0; i < 4; ++i) f(cell(tr, tt, 4 * c + i, r), acc[tt][tr][i]);
+    };
+    if constexpr (kAll) {
+        float* mine = sums + wave * kWaveSums;
+        each([&](uint32_t at, float v) { mine[at] = v; });
+    } else {
+        float* mine = sums + (wave % (kWaves / 2)) * kWaveSums;
+        if (wave >= kWaves / 2) each([&](uint32_t at, float v) { mine[at] = v; });
+        __syncthreads();
+        if (wave < kWaves / 2) each([&](uint32_t at, float v) { mine[at] = v + mine[at]; });
     }
     __syncthreads();
 #pragma unroll
     for (uint32_t i = 0; i < kOuts; ++i) {
         const uint32_t o = threadIdx.x + i * kThreads;
         if (o >= kOutputs) break;
-        const uint32_t t = o / kTileRows, rr = o % kTileRows, row = tile0 * kRows + rr;
+        const uint32_t local = o / kTileRows, t = token0 + local, rr = o % kTileRows, row = tile0 * kRows + rr;
         if (t >= n) break;
         if (row >= rows) continue;
-        const uint32_t at = cell(rr / kRows, t / kTokenTile, t % kTokenTile, rr % kRows);
-        float s = sums[at];
+        const uint32_t at = cell(rr / kRows, local / kTokenTile, local % kTokenTile, rr % kRows);
+        const auto pair = [&](uint32_t h) { return kAll ? sums[h * kWaveSums + at] + sums[(h + kWaves / 2) * kWaveSums + at] : sums[h * kWaveSums + at]; };
+        float s = pair(0);
 #pragma unroll
-        for (uint32_t h = 1; h < kWaves / 2; ++h) s += sums[h * kWaveSums + at];
+        for (uint32_t h = 1; h < kWaves / 2; ++h) s += pair(h);
         if constexpr (P == 2) s = ldexpf(s, out_e[i]);
         if (gridDim.y > 1) {
             partials[(static_cast<size_t>(chunk) * n + t) * rows + row] = s;
@@ -649,7 +652,8 @@ bool launch_shape(const Side& a, const TilesShape& shape, hipStream_t stream) {
         return false;
     } else {
         if (shape.s != S || shape.tr != TR) return false;
-        hipLaunchKernelGGL((tiles_kernel<V, TT, S, TR, COMPACT>), dim3(shape.blocks, shape.chunks), dim3(kThreads), 0, stream, a.in, a.store,
+        hipLaunchKernelGGL((tiles_kernel<V, TT, S, TR, COMPACT>), dim3(shape.blocks, shape.chunks, (a.n + TT * kTokenTile - 1) / (TT * kTokenTile)),
+                           dim3(kThreads), 0, stream, a.in, a.store,
                            a.table, a.binades, a.bias, a.out, a.partials, a.rows, a.K, a.n, a.subchunks, a.up, a.cidx,
                            static_cast<const V*>(a.cval), static_cast<int32_t>(a.nnz));
         return true;
@@ -666,9 +670,15 @@ bool launch_tokens(const Side& a, const TilesShape& shape, hipStream_t stream) {
 template <typename V, bool COMPACT = false>
 hipError_t tiles_side(const Side& a, hipStream_t stream) {
     const TilesShape shape = tiles_shape(Planes<V>::count == 1 ? kBF16 : kF32, a.rows, a.K, a.nnz);
-    const bool launched = a.n <= kTokenTile       ? launch_tokens<V, 1, COMPACT>(a, shape, stream)
-                          : a.n <= 2 * kTokenTile ? launch_tokens<V, 2, COMPACT>(a, shape, stream)
-                                                  : launch_tokens<V, 4, COMPACT>(a, shape, stream);
+    // A side of few blocks takes its token tiles on several blocks each (the same sums per token): every block densifies
+    // its rows again, but a block's time grows by 1.6 us per token tile (the inputs' split) while the other CUs idle. 512 x
+    // 2048 at 10 %, 37 tokens (128 up, 32 down blocks): 23.3 -> 16.4 us a call.
+    const uint32_t tiles = (a.n + kTokenTile - 1) / kTokenTile, grid = shape.blocks * shape.chunks;
+    const uint32_t groups = std::max(1u, std::min(tiles, kCUs / grid)), each = (tiles + groups - 1) / groups;
+    const bool launched = each == 1   ? launch_tokens<V, 1, COMPACT>(a, shape, stream)
+                          : each == 2 ? launch_tokens<V, 2, COMPACT>(a, shape, stream)
+                          : each == 3 ? launch_tokens<V, 3, COMPACT>(a, shape, stream)
+                                      : launch_tokens<V, 4, COMPACT>(a, shape, stream);
     if (!launched) return hipErrorInvalidValue;
     if (hipError_t status = hipGetLastError(); status != hipSuccess || shape.chunks == 1) return status;
     hipLaunchKernelGGL(tiles_reduce_kernel, dim3((a.n * a.rows + 255) / 256), dim3(256), 0, stream, a.partials, shape.chunks, a.bias, a.out,
