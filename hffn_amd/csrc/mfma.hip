@@ -1561,7 +1561,7 @@ uint32_t dma_up_splits(uint32_t m, uint32_t ncol, uint32_t k) {
 // Sampled products of the training backward from a dense product: G[rows, cols] = A[rows, n] B[cols, n]^T by the
 // streamed GEMM (Epi::UpSplit partials [splits, rows, cols], powers of two undone), then one wave per owner row o:
 // g[q] = sum over the splits (in split order) of G[o, idx[q]] for the row's slots q, and gb[o] = sum_t A[o, t]
-// (lanes over the tokens, then the fixed xor butterfly).
+// (lanes over the tokens, then wave_sum).
 __global__ __launch_bounds__(kThreads) void gather_dense_kernel(const float* __restrict__ partials, uint32_t splits,
                                                                const float* __restrict__ a, uint32_t ld, uint32_t n,
                                                                const int32_t* __restrict__ off, const int16_t* __restrict__ idx,

@@ -22,7 +22,7 @@ uint32_t ceil_div(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
 // over the hidden-major up slots with row = gz and mat = x_t; kernels_train.py:115-137 and 162-184). One wave per
 // owner o and token tile k; lane l holds row[o, t] for its 4 consecutive tokens t = 256 k + 4 l + j. Per slot q the
 // lane forms sum_j row[o, t] * mat[idx[q], t] (ascending j, tokens past n skipped) and the wave adds the lanes with
-// the fixed xor butterfly. The slots are taken 4 at a time, so that 4 row reads are in flight per wave.
+// wave_sum. The slots are taken 4 at a time, so that 4 row reads are in flight per wave.
 __global__ __launch_bounds__(kBlock) void grad_sddmm_kernel(const float* __restrict__ row, const float* __restrict__ mat,
                                                            const int32_t* __restrict__ off, const int16_t* __restrict__ idx,
                                                            float* __restrict__ g, float* __restrict__ gb, uint32_t rows,

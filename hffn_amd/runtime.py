@@ -613,7 +613,7 @@ class HFFNRuntime:
         value_type, *model = self._args[index]
         x_t, act, y_t, y = self._work
         stream = torch.cuda.current_stream(self.device).cuda_stream
-        if self.transient(n):
+        if n > TILES_MAX_TOKENS and self.transient(n):
             x = _aligned(x)  # read 16 bytes at a time
             _lib.check(self._lib.hffn_forward_prefill(value_type, x.data_ptr(), *model, self._prefill_work.data_ptr(),
                                                       4 * self._prefill_work.numel(), y, self.d_model, self.d_ff, n, stream),
