@@ -44,7 +44,6 @@ SIGNATURES = {
     "hffn_adamw": [_P] * 4 + [_U32] + [ctypes.c_float] * 8 + [_P],
     "hffn_adamw_arrays": [_U32] + [_P] * 5 + [ctypes.c_float] * 8 + [_P],
     "hffn_train_planes_workspace": [_U32, _U32, _U32, ctypes.POINTER(_U64)],
-    "hffn_forward_planes_z": [_P] * 10 + [_U64] + [_P] * 4 + [_U32] * 4 + [_P],
     "hffn_backward_planes": [_P] * 13 + [_U64] + [_P] * 3 + [_U32] * 6 + [_P],
     "hffn_backward_prepare": [_P] * 8 + [_U32] * 5 + [_P],
     "hffn_gather_values": [_P, _P, _P, _U32, _P],

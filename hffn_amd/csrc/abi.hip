@@ -788,6 +788,8 @@ int hffn_backward_mfma(const float* gy, const float* z, const void* down_t_plane
 int hffn_train_planes_workspace(uint32_t n, uint32_t d_model, uint32_t d_ff, uint64_t* bytes) {
     if (!bytes) return fail(HFFN_ERROR_ARGUMENT, "train_planes_workspace: null result");
     if (int status = check_mfma(HFFN_VALUE_F32, d_model, d_ff, n)) return status;
+    if (!hffn::mfma_streamed(n, d_model, d_ff))
+        return fail(HFFN_ERROR_ARGUMENT, "train_planes: the streamed GEMM does not take n=%u on %u x %u", n, d_model, d_ff);
     *bytes = hffn::train_planes_workspace_bytes(n, d_model, d_ff);
     return HFFN_OK;
 }
@@ -810,17 +812,6 @@ int check_train_planes(const char* what, uint32_t d_model, uint32_t d_ff, uint32
     return HFFN_OK;
 }
 }  // namespace
-
-int hffn_forward_planes_z(const float* x, const int32_t* up_offsets, const int16_t* up_idx, const float* up_val, const float* b_up,
-                          const int32_t* out_offsets, const int16_t* out_hidden, const float* out_val, const float* b_down,
-                          void* workspace, uint64_t workspace_bytes, float* x_t, float* act, float* z, float* y, uint32_t d_model,
-                          uint32_t d_ff, uint32_t n, uint32_t ld, void* stream) {
-    if (int status = check_train_planes("forward_planes_z", d_model, d_ff, n, ld, workspace, workspace_bytes, {x, b_up, b_down, x_t, act, z, y},
-                                        {up_offsets, up_idx, up_val, out_offsets, out_hidden, out_val}))
-        return status;
-    const hffn::PrefillCall call{x, up_offsets, up_idx, up_val, b_up, out_offsets, out_hidden, out_val, b_down, workspace, y, d_model, d_ff, n};
-    return launched(hffn::launch_train_planes_forward(call, x_t, act, z, ld, static_cast<hipStream_t>(stream)), "forward_planes_z");
-}
 
 int hffn_backward_planes(const float* gy, const float* z, const int32_t* hid_offsets, const int16_t* hid_output, const int32_t* hid_pos,
                          const float* out_val, const int32_t* in_offsets, const int16_t* in_hidden, const int32_t* in_pos,

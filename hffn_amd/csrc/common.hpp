@@ -81,23 +81,25 @@ __device__ __forceinline__ float gelu_grad(float z) {
 __device__ __forceinline__ float widen(float v) { return v; }
 __device__ __forceinline__ float widen(uint16_t v) { return __uint_as_float(static_cast<uint32_t>(v) << 16); }
 
-// Sum over the 64 lanes of a wave; every lane receives the same total (a fixed order: lanes 1 and 2 apart, halves of 8
-// and of 16 mirrored, rows of 16, halves of 32 - each step adds a partner that holds the other half's sum - so the result
-// does not depend on scheduling). On the vector unit's lane paths (DPP, the row and half swaps) rather than through LDS
-// (six dependent permutes): the 410M layer (1024 x 4096 at 50 %) at one token 10.88 -> 10.41 us a call.
+// Sum over the 64 lanes of a wave; every lane receives the same total (fixed xor-butterfly order, 32 first, so the
+// result does not depend on scheduling). On the vector unit's lane paths rather than six dependent permutes through LDS:
+// halves and rows swapped (v + v is the two halves' sum in every lane), then, as lanes 8 (4) apart hold equal sums, the
+// partner lane ^ 8 (^ 4) is 8 (4) lanes on within the row, then quad permutes. The 410M layer (1024 x 4096 at 50 %) at
+// one token: 10.88 -> 10.41 us a call.
 template <int CTRL>
 __device__ __forceinline__ float dpp(float v) {
     return __uint_as_float(__builtin_amdgcn_update_dpp(0, static_cast<int>(__float_as_uint(v)), CTRL, 0xf, 0xf, true));
 }
 __device__ __forceinline__ float wave_sum(float v) {
-    v += dpp<0xB1>(v);   // quad_perm 1 0 3 2
-    v += dpp<0x4E>(v);   // quad_perm 2 3 0 1
-    v += dpp<0x141>(v);  // row_half_mirror
-    v += dpp<0x140>(v);  // row_mirror
+    const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(halves[0]) + __uint_as_float(halves[1]);
     const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     v = __uint_as_float(rows[0]) + __uint_as_float(rows[1]);
-    const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return __uint_as_float(halves[0]) + __uint_as_float(halves[1]);
+    v += dpp<0x128>(v);  // row_ror 8
+    v += dpp<0x124>(v);  // row_ror 4
+    v += dpp<0x4E>(v);   // quad_perm 2 3 0 1
+    v += dpp<0xB1>(v);   // quad_perm 1 0 3 2
+    return v;
 }
 
 __device__ __forceinline__ uint32_t uniform(uint32_t v) {

@@ -11,7 +11,7 @@
 // inputs in LDS (by DMA, every transfer issued before any is waited for), so the store streams while the block waits:
 // one memory round trip for the row offsets, then one for the slots and the inputs together.
 // Long rows are split over P waves of the block (each takes a contiguous segment cut on the group grid); the P
-// partial sums are added in segment order. Within a wave the 64 lane partials are added in a fixed order (wave_sum). Inputs are
+// partial sums are added in segment order. Within a wave the 64 lane partials are added by a fixed xor butterfly. Inputs are
 // staged in LDS when they fit (x for up, act for down at small n), otherwise act is gathered from L2.
 // Tokens are processed NT at a time (NT = 1, 2, 4 or 8); every activation and output is written by one lane: no
 // atomics, bitwise repeatable, and a token's result does not depend on the other tokens of the call.

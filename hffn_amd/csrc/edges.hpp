@@ -3,7 +3,7 @@
 // (a 16-byte value load and an 8-byte index load), bfloat16 groups of 8 (a 16-byte value load and a 16-byte index
 // load: half the load instructions of 4-slot groups; 8 float32 values per lane would split a wave's value loads into
 // two 2 KB ranges of half-used lines). The groups of a wave are strided by 64 groups, the lane partials of NT tokens
-// are added in a fixed order (wave_sum), and a long row split in P segments (one wave each) is added in segment order.
+// are added by a fixed xor butterfly, and a long row split in P segments (one wave each) is added in segment order.
 // Every kernel that runs a row through these pieces with the same P produces the same bits (the number of groups a
 // lane holds at once does not change them).
 #pragma once

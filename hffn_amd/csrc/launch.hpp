@@ -147,9 +147,8 @@ hipError_t launch_train_backward(const float* gy, const float* z, const void* do
                                  const void* up_t_planes, const int32_t* up_t_exp, void* workspace, float* gz, float* gx, uint32_t n,
                                  uint32_t d, uint32_t h, uint32_t ld, hipStream_t stream);
 
-// The same on planes densified per call from the compact rows (d and h multiples of 256, any n): the forward of
-// PrefillCall (float32) that also writes x_t, act and z; the backward that also writes gy_t, its sides densified from the
-// transposed supports, their values read in place by position. Workspace: train_planes_workspace_bytes, any content.
+// The training backward's products on planes densified per call (mfma_streamed shapes), which also writes gy_t: the sides
+// from the transposed supports, their values read by position. Workspace: train_planes_workspace_bytes, any content.
 struct TrainBackward {
     const float *gy, *z;
     const int32_t* hid_off;
@@ -166,7 +165,6 @@ struct TrainBackward {
     uint32_t d, h, nnz_up, nnz_down, n, ld;
 };
 uint64_t train_planes_workspace_bytes(uint32_t n, uint32_t d, uint32_t h);
-hipError_t launch_train_planes_forward(const PrefillCall& call, float* x_t, float* act, float* z, uint32_t ld, hipStream_t stream);
 hipError_t launch_train_planes_backward(const TrainBackward& call, hipStream_t stream);
 
 // Decode-sized projections over the same planes (gemv.hip): act token-major [n, h] (16-byte aligned), y token-major

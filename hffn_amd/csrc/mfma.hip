@@ -123,7 +123,7 @@ constexpr uint32_t kSplitWaves = kThreads / kWave;
 // The work of kThreads threads (tid) on row group `group`; part: their maxima in LDS. Every thread of the block calls it.
 __device__ __forceinline__ void split_rows(uint32_t (&part)[kSplitWaves][kSplitBlockRows], uint32_t tid, uint32_t group,
                                            const float* __restrict__ x, uint32_t M, uint32_t rows_pad, uint32_t K, uint32_t ld,
-                                           uint32_t k_real, uint32_t bits, _Float16* __restrict__ planes, int32_t* __restrict__ e) {
+                                           uint32_t k_real, _Float16* __restrict__ planes, int32_t* __restrict__ e) {
     constexpr uint32_t kWaves = kSplitWaves;
     const uint32_t lane = tid % kWave, wave = uniform(tid / kWave);
     const uint32_t r = lane % kSplitBlockRows, piece = lane / kSplitBlockRows;
@@ -182,11 +182,10 @@ __device__ __forceinline__ void split_rows(uint32_t (&part)[kSplitWaves][kSplitB
             if (k0 + 64 * i >= k_end) break;
             half8 h, l;
             const uint32_t k = k0 + 64 * i + 8 * piece;
-            const float by = chain_odd(k, bits) ? -scale : scale;
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
                 _Float16 hh, ll;
-                split(v[i][q] * by, hh, ll);
+                split(v[i][q] * scale, hh, ll);
                 h[q] = hh;
                 l[q] = ll;
             }
@@ -199,29 +198,30 @@ __global__ __launch_bounds__(kThreads) void split_rows_kernel(const float* __res
                                                              uint32_t K, uint32_t ld, uint32_t k_real, _Float16* __restrict__ planes,
                                                              int32_t* __restrict__ e) {
     __shared__ uint32_t part[kSplitWaves][kSplitBlockRows];
-    split_rows(part, threadIdx.x, blockIdx.x, x, M, rows_pad, K, ld, k_real, kNoChains, planes, e);
+    split_rows(part, threadIdx.x, blockIdx.x, x, M, rows_pad, K, ld, k_real, planes, e);
 }
 
 // Two matrices of the same columns in one launch (the operands of a sampled product).
 __global__ __launch_bounds__(kThreads) void split_pair_kernel(const float* __restrict__ a, uint32_t a_rows, _Float16* __restrict__ a_planes,
                                                              int32_t* __restrict__ a_e, const float* __restrict__ b, uint32_t b_rows,
                                                              _Float16* __restrict__ b_planes, int32_t* __restrict__ b_e, uint32_t K,
-                                                             uint32_t ld, uint32_t k_real, uint32_t b_bits) {
+                                                             uint32_t ld, uint32_t k_real) {
     __shared__ uint32_t part[kSplitWaves][kSplitBlockRows];
     const uint32_t a_blocks = a_rows / kSplitBlockRows;
-    if (blockIdx.x < a_blocks) split_rows(part, threadIdx.x, blockIdx.x, a, a_rows, a_rows, K, ld, k_real, kNoChains, a_planes, a_e);
-    else split_rows(part, threadIdx.x, blockIdx.x - a_blocks, b, b_rows, b_rows, K, ld, k_real, b_bits, b_planes, b_e);
+    if (blockIdx.x < a_blocks) split_rows(part, threadIdx.x, blockIdx.x, a, a_rows, a_rows, K, ld, k_real, a_planes, a_e);
+    else split_rows(part, threadIdx.x, blockIdx.x - a_blocks, b, b_rows, b_rows, K, ld, k_real, b_planes, b_e);
 }
 
 // --------------------------------------------------------------------------------------------- densify
 // Row n of the dense matrix (a neuron of W_up, or an output of W_down^T) has its slots [off[n], off[n+1]) at columns
 // idx[] (distinct within a row; the host checks it); densifying writes the whole row of both planes (zeros outside
-// the support) and its binade. A block takes kDensRows consecutive rows and kDensChunk columns: the rows'
-// maxima (two waves per row, over all their slots), then their hi/lo parts in its columns assembled in LDS (zeroed
+// the support) and its binade. A block takes kDensRows consecutive rows and dens_chunk columns: the rows'
+// maxima (a wave per row, over all its slots), then their hi/lo parts in its columns assembled in LDS (zeroed
 // meanwhile, then each slot of the chunk in its column) and written out whole: for every 16-byte chunk run the block's rows are
 // kDensRows consecutive 16-byte pieces, one 128-byte line per (run, row group). The rows are padded by 16 bytes in
-// LDS so that the eight rows of a chunk fall in different banks; the tile (66 KB) leaves room for two blocks per CU.
-constexpr uint32_t kDensRows = 8, kDensChunk = 2048, kDensThreads = 1024, kDensPad = 8;
+// LDS so that the eight rows of a chunk fall in different banks; the tile (33 KB) leaves room for four blocks per CU.
+constexpr uint32_t kDensRows = 8, kDensThreads = 512, kDensPad = 8;
+constexpr uint32_t dens_chunk(uint32_t parts) { return parts == 2 ? 1024 : 2048; }  // columns of a block's tile (33 KB)
 // Slots [8 q, 8 q + 8) of the compact rows: one 16-byte load of their indices, one (float32: two) of their values. vec:
 // idx and val start on 16-byte boundaries.
 template <typename V>
@@ -271,12 +271,12 @@ struct SlotPiece {
     }
 };
 
-// The slots [begin, end) of one row on two waves (half h of them), in pieces of 8 on 8-slot boundaries, 64 pieces at a
-// time in turn (lane l of half h: pieces first + 128 q). The first piece of a lane is requested at construction and held;
-// those of rows of more than 1016 slots are read at each pass.
+// The slots [begin, end) of one row on a wave, in pieces of 8 on 8-slot boundaries, 64 at a time (lane l: pieces first + 64
+// q). The first piece of a lane is requested at construction and held; the further ones of rows of more than 504 slots are
+// read at each pass.
 template <typename V>
 struct RowSlots {
-    static constexpr int32_t kStride = 2 * kWave;
+    static constexpr int32_t kStride = kWave;
     const int16_t* idx;
     const V* val;
     const int32_t* pos;
@@ -284,8 +284,8 @@ struct RowSlots {
     bool vec;
     SlotPiece<V> held;
     __device__ __forceinline__ RowSlots(const int16_t* __restrict__ i, const V* __restrict__ v, const int32_t* __restrict__ positions, int32_t b,
-                                        int32_t e, int32_t slots, bool aligned, uint32_t half, uint32_t lane)
-        : idx(i), val(v), pos(positions), begin(b), end(e), first((b >> 3) + static_cast<int32_t>(half * kWave + lane)), last(e > b ? (e + 7) >> 3 : 0),
+                                        int32_t e, int32_t slots, bool aligned, uint32_t lane)
+        : idx(i), val(v), pos(positions), begin(b), end(e), first((b >> 3) + static_cast<int32_t>(lane)), last(e > b ? (e + 7) >> 3 : 0),
           nnz(slots), vec(aligned) {
         if (first < last) held.load(idx, val, pos, first, nnz, vec);
     }
@@ -307,9 +307,9 @@ struct RowSlots {
             f(p.index(u), p.value(u), static_cast<uint32_t>(8 * q + u - begin) < static_cast<uint32_t>(end - begin));
     }
 };
+template <uint32_t PARTS>
 struct DensTile {
-    _Float16 tile[2][kDensRows][kDensChunk + kDensPad];
-    uint32_t row_max[2][kDensRows];
+    _Float16 tile[PARTS][kDensRows][dens_chunk(PARTS) + kDensPad];
 };
 struct DensSide {
     const int32_t* off;
@@ -323,35 +323,34 @@ struct DensSide {
     int32_t* exps;
 };
 // A side's blocks: (row group, column chunk), chunk-major.
-constexpr uint32_t dens_blocks(uint32_t rows_pad, uint32_t k) { return (rows_pad + kDensRows - 1) / kDensRows * ((k + kDensChunk - 1) / kDensChunk); }
-constexpr uint32_t kDensOccupancy = 8;  // waves per SIMD of two blocks: at most 64 VGPRs
+constexpr uint32_t dens_blocks(uint32_t rows_pad, uint32_t k, uint32_t parts) {
+    return (rows_pad + kDensRows - 1) / kDensRows * ((k + dens_chunk(parts) - 1) / dens_chunk(parts));
+}
+constexpr uint32_t kDensOccupancy = 8;  // waves per SIMD of four blocks: at most 64 VGPRs
 
 // PARTS 1 (bfloat16 planes of one call): the hi plane alone, the only one its GEMMs read. Rows `rows` .. rows_pad - 1 and
 // columns past the indices are zeros.
 template <typename V, uint32_t PARTS>
-__device__ __forceinline__ void densify(DensTile& lds, const DensSide& side, uint32_t block) {
+__device__ __forceinline__ void densify(DensTile<PARTS>& lds, const DensSide& side, uint32_t block) {
     static_assert(kDensRows * 16 == 128, "a row group's pieces of one chunk run fill one 128-byte line");
     auto& tile = lds.tile;
-    auto& row_max = lds.row_max;
-    static_assert(kDensThreads / kWave == 2 * kDensRows, "two waves per row");
-    const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = uniform(tid / kWave);
-    const uint32_t row = wave % kDensRows, half = wave / kDensRows;  // wave-uniform
+    constexpr uint32_t kDensChunk = dens_chunk(PARTS);
+    static_assert(kDensThreads / kWave == kDensRows, "a wave per row");
+    const uint32_t tid = threadIdx.x, lane = tid % kWave, row = uniform(tid / kWave);
     const uint32_t groups = (side.rows_pad + kDensRows - 1) / kDensRows, chunk = block / groups;
     const uint32_t r0 = block % groups * kDensRows, n = r0 + row, c0 = chunk * kDensChunk;
     const uint32_t width = min(kDensChunk, side.k - c0), pieces = width / 8;  // width: a multiple of 32
-    // Waves w and w + kDensRows take row r0 + w. The two halves' maxima meet in LDS.
     const bool real = n < side.rows;
     RowSlots<V> slots(side.idx, static_cast<const V*>(side.val), side.pos, real ? side.off[n] : 0, real ? side.off[n + 1] : 0, side.off[side.rows],
-                      side.vec, half, lane);
+                      side.vec, lane);
     // the tile zeroed while the slots are in flight
     for (uint32_t i = tid; i < PARTS * sizeof(tile[0]) / 16; i += kDensThreads) reinterpret_cast<uint4*>(tile)[i] = make_uint4(0, 0, 0, 0);
     uint32_t m = 0;
     slots.each([&](uint32_t, float v, bool inside) { m = max(m, inside ? abs_bits(v) : 0u); });
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) m = max(m, static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), o, kWave)));
-    if (lane == 0) row_max[half][row] = m;
-    __syncthreads();  // the tile is zeroed, the halves' maxima are in
-    const int e = binade_of_bits(max(row_max[0][row], row_max[1][row]));
+    const int e = binade_of_bits(m);
+    __syncthreads();  // the tile is zeroed
     slots.each([&](uint32_t column, float v, bool inside) {
         // a slot of another row or column block goes to the row's padding, which nothing reads: no branch per slot
         const uint32_t c = column - c0, at = inside && c < width ? c : kDensChunk;
@@ -361,7 +360,7 @@ __device__ __forceinline__ void densify(DensTile& lds, const DensSide& side, uin
         if constexpr (PARTS == 2) tile[1][row][at] = lo;
     });
     __syncthreads();
-    // thread t: row t % 8, pieces t / 8, t / 8 + 128, ... of every part (no division by the width: two per 16 bytes moved
+    // thread t: row t % 8, pieces t / 8, t / 8 + 64, ... of every part (no division by the width: two per 16 bytes moved
     // cost more than the moves)
     const uint32_t rr = tid % kDensRows;
     if (r0 + rr < side.rows_pad)
@@ -370,45 +369,51 @@ __device__ __forceinline__ void densify(DensTile& lds, const DensSide& side, uin
             for (uint32_t part = 0; part < PARTS; ++part)
                 *reinterpret_cast<uint4*>(side.planes + plane_at(side.rows_pad, r0 + rr, c0 + j * 8, part)) =
                     *reinterpret_cast<const uint4*>(&tile[part][rr][j * 8]);
-    if (chunk == 0 && half == 0 && lane == 0 && n < side.rows_pad) side.exps[n] = e;
+    if (chunk == 0 && lane == 0 && n < side.rows_pad) side.exps[n] = e;
 }
 template <typename V>
 __global__ __launch_bounds__(kDensThreads, kDensOccupancy) void densify_kernel(DensSide side) {
-    __shared__ __attribute__((aligned(16))) DensTile lds;
+    __shared__ __attribute__((aligned(16))) DensTile<2> lds;
     densify<V, 2>(lds, side, blockIdx.x);
 }
 
 // What a call that densifies its own planes (launch_prefill) needs before its first GEMM, in one launch: the planes of
-// both sides from the compact rows and the input planes of x. Blocks 0 .. up_blocks - 1 densify W_up, the next
-// down_blocks W_down, the next split_blocks split x, kSplitGroups groups of 8 rows a block (training: the others transpose
-// it). MI355X, at 128 / 2048 tokens: 9.9 / 7.4 us
-// on 512 x 2048 at 20 % (float32), 17.9 / 15.2 on 1024 x 4096 at 10 %, 38 / 46 on 2048 x 8192 at 20 % (bfloat16; 72 with
-// single slots a lane in place of 8, 2-byte loads). A block is a chain of four round trips (offsets, slots, LDS, stores).
+// both sides from the compact rows and the input planes of x. The first split_blocks split x, kSplitGroups groups of 8
+// rows a block, the next trans_blocks transpose it (training), the next up_blocks densify W_up, the others W_down (the
+// split, a block's longest work, first: last it was the launch's tail, 46 us instead of PREPT at 1999 tokens on 2048 x 8192).
+// MI355X: 7.8 us on 512 x 2048 at 20 % (float32, 128 tokens), 17 on 1024 x 4096 at 10 % with uneven rows, 28 on 2048 x
+// 8192 at 20 % (bfloat16, 128 tokens; 72 with single slots a lane in place of 8, 38 in blocks of 1024 threads, two per CU).
+// A block is a chain of four round trips (offsets, slots, LDS, stores): many small blocks cover one another.
 constexpr uint32_t kSplitGroups = kDensThreads / kThreads;
 template <typename V>
 __global__ __launch_bounds__(kDensThreads, kDensOccupancy) void prefill_prep_kernel(DensSide up, DensSide down, uint32_t up_blocks,
-                                                                                   uint32_t down_blocks, uint32_t split_blocks,
+                                                                                   uint32_t split_blocks, uint32_t trans_blocks,
                                                                                    const float* __restrict__ x, uint32_t M,
                                                                                    uint32_t rows_pad, uint32_t K, uint32_t ld,
                                                                                    _Float16* __restrict__ planes, int32_t* __restrict__ e,
                                                                                    float* __restrict__ x_t, uint32_t t_ld, uint32_t tiles_c,
                                                                                    bool vectors) {
     constexpr uint32_t kParts = sizeof(V) == 2 ? 1 : 2;
-    __shared__ __attribute__((aligned(16))) DensTile lds;
-    if (blockIdx.x < up_blocks) return densify<V, kParts>(lds, up, blockIdx.x);
-    if (blockIdx.x < up_blocks + down_blocks) return densify<V, kParts>(lds, down, blockIdx.x - up_blocks);
-    using Parts = uint32_t[kSplitGroups][kSplitWaves][kSplitBlockRows];
-    Parts& parts = reinterpret_cast<Parts&>(lds);
-    const uint32_t g = uniform(threadIdx.x / kThreads), block = blockIdx.x - up_blocks - down_blocks;
+    __shared__ __attribute__((aligned(16))) DensTile<kParts> lds;
+    const uint32_t g = uniform(threadIdx.x / kThreads);
+    uint32_t block = blockIdx.x;
     if (block < split_blocks) {
-        split_rows(parts[g], threadIdx.x % kThreads, block * kSplitGroups + g, x, M, rows_pad, K, ld, ld, kNoChains, planes, e);
+        using Parts = uint32_t[kSplitGroups][kSplitWaves][kSplitBlockRows];
+        split_rows(reinterpret_cast<Parts&>(lds)[g], threadIdx.x % kThreads, block * kSplitGroups + g, x, M, rows_pad, K, ld, ld, planes, e);
         return;
     }
-    // training: x [M, ld] transposed too, a tile per group (a tile past the rows moves nothing)
-    static_assert(kThreads == kTransThreads && sizeof(TransposeTile) * kSplitGroups <= sizeof(DensTile), "a tile per group of threads");
-    const uint32_t tile = (block - split_blocks) * kSplitGroups + g;
-    transpose_tile(reinterpret_cast<TransposeTile*>(&lds)[g], threadIdx.x % kThreads, tile / tiles_c * kTransRows, tile % tiles_c * kTransCols, x,
-                   x_t, M, ld, ld, t_ld, vectors);
+    block -= split_blocks;
+    if (block < trans_blocks) {
+        // training: x [M, ld] transposed too, a tile per group (a tile past the rows moves nothing)
+        static_assert(kThreads == kTransThreads && sizeof(TransposeTile) * kSplitGroups <= sizeof(lds), "a tile per group of threads");
+        const uint32_t tile = block * kSplitGroups + g;
+        transpose_tile(reinterpret_cast<TransposeTile*>(&lds)[g], threadIdx.x % kThreads, tile / tiles_c * kTransRows,
+                       tile % tiles_c * kTransCols, x, x_t, M, ld, ld, t_ld, vectors);
+        return;
+    }
+    block -= trans_blocks;
+    if (block < up_blocks) densify<V, kParts>(lds, up, block);
+    else densify<V, kParts>(lds, down, block - up_blocks);
 }
 
 // ------------------------------------------------------------------------------------------------ GEMM
@@ -791,9 +796,9 @@ __device__ __forceinline__ void wait_stages(uint32_t later) {
 // three times as much as the tiles path it stands in for (2.05e-7); in chains of one activation block it keeps 2.0e-7, for
 // ~4 % of the GEMMs' time.
 //
-// The MFMAs' own sums are biased downwards (mean error -1.3e-8 of an output's deviation, whatever its sign), which a sum
-// over many tokens adds up: the b_up gradient of 2048 tokens lost 6.5e-7 where gathers lose 2.5e-7. So the B planes of
-// these calls hold -w in every odd chain's columns (chain_odd), whose sums are subtracted: the bias cancels.
+// The MFMAs' own sums are biased downwards (mean error -1.3e-8 of a pre-activation's deviation, whatever its sign). So the
+// B planes of these calls hold -w in every odd chain's columns (chain_odd), whose sums are subtracted: the bias cancels
+// (4e-10).
 //
 // BM < 256 (those calls too): row tiles of 128 (waves of 32 x 64) or 64 (32 x 32), where 256 rows by 128 columns leave
 // CUs idle or would have to be split over K, with the partials' round trip and another launch. A k-tile of such a tile
@@ -1561,7 +1566,7 @@ uint32_t dma_up_splits(uint32_t m, uint32_t ncol, uint32_t k) {
 // Sampled products of the training backward from a dense product: G[rows, cols] = A[rows, n] B[cols, n]^T by the
 // streamed GEMM (Epi::UpSplit partials [splits, rows, cols], powers of two undone), then one wave per owner row o:
 // g[q] = sum over the splits (in split order) of G[o, idx[q]] for the row's slots q, and gb[o] = sum_t A[o, t]
-// (lanes over the tokens, then wave_sum).
+// (lanes over the tokens, then the fixed xor butterfly).
 __global__ __launch_bounds__(kThreads) void gather_dense_kernel(const float* __restrict__ partials, uint32_t splits,
                                                                const float* __restrict__ a, uint32_t ld, uint32_t n,
                                                                const int32_t* __restrict__ off, const int16_t* __restrict__ idx,
@@ -1742,7 +1747,7 @@ bool slots_aligned(const void* idx, const void* val) {
 
 hipError_t launch_densify(int vt, const int32_t* off, const int16_t* idx, const void* val, uint32_t rows, uint32_t k,
                           void* planes, int32_t* exps, hipStream_t stream) {
-    const dim3 grid(dens_blocks(rows, k)), block(kDensThreads);
+    const dim3 grid(dens_blocks(rows, k, 2)), block(kDensThreads);
     const DensSide side{off, idx, val, nullptr, rows, rows, k, kNoChains, slots_aligned(idx, val), static_cast<_Float16*>(planes), exps};
     if (vt == kBF16) hipLaunchKernelGGL((densify_kernel<uint16_t>), grid, block, 0, stream, side);
     else hipLaunchKernelGGL((densify_kernel<float>), grid, block, 0, stream, side);
@@ -1875,12 +1880,11 @@ struct PrefillLayout {
     size_t up_planes, up_exp, down_planes, down_exp, x_exp, act_exp, x_planes, act_planes, partials, bytes;
 };
 // Byte offsets (256-byte aligned) for calls of up to n tokens; the partials hold the largest of any smaller call's.
-// training: not in pieces, and the up projection's sums always go through the partials.
-PrefillLayout plan_layout(bool bf16, bool training, uint32_t n, uint32_t d, uint32_t h) {
+PrefillLayout plan_layout(bool bf16, uint32_t n, uint32_t d, uint32_t h) {
     PrefillLayout l{};
     l.d = pad256(d);
     l.h = pad256(h);
-    if (!training) n = min(n, kPrefillPiece);
+    n = min(n, kPrefillPiece);
     const size_t rows = rows_padded(n);
     size_t at = 0;
     const auto take = [&at](size_t bytes) {
@@ -1899,7 +1903,7 @@ PrefillLayout plan_layout(bool bf16, bool training, uint32_t n, uint32_t d, uint
     size_t most = 0;
     for (uint32_t m = 128; m <= max(rows, size_t{128}); m += m == 128 ? 128 : kRowPad) {
         const PrefillPlan plan = prefill_plan(m, l.d, l.h, bf16);
-        if (training || plan.up.splits > 1) most = max(most, static_cast<size_t>(plan.up.splits) * min(m, n) * l.h);
+        if (plan.up.splits > 1) most = max(most, static_cast<size_t>(plan.up.splits) * min(m, n) * l.h);
         if (plan.down.splits > 1) most = max(most, static_cast<size_t>(plan.down.splits) * min(m, n) * l.d);
     }
     l.partials = take(most * 4);
@@ -1908,29 +1912,30 @@ PrefillLayout plan_layout(bool bf16, bool training, uint32_t n, uint32_t d, uint
 }
 
 // The last layouts of the thread by their arguments (each plans every row count up to n: ~10 us of host time at 2048).
-PrefillLayout prefill_layout(bool bf16, bool training, uint32_t n, uint32_t d, uint32_t h) {
+PrefillLayout prefill_layout(bool bf16, uint32_t n, uint32_t d, uint32_t h) {
     struct Entry {
-        bool bf16, training;
+        bool bf16;
         uint32_t n, d, h;
         PrefillLayout layout;
     };
     thread_local Entry entries[8] = {};
     thread_local uint32_t next = 0;
     for (const Entry& e : entries)
-        if (e.n == n && e.d == d && e.h == h && e.bf16 == bf16 && e.training == training) return e.layout;
+        if (e.n == n && e.d == d && e.h == h && e.bf16 == bf16) return e.layout;
     Entry& e = entries[next++ % 8];
-    e = {bf16, training, n, d, h, plan_layout(bf16, training, n, d, h)};
+    e = {bf16, n, d, h, plan_layout(bf16, n, d, h)};
     return e.layout;
 }
 
-uint64_t prefill_workspace_bytes(int vt, uint32_t n, uint32_t d, uint32_t h) { return prefill_layout(vt == kBF16, false, n, d, h).bytes; }
+uint64_t prefill_workspace_bytes(int vt, uint32_t n, uint32_t d, uint32_t h) { return prefill_layout(vt == kBF16, n, d, h).bytes; }
 
 namespace {
 template <typename V>
 hipError_t prefill(const PrefillCall& c, hipStream_t stream) {
     constexpr bool kLoB = sizeof(V) == 4;
+    constexpr uint32_t kParts = kLoB ? 2 : 1;
     constexpr int kUpChain = kLoB ? kUpChainF32 : kUpChainBf16;
-    const PrefillLayout l = prefill_layout(!kLoB, false, c.n, c.d, c.h);
+    const PrefillLayout l = prefill_layout(!kLoB, c.n, c.d, c.h);
     char* w = static_cast<char*>(c.workspace);
     const auto halves = [&](size_t at) { return reinterpret_cast<_Float16*>(w + at); };
     const auto words = [&](size_t at) { return reinterpret_cast<int32_t*>(w + at); };
@@ -1939,11 +1944,11 @@ hipError_t prefill(const PrefillCall& c, hipStream_t stream) {
     const DensSide down{c.down_off, c.down_idx, c.down_val, nullptr, c.d, l.d, l.h, chain_bits(kPrefillDownChain), slots_aligned(c.down_idx, c.down_val), halves(l.down_planes), words(l.down_exp)};
     for (uint32_t t0 = 0; t0 < c.n; t0 += kPrefillPiece) {
         const uint32_t n = min(kPrefillPiece, c.n - t0), rows = rows_padded(n), split_blocks = rows_live(n) / kSplitBlockRows / kSplitGroups;
-        const uint32_t up_blocks = t0 == 0 ? dens_blocks(l.h, l.d) : 0, down_blocks = t0 == 0 ? dens_blocks(l.d, l.h) : 0;
+        const uint32_t up_blocks = t0 == 0 ? dens_blocks(l.h, l.d, kParts) : 0, down_blocks = t0 == 0 ? dens_blocks(l.d, l.h, kParts) : 0;
         const float* x = c.x + static_cast<size_t>(t0) * c.d;
         float* y = c.y + static_cast<size_t>(t0) * c.d;
         hipLaunchKernelGGL(prefill_prep_kernel<V>, dim3(up_blocks + down_blocks + split_blocks), dim3(kDensThreads), 0, stream, up, down,
-                           up_blocks, down_blocks, split_blocks, x, n, rows, l.d, c.d, halves(l.x_planes), words(l.x_exp),
+                           up_blocks, split_blocks, 0u, x, n, rows, l.d, c.d, halves(l.x_planes), words(l.x_exp),
                            static_cast<float*>(nullptr), 0u, 1u, false);
         if (hipError_t status = hipGetLastError(); status != hipSuccess) return status;
         const PrefillPlan plan = prefill_plan(n, l.d, l.h, !kLoB);
@@ -1977,32 +1982,30 @@ hipError_t launch_prefill(int vt, const PrefillCall& call, hipStream_t stream) {
 }
 
 // Workspace of the dense sampled product (bytes, 256-aligned parts): the planes of A [rows, k_pad] and B [cols,
-// k_pad] (tokens padded to a multiple of 256, split_rows' k granularity), their row binades and the GEMM's partials. The GEMM
-// takes the chained tiles: 2048 tokens on 1024 x 4096 are 128 tiles of 256 rows, half of the CUs, and 256 of 128 rows.
+// k_pad] (tokens padded to a multiple of 256, split_rows' k granularity), their row binades and the GEMM's partials.
 namespace {
 struct GradDenseLayout {
     size_t a_planes, b_planes, a_exp, b_exp, partials, bytes;
-    uint32_t k_pad;
-    ChainPlan plan;
+    uint32_t k_pad, splits;
 };
 GradDenseLayout grad_dense_layout(uint32_t rows, uint32_t cols, uint32_t n) {
     GradDenseLayout l{};
     l.k_pad = ceil_div(n, 256) * 256;
-    l.plan = chain_plan(rows, cols, l.k_pad, false, 1, 1);
+    l.splits = dma_up_splits(rows, cols, l.k_pad);
     l.a_planes = 0;
     l.b_planes = align256(l.a_planes + dense_plane_halves(rows, l.k_pad) * 2);
     l.a_exp = align256(l.b_planes + dense_plane_halves(cols, l.k_pad) * 2);
     l.b_exp = align256(l.a_exp + static_cast<size_t>(rows) * 4);
     l.partials = align256(l.b_exp + static_cast<size_t>(cols) * 4);
-    l.bytes = l.partials + static_cast<size_t>(l.plan.splits) * rows * cols * 4;
+    l.bytes = l.partials + static_cast<size_t>(l.splits) * rows * cols * 4;
     return l;
 }
 }  // namespace
 
 size_t grad_dense_workspace_bytes(uint32_t rows, uint32_t cols, uint32_t n) {
     if (rows % kRowPad != 0 || cols % kDmaBN != 0) return 0;
-    // (few tiles: the gather is the better one)
-    return dma_up_splits(rows, cols, ceil_div(n, 256) * 256) == 0 ? 0 : grad_dense_layout(rows, cols, n).bytes;
+    const GradDenseLayout l = grad_dense_layout(rows, cols, n);
+    return l.splits == 0 ? 0 : l.bytes;
 }
 
 hipError_t launch_grad_dense(const float* row, const float* mat, const int32_t* off, const int16_t* idx, float* g, float* gb,
@@ -2015,13 +2018,13 @@ hipError_t launch_grad_dense(const float* row, const float* mat, const int32_t* 
     auto* b_exp = reinterpret_cast<int32_t*>(w + l.b_exp);
     auto* partials = reinterpret_cast<float*>(w + l.partials);
     hipLaunchKernelGGL(split_pair_kernel, dim3((rows + cols) / kSplitBlockRows), dim3(kThreads), 0, stream, row, rows, a_planes, a_exp, mat, cols,
-                       b_planes, b_exp, l.k_pad, ld, n, chain_bits(kUpChainF32));
+                       b_planes, b_exp, l.k_pad, ld, n);
     if (hipError_t status = hipGetLastError(); status != hipSuccess) return status;
-    if (hipError_t status = launch_chained<Epi::UpSplit, true, kUpChainF32>(l.plan.bm, a_planes, a_exp, b_planes, b_exp, nullptr, partials,
-                                                                            nullptr, nullptr, rows, cols, l.k_pad, l.plan.splits, cols, stream);
+    if (hipError_t status = launch_dma<Epi::UpSplit, true>(a_planes, a_exp, b_planes, b_exp, nullptr, partials, nullptr, nullptr, rows,
+                                                           cols, l.k_pad, l.splits, stream);
         status != hipSuccess)
         return status;
-    hipLaunchKernelGGL(gather_dense_kernel, dim3(ceil_div(rows, kThreads / kWave)), dim3(kThreads), 0, stream, partials, l.plan.splits, row,
+    hipLaunchKernelGGL(gather_dense_kernel, dim3(ceil_div(rows, kThreads / kWave)), dim3(kThreads), 0, stream, partials, l.splits, row,
                        ld, n, off, idx, g, gb, rows, cols);
     return hipGetLastError();
 }
@@ -2057,96 +2060,6 @@ hipError_t launch_train_forward(const float* x, const void* up_planes, const int
     return launch_mfma_down(kF32, down_planes, down_exp, b_down, y, workspace, n, d, h, stream);
 }
 
-// Training on planes densified per call, in the workspace of the training layout (train_planes_workspace_bytes): the
-// chained GEMMs, as launch_prefill. `in` is x or gy; the sides are W_up and W_down, or W_down^T and W_up^T.
-namespace {
-struct TrainWork {
-    PrefillLayout l;
-    _Float16 *in_planes, *mid_planes;
-    int32_t *in_exp, *mid_exp;
-    float* partials;
-    DensSide first, second;  // [h rows, d k] and [d rows, h k]
-};
-TrainWork train_work(void* workspace, uint32_t n, uint32_t d, uint32_t h) {
-    const PrefillLayout l = prefill_layout(false, true, n, d, h);
-    char* w = static_cast<char*>(workspace);
-    const auto halves = [&](size_t at) { return reinterpret_cast<_Float16*>(w + at); };
-    const auto words = [&](size_t at) { return reinterpret_cast<int32_t*>(w + at); };
-    TrainWork t{l, halves(l.x_planes), halves(l.act_planes), words(l.x_exp), words(l.act_exp), reinterpret_cast<float*>(w + l.partials), {}, {}};
-    t.first = {nullptr, nullptr, nullptr, nullptr, h, l.h, l.d, chain_bits(kUpChainF32), true, halves(l.up_planes), words(l.up_exp)};
-    t.second = {nullptr, nullptr, nullptr, nullptr, d, l.d, l.h, chain_bits(kPrefillDownChain), true, halves(l.down_planes), words(l.down_exp)};
-    return t;
-}
-void set_slots(DensSide& side, const int32_t* off, const int16_t* idx, const float* val, const int32_t* pos) {
-    side.off = off, side.idx = idx, side.val = val, side.pos = pos;
-    side.vec = slots_aligned(idx, pos != nullptr ? static_cast<const void*>(pos) : val);
-}
-// Whether densifying reads a side's values by position as it goes, or from a copy gathered first: a block of each column
-// chunk reads its rows' slots, twice where a wave does not hold them, and a gathered 4-byte read costs a cache line. 1024 x
-// 4096 at 512 and 2048 tokens: up_t at 50 % (2 chunks of rows of 2048 slots, 8.4 M reads) 68 us in place, 14.6 + 12 us
-// gathered first; at 10 % (0.84 M reads) in place costs the launch 4 us, gathering first 4.8 and a launch.
-bool gathers_in_place(const DensSide& side, uint32_t nnz) {
-    const uint32_t reads = ceil_div(side.k, kDensChunk) * (nnz / side.rows > 1016 ? 2 : 1);
-    return reads == 1 || static_cast<uint64_t>(reads) * nnz <= 1u << 20;
-}
-hipError_t train_prep(const TrainWork& t, const float* in, float* in_t, uint32_t n, uint32_t d, uint32_t ld, hipStream_t stream) {
-    const uint32_t up_blocks = dens_blocks(t.l.h, t.l.d), down_blocks = dens_blocks(t.l.d, t.l.h);
-    const uint32_t split_blocks = rows_live(n) / kSplitBlockRows / kSplitGroups, tiles_c = d / kTransCols;
-    hipLaunchKernelGGL(prefill_prep_kernel<float>,
-                       dim3(up_blocks + down_blocks + split_blocks + ceil_div(tiles_c * ceil_div(n, kTransRows), kSplitGroups)), dim3(kDensThreads),
-                       0, stream, t.first, t.second, up_blocks, down_blocks, split_blocks, in, n, rows_padded(n), t.l.d, d, t.in_planes, t.in_exp,
-                       in_t, ld, tiles_c, transpose_vectors(in, in_t, d, ld));
-    return hipGetLastError();
-}
-// partials = in [n, d] first^T, then the epilogue MODE (train_planes_kernel); out = mid [n, h] second^T (+ bias)
-template <TrainPost MODE>
-hipError_t train_products(const TrainWork& t, const float* b_up, const float* z_in, float* out_a, float* out_b, const float* bias, float* out,
-                          uint32_t n, uint32_t d, uint32_t h, uint32_t ld, hipStream_t stream) {
-    const PrefillPlan plan = prefill_plan(n, t.l.d, t.l.h, false);
-    if (hipError_t status = launch_chained<Epi::UpSplit, true, kUpChainF32>(plan.up.bm, t.in_planes, t.in_exp, t.first.planes, t.first.exps,
-                                                                            nullptr, t.partials, nullptr, nullptr, n, h, d, plan.up.splits, h,
-                                                                            stream);
-        status != hipSuccess)
-        return status;
-    hipLaunchKernelGGL(train_planes_kernel<MODE>, dim3(rows_live(n) / kTrainRows, h / kActBlock), dim3(kTrainThreads), 0, stream, t.partials,
-                       plan.up.splits, b_up, z_in, out_a, out_b, t.mid_planes, reinterpret_cast<int8_t*>(t.mid_exp), n, rows_padded(n), h, ld);
-    if (hipError_t status = hipGetLastError(); status != hipSuccess) return status;
-    const bool parts = plan.down.splits > 1;
-    if (hipError_t status = launch_chained<Epi::Down, true, kPrefillDownChain>(plan.down.bm, t.mid_planes, t.mid_exp, t.second.planes,
-                                                                               t.second.exps, bias, parts ? t.partials : out, nullptr, nullptr,
-                                                                               n, d, h, plan.down.splits, d, stream);
-        status != hipSuccess || !parts)
-        return status;
-    return launch_reduce_splits(t.partials, bias, out, n, plan.down.splits, d, 0, d, stream);
-}
-}  // namespace
-
-uint64_t train_planes_workspace_bytes(uint32_t n, uint32_t d, uint32_t h) { return prefill_layout(false, true, n, d, h).bytes; }
-
-hipError_t launch_train_planes_forward(const PrefillCall& c, float* x_t, float* act, float* z, uint32_t ld, hipStream_t stream) {
-    TrainWork t = train_work(c.workspace, c.n, c.d, c.h);
-    set_slots(t.first, c.up_off, c.up_idx, static_cast<const float*>(c.up_val), nullptr);
-    set_slots(t.second, c.down_off, c.down_idx, static_cast<const float*>(c.down_val), nullptr);
-    if (hipError_t status = train_prep(t, c.x, x_t, c.n, c.d, ld, stream); status != hipSuccess) return status;
-    return train_products<TrainPost::Forward>(t, c.b_up, nullptr, z, act, c.b_down, c.y, c.n, c.d, c.h, ld, stream);
-}
-
-hipError_t launch_train_planes_backward(const TrainBackward& c, hipStream_t stream) {
-    TrainWork t = train_work(c.workspace, c.n, c.d, c.h);
-    const auto side = [&](DensSide& to, const int32_t* off, const int16_t* idx, const int32_t* pos, const float* val, float* values, uint32_t nnz) {
-        if (gathers_in_place(to, nnz)) {
-            set_slots(to, off, idx, val, pos);
-            return hipSuccess;
-        }
-        set_slots(to, off, idx, values, nullptr);
-        return launch_gather_values(val, pos, values, nnz, stream);
-    };
-    if (hipError_t status = side(t.first, c.hid_off, c.hid_output, c.hid_pos, c.out_val, c.hid_val, c.nnz_down); status != hipSuccess) return status;
-    if (hipError_t status = side(t.second, c.in_off, c.in_hidden, c.in_pos, c.up_val, c.in_val, c.nnz_up); status != hipSuccess) return status;
-    if (hipError_t status = train_prep(t, c.gy, c.gy_t, c.n, c.d, c.ld, stream); status != hipSuccess) return status;
-    return train_products<TrainPost::GradZ>(t, nullptr, c.z, c.gz, nullptr, nullptr, c.gx, c.n, c.d, c.h, c.ld, stream);
-}
-
 // Training backward products on the planes: gy split into planes; gz = (gy W_down) * gelu'(z) as a split product over
 // the planes of W_down^T [d_ff rows, d_model k] whose epilogue (train_planes_kernel<GradZ>) writes gz hidden-major and
 // as planes; gx = gz W_up by the down GEMM over the planes of W_up^T [d_model rows, d_ff k], without bias.
@@ -2172,6 +2085,82 @@ hipError_t launch_train_backward(const float* gy, const float* z, const void* do
                        rows_padded(n), h, ld);
     if (hipError_t status = hipGetLastError(); status != hipSuccess) return status;
     return launch_mfma_down(kF32, up_t_planes, up_t_exp, nullptr, gx, workspace, n, d, h, stream);
+}
+
+// The training backward with its planes densified per call into the workspace (train_planes_workspace_bytes): W_down^T and
+// W_up^T from the transposed supports (values read by position), gy split and transposed, all in one launch, then the
+// products of launch_train_backward with the same splits: the same bits.
+namespace {
+struct TrainPlanes {
+    size_t up_planes, up_exp, down_planes, down_exp, x_exp, act_exp, x_planes, act_planes, partials, bytes;
+};
+TrainPlanes train_planes_layout(uint32_t n, uint32_t d, uint32_t h) {
+    TrainPlanes l{};
+    const size_t rows = rows_padded(n);
+    size_t at = 0;
+    const auto take = [&at](size_t bytes) {
+        const size_t from = at;
+        at = align256(at + bytes);
+        return from;
+    };
+    l.up_planes = take(dense_plane_halves(h, d) * 2);
+    l.up_exp = take(static_cast<size_t>(h) * 4);
+    l.down_planes = take(dense_plane_halves(d, h) * 2);
+    l.down_exp = take(static_cast<size_t>(d) * 4);
+    l.x_exp = take(rows * 4);
+    l.act_exp = take(rows * (h / kActBlock));
+    l.x_planes = take(dense_plane_halves(rows, d) * 2);
+    l.act_planes = take(dense_plane_halves(rows, h) * 2);
+    l.partials = at;  // the last: no other offset depends on n's splits
+    l.bytes = at + train_partial_floats(n, d, h) * 4;
+    return l;
+}
+// Whether densifying reads a side's values by position as it goes, or from a copy gathered first: a block of each column
+// chunk reads its rows' slots, twice where a wave does not hold them, and a gathered 4-byte read costs a cache line. 1024 x
+// 4096: up_t at 50 % (rows of 2048 slots, 8.4 M reads) 68 us in place, 14.6 + 12 us gathered first.
+bool gathers_in_place(const DensSide& side, uint32_t nnz) {
+    const uint32_t reads = ceil_div(side.k, dens_chunk(2)) * (nnz / side.rows > 512 ? 2 : 1);
+    return reads == 1 || static_cast<uint64_t>(reads) * nnz <= 1u << 20;
+}
+}  // namespace
+
+uint64_t train_planes_workspace_bytes(uint32_t n, uint32_t d, uint32_t h) { return train_planes_layout(n, d, h).bytes; }
+
+hipError_t launch_train_planes_backward(const TrainBackward& c, hipStream_t stream) {
+    const TrainPlanes l = train_planes_layout(c.n, c.d, c.h);
+    char* w = static_cast<char*>(c.workspace);
+    const auto halves = [&](size_t at) { return reinterpret_cast<_Float16*>(w + at); };
+    const auto words = [&](size_t at) { return reinterpret_cast<int32_t*>(w + at); };
+    DensSide down_t{c.hid_off, c.hid_output, nullptr, nullptr, c.h, c.h, c.d, kNoChains, true, halves(l.up_planes), words(l.up_exp)};
+    DensSide up_t{c.in_off, c.in_hidden, nullptr, nullptr, c.d, c.d, c.h, kNoChains, true, halves(l.down_planes), words(l.down_exp)};
+    const auto values = [&](DensSide& side, const int32_t* pos, const float* val, float* gathered, uint32_t nnz) {
+        const bool in_place = gathers_in_place(side, nnz);
+        side.val = in_place ? val : gathered;
+        side.pos = in_place ? pos : nullptr;
+        side.vec = slots_aligned(side.idx, in_place ? static_cast<const void*>(pos) : gathered);
+        return in_place ? hipSuccess : launch_gather_values(val, pos, gathered, nnz, stream);
+    };
+    if (hipError_t status = values(down_t, c.hid_pos, c.out_val, c.hid_val, c.nnz_down); status != hipSuccess) return status;
+    if (hipError_t status = values(up_t, c.in_pos, c.up_val, c.in_val, c.nnz_up); status != hipSuccess) return status;
+    const uint32_t up_blocks = dens_blocks(c.h, c.d, 2), down_blocks = dens_blocks(c.d, c.h, 2), rows = rows_padded(c.n);
+    const uint32_t split_blocks = rows_live(c.n) / kSplitBlockRows / kSplitGroups, tiles_c = c.d / kTransCols;
+    const uint32_t trans_blocks = ceil_div(tiles_c * ceil_div(c.n, kTransRows), kSplitGroups);
+    hipLaunchKernelGGL(prefill_prep_kernel<float>, dim3(up_blocks + down_blocks + split_blocks + trans_blocks), dim3(kDensThreads), 0, stream,
+                       down_t, up_t, up_blocks, split_blocks, trans_blocks, c.gy, c.n, rows, c.d, c.d, halves(l.x_planes), words(l.x_exp),
+                       c.gy_t, c.ld, tiles_c, transpose_vectors(c.gy, c.gy_t, c.d, c.ld));
+    if (hipError_t status = hipGetLastError(); status != hipSuccess) return status;
+    float* partials = reinterpret_cast<float*>(w + l.partials);
+    const uint32_t splits = max(1u, dma_up_splits(c.n, c.h, c.d));
+    if (hipError_t status = launch_dma<Epi::UpSplit, true>(halves(l.x_planes), words(l.x_exp), down_t.planes, down_t.exps, nullptr, partials,
+                                                           nullptr, nullptr, c.n, c.h, c.d, splits, stream);
+        status != hipSuccess)
+        return status;
+    hipLaunchKernelGGL(train_planes_kernel<TrainPost::GradZ>, dim3(rows_live(c.n) / kTrainRows, c.h / kActBlock), dim3(kTrainThreads), 0, stream,
+                       partials, splits, nullptr, c.z, c.gz, nullptr, halves(l.act_planes), reinterpret_cast<int8_t*>(w + l.act_exp), c.n, rows,
+                       c.h, c.ld);
+    if (hipError_t status = hipGetLastError(); status != hipSuccess) return status;
+    return dma_down<true>(dma_down_plan(c.n, c.d, c.h, false), halves(l.act_planes), words(l.act_exp), up_t.planes, up_t.exps, nullptr, c.gx,
+                          partials, c.n, c.d, c.h, stream);
 }
 
 }  // namespace hffn

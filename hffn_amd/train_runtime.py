@@ -22,11 +22,10 @@ and ``g_up``/``gb_up`` as gathers over 256-token tiles (``hffn_grad_sddmm``, til
 ``hffn_reduce_tiles``) or, from ``GRAD_DENSE_MIN_TOKENS`` tokens on dense enough layers, as split-fp16 MFMA products
 sampled at the support (``hffn_grad_dense``); ``gz`` by ``hffn_grad_hidden``; ``gx`` by ``hffn_grad_x``; AdamW in
 one launch (``hffn_adamw_arrays``). After an update the runtime's densified planes of that layer are rebuilt before their next use.
-From ``TRAIN_MFMA_MIN_TOKENS`` tokens (``train_mode``) the forward with z, gz and gx run as split-fp16 MFMA products
-instead: the forward on the runtime's densified planes where it holds them (``hffn_forward_mfma_z``), else, where
-estimated faster than the gathers, on planes densified for the call (``hffn_forward_planes_z``); the backward always on
-planes of W_down^T and W_up^T densified for the call, the values read from the compact arrays by position
-(``hffn_backward_planes``), so that the values in the transposed orders are gathered by the gather backward only.
+On layers whose runtime holds densified planes, from ``TRAIN_MFMA_MIN_TOKENS`` tokens (``train_mode``), the forward
+with z (``hffn_forward_mfma_z``) and gz, gx (``hffn_backward_planes``) run as split-fp16 MFMA products instead, the
+backward over planes of W_down^T and W_up^T densified at every backward, the values read from the compact arrays by
+position (the gather backward gathers them into the transposed orders first).
 """
 from __future__ import annotations
 
@@ -38,8 +37,7 @@ from dataclasses import dataclass
 import torch
 
 from . import _lib
-from .runtime import (MAX_TOKENS, PAIR_MODES, ROWS_SHARE, ROWS_WALK_SLOT_US, ROWS_WALK_US, HFFNRuntime, _aligned, down_mode,
-                      edges_supported, leading_dim, mfma_streamed, prefill_us, rows_us, up_mode)
+from .runtime import MAX_TOKENS, PAIR_MODES, HFFNRuntime, _aligned, down_mode, edges_supported, leading_dim, mfma_streamed, up_mode
 
 PARAMETERS = ("up_val", "b_up", "out_val", "b_down")
 SUPPORTS = ("in_offsets", "in_pos", "in_hidden", "hid_offsets", "hid_pos", "hid_output")
@@ -106,8 +104,7 @@ class HFFNTrainRuntime:
         self.forced_grad: str | None = None    # diagnostic: the sampled products' formulation, else the policy's
         self.forced_train: str | None = None   # diagnostic: the forward with z, gz and gx on gathers or planes
         self._mfma_work: torch.Tensor | None = None    # forward on the runtime's planes
-        self._planes_work: torch.Tensor | None = None  # planes densified per call
-        self._planes_shapes = bool(self._lib.hffn_mfma_supported(self.d_model, self.d_ff))
+        self._planes_work: torch.Tensor | None = None  # the backward's planes and buffers
         self._modes: dict = {}                  # (what, N, forced) -> mode
         self._tokens = 0                        # N the dense buffers hold
         self._tiles = 1                         # token tiles the partials hold (none allocated for 1)
@@ -169,25 +166,14 @@ class HFFNTrainRuntime:
     def _mfma_possible(self, n: int) -> bool:
         return self.runtime.mfma_available and mfma_streamed(n, self.d_model, self.d_ff)
 
-    def _planes_possible(self, n: int) -> bool:
-        """Whether the forward with z may run on planes densified for the call at N."""
-        return self._planes_shapes and self.runtime._transient_allowed and not self.runtime.mfma_available
-
-    def _planes_preferred(self, n: int) -> bool:
-        """Whether the forward with z is estimated faster on planes densified for the call than on the lane-per-token
-        gathers (the backward's gz and gx are the same products)."""
-        gather = max(ROWS_SHARE * rows_us(n, self.runtime._store), ROWS_WALK_US + ROWS_WALK_SLOT_US * self.runtime._longest)
-        return self._planes_possible(n) and prefill_us(n, self.d_model, self.d_ff, False) < gather
-
     def _grow_mfma(self, n: int) -> None:
         """The workspaces of the MFMA products at N, when they may run at N."""
-        if self.train_mode(n) != "mfma":
+        if not self._mfma_possible(n):
             return
-        if self._mfma_possible(n):
-            need = _lib.query_bytes(self._lib.hffn_train_mfma_workspace, n, self.d_model, self.d_ff)
-            if self._mfma_work is None or need > self._mfma_work.numel():
-                self._mfma_work = torch.zeros(need, dtype=torch.uint8, device=self.runtime.device)
-                self.growths += 1
+        need = _lib.query_bytes(self._lib.hffn_train_mfma_workspace, n, self.d_model, self.d_ff)
+        if self._mfma_work is None or need > self._mfma_work.numel():
+            self._mfma_work = torch.zeros(need, dtype=torch.uint8, device=self.runtime.device)
+            self.growths += 1
         need = _lib.query_bytes(self._lib.hffn_train_planes_workspace, n, self.d_model, self.d_ff)
         if self._planes_work is None or need > self._planes_work.numel():
             self._planes_work = torch.empty(need, dtype=torch.uint8, device=self.runtime.device)
@@ -240,13 +226,12 @@ class HFFNTrainRuntime:
 
     def train_mode(self, n: int) -> str:
         """``mfma`` (the forward with z, gz and gx as split-fp16 MFMA products over densified planes) from
-        ``TRAIN_MFMA_MIN_TOKENS`` tokens when the runtime runs its policy (no forced pair) and either holds planes and the
-        streamed GEMM takes N, or holds none and planes densified for the call are estimated faster; else ``gather``.
-        ``forced_train`` overrides the choice."""
+        ``TRAIN_MFMA_MIN_TOKENS`` tokens when the runtime holds planes, runs its policy (no forced pair) and the streamed
+        GEMM takes N, else ``gather``; ``forced_train`` overrides the choice."""
         if self.forced_train is not None:
             if self.forced_train not in TRAIN_MODES:
                 raise ValueError(f"training mode is one of {TRAIN_MODES}, not {self.forced_train!r}")
-            if self.forced_train == "mfma" and not (self._mfma_possible(n) or self._planes_possible(n)):
+            if self.forced_train == "mfma" and not self._mfma_possible(n):
                 raise ValueError(f"the planes products do not run at N={n} on {self.d_model} x {self.d_ff} (no planes, or "
                                  "a shape the streamed GEMM refuses)")
             return self.forced_train
@@ -254,7 +239,7 @@ class HFFNTrainRuntime:
             return "gather"
         mode = self._modes.get(("train", n))
         if mode is None:
-            mode = self._modes["train", n] = "mfma" if self._mfma_possible(n) or self._planes_preferred(n) else "gather"
+            mode = self._modes["train", n] = "mfma" if self._mfma_possible(n) else "gather"
         return mode
 
     def _runtime_planes(self, index: int) -> dict:
@@ -299,14 +284,7 @@ class HFFNTrainRuntime:
             raise ValueError(f"z must be a contiguous float32 device tensor of at least {self.d_ff * ld} entries")
         self.reserve(n)
         x_t, act, y_t, y = runtime._work
-        if self.train_mode(n) == "mfma" and not runtime.mfma_available:
-            x = _aligned(x)
-            _, *model = runtime._args[index]
-            _lib.check(self._lib.hffn_forward_planes_z(x.data_ptr(), *model, self._planes_work.data_ptr(), self._planes_work.numel(), x_t,
-                                                       act, z.data_ptr(), y, self.d_model, self.d_ff, n, ld, _stream(runtime.device)),
-                       "forward with z (planes of the call)")
-            self.calls["mfma", "mfma"] += 1
-        elif self.train_mode(n) == "mfma":
+        if self.train_mode(n) == "mfma":
             planes, tensors, x = self._runtime_planes(index), runtime._tensors[index], _aligned(x)
             _lib.check(self._lib.hffn_forward_mfma_z(x.data_ptr(), planes["up"].data_ptr(), planes["up_binades"].data_ptr(),
                                                      tensors["b_up"].data_ptr(), planes["down"].data_ptr(),
@@ -348,7 +326,7 @@ class HFFNTrainRuntime:
                                                 arrays["up_val"].data_ptr(), values["hid_val"].data_ptr(), values["in_val"].data_ptr(),
                                                 self._planes_work.data_ptr(), self._planes_work.numel(), self._gy_t.data_ptr(),
                                                 self._gz.data_ptr(), self._gx.data_ptr(), d, h, *runtime._nnz[index], n, ld, stream),
-                       "gz, gx (planes of the call)")
+                       "gz, gx (mfma)")
         else:
             _lib.check(lib.hffn_backward_prepare(gy.data_ptr(), self._gy_t.data_ptr(), arrays["out_val"].data_ptr(),
                                                  supports["hid_pos"].data_ptr(), values["hid_val"].data_ptr(), arrays["up_val"].data_ptr(),

@@ -329,16 +329,11 @@ int hffn_backward_mfma(const float* gy, const float* z, const void* down_t_plane
                        const int32_t* up_t_binades, void* workspace, uint64_t workspace_bytes, float* gz, float* gx, uint32_t d_model,
                        uint32_t d_ff, uint32_t n, uint32_t ld, void* stream);
 
-/* The same products on planes densified for the call (widths multiples of 256, any n, no resident planes; float32 sums
- * in chains of at most 128 k): hffn_forward_planes_z from the compact rows; hffn_backward_planes, which also writes gy_t
- * (gy transposed, [d_model, ld]), from the transposed supports, whose slot s holds out_val[hid_pos[s]] or
- * up_val[in_pos[s]] (hid_val and in_val: buffers of nnz_down and nnz_up floats for them). The workspace (hffn_train_planes_workspace bytes, any content) is 256-byte aligned, float buffers
- * 16-byte aligned. */
+/* hffn_backward_mfma with its planes densified for the call, the same bits; it also writes gy_t (gy transposed, [d_model,
+ * ld]). The planes come from the transposed supports, whose slot s holds out_val[hid_pos[s]] or up_val[in_pos[s]]
+ * (hid_val and in_val: buffers of nnz_down and nnz_up floats for them). The workspace (hffn_train_planes_workspace bytes,
+ * any content) is 256-byte aligned, float buffers 16-byte aligned. */
 int hffn_train_planes_workspace(uint32_t n, uint32_t d_model, uint32_t d_ff, uint64_t* bytes);
-int hffn_forward_planes_z(const float* x, const int32_t* up_offsets, const int16_t* up_idx, const float* up_val, const float* b_up,
-                          const int32_t* out_offsets, const int16_t* out_hidden, const float* out_val, const float* b_down,
-                          void* workspace, uint64_t workspace_bytes, float* x_t, float* act, float* z, float* y, uint32_t d_model,
-                          uint32_t d_ff, uint32_t n, uint32_t ld, void* stream);
 int hffn_backward_planes(const float* gy, const float* z, const int32_t* hid_offsets, const int16_t* hid_output, const int32_t* hid_pos,
                          const float* out_val, const int32_t* in_offsets, const int16_t* in_hidden, const int32_t* in_pos,
                          const float* up_val, float* hid_val, float* in_val, void* workspace, uint64_t workspace_bytes, float* gy_t,

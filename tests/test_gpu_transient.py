@@ -133,47 +133,6 @@ def test_policy_plans_and_capture(device):
     assert not never.transient(n) and never._prefill_work is None
 
 
-@pytest.mark.parametrize("name,n,mode", [("homog_256_1024", 65, "mfma"), ("irreg_512_2048", 100, "mfma"), ("irreg_512_2048", 300, None),
-                                         ("homog_512_2048", 2100, None)])
-def test_training_on_planes_of_the_call(name, n, mode, device):
-    """The training step of a runtime without planes, forward with z, gz and gx on planes densified for the call: every
-    group within 10x the float64 distance of the dense float32 control (floor 1e-7 of its largest entry), the updates
-    against AdamW's closed form, the same bits twice from the same state, no buffer growth in a step after reserve."""
-    from oracle import train as oracle_train
-    from test_gpu_train import GRAD_OF, GROUPS, HYPER, _update_errors, build_groups, control_groups, hidden_major_state, make_gy
-
-    from hffn_amd.train_runtime import HFFNTrainRuntime
-    case = synth.CASES[name]
-    layer = synth.make_layer(case)
-    x, gy = torch.from_numpy(synth.make_input(case, n)).to(device), make_gy(case, n, 0).to(device)
-    train = HFFNTrainRuntime(HFFNRuntime([hip_layer(layer)], device), **HYPER, max_tokens=n)
-    train.forced_train = mode
-    assert not train.runtime.mfma_available and train.train_mode(n) == "mfma"
-    train.reserve(n)
-    growths, initial = train.growths, {k: v.clone() for k, v in train.parameters(0).items()}
-    before = hidden_major_state(train, layer)
-    ref, control = oracle_train.step_groups(layer, x.cpu().numpy(), gy.cpu().numpy()), control_groups(layer, x, gy)
-    train.step(0, x, gy)
-    torch.cuda.synchronize()
-    assert train.growths == growths and train.calls["mfma", "mfma"] == 1
-    groups = build_groups(train, layer, n)
-    for g in GROUPS:
-        scale = float(np.abs(ref[g]).max())
-        assert float(np.abs(groups[g] - ref[g]).max()) <= 10 * max(float(np.abs(control[g] - ref[g]).max()), 1e-7 * scale), g
-    masks = {g: np.abs(ref[g]) >= 100 * float(np.abs(control[g] - ref[g]).max()) for g in GRAD_OF.values()}
-    assert _update_errors(before, hidden_major_state(train, layer), groups, masks, 1) <= 1e-5
-    first = [t.clone() for t in (train._gx[:n], *train.gradients(0).values(), *train.parameters(0).values())]
-    for k, v in train.parameters(0).items():
-        v.copy_(initial[k])
-    for pair in train.moments(0).values():
-        for t in pair:
-            t.zero_()
-    train.steps[0] = 0
-    train.step(0, x, gy)
-    again = (train._gx[:n], *train.gradients(0).values(), *train.parameters(0).values())
-    assert all(torch.equal(a, b) for a, b in zip(first, again))
-
-
 def test_prefill_refusals(device):
     lib, size = _lib.load(), ctypes.c_uint64(0)
     p, odd = 256, 264  # never dereferenced: the calls are refused before any launch
