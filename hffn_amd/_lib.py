@@ -36,6 +36,7 @@ SIGNATURES = {
     "hffn_grad_dense": [_P] * 6 + [_U32] * 4 + [_P, _U64, _P],
     "hffn_train_mfma_workspace": [_U32, _U32, _U32, ctypes.POINTER(_U64)],
     "hffn_forward_mfma_z": [_P] * 7 + [_P, _U64] + [_P] * 4 + [_U32] * 4 + [_P],
+    "hffn_forward_mfma_z_refresh": [_P] * 14 + [_U64] + [_P] * 4 + [_U32] * 4 + [_P],
     "hffn_backward_mfma": [_P] * 7 + [_U64, _P, _P] + [_U32] * 4 + [_P],
     "hffn_grad_sddmm": [_P] * 6 + [_U32] * 4 + [_P],
     "hffn_grad_hidden": [_P] * 7 + [_U32] * 5 + [_P],

@@ -785,6 +785,21 @@ int hffn_backward_mfma(const float* gy, const float* z, const void* down_t_plane
                     "backward_mfma");
 }
 
+int hffn_forward_mfma_z_refresh(const float* x, const int32_t* up_offsets, const int16_t* up_idx, const float* up_val, const float* b_up,
+                                const int32_t* out_offsets, const int16_t* out_hidden, const float* out_val, const float* b_down,
+                                void* up_planes, int32_t* up_binades, void* down_planes, int32_t* down_binades, void* workspace,
+                                uint64_t workspace_bytes, float* x_t, float* act, float* z, float* y, uint32_t d_model, uint32_t d_ff,
+                                uint32_t n, uint32_t ld, void* stream) {
+    if (int status = check_train_mfma("forward_mfma_z_refresh", d_model, d_ff, n, ld, workspace, workspace_bytes,
+                                      {x, b_up, b_down, x_t, act, z, y, up_planes, down_planes},
+                                      {up_binades, down_binades, up_offsets, up_idx, up_val, out_offsets, out_hidden, out_val}))
+        return status;
+    const hffn::TrainSlots slots{up_offsets, up_idx, up_val, out_offsets, out_hidden, out_val};
+    return launched(hffn::launch_train_forward(x, up_planes, up_binades, b_up, down_planes, down_binades, b_down, workspace, x_t, act, z, y,
+                                               n, d_model, d_ff, ld, static_cast<hipStream_t>(stream), &slots),
+                    "forward_mfma_z_refresh");
+}
+
 int hffn_train_planes_workspace(uint32_t n, uint32_t d_model, uint32_t d_ff, uint64_t* bytes) {
     if (!bytes) return fail(HFFN_ERROR_ARGUMENT, "train_planes_workspace: null result");
     if (int status = check_mfma(HFFN_VALUE_F32, d_model, d_ff, n)) return status;

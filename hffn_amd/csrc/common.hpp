@@ -125,6 +125,13 @@ __device__ __forceinline__ void load_vec(const float* p, float (&out)[N]) {
     }
 }
 
+// Block `block` of `blocks` -> its place in an order that gives every XCD (blocks are dealt to the 8 of them in turn) one
+// contiguous run: neighbours in the order share an L2.
+__device__ __forceinline__ uint32_t xcd_order(uint32_t block, uint32_t blocks) {
+    const uint32_t per = blocks / 8;
+    return block < 8 * per ? block % 8 * per + block / 8 : block;
+}
+
 // out[c, r] = in[r, c] of the tile of kTransRows x kTransCols at (r0, c0), by the kTransThreads threads t, through LDS
 // (padded by one float per row). Every thread of the block calls it (one barrier). A full tile whose rows start on
 // 16-byte boundaries on both sides (vectors: strides multiples of 4 floats, aligned pointers) moves float4s: thread t

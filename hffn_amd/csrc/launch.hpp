@@ -140,9 +140,17 @@ hipError_t launch_grad_dense(const float* row, const float* mat, const int32_t* 
 // on the inference down GEMM. The workspace is the MFMA workspace with partials at every split count; both need the
 // streamed GEMM (mfma_streamed).
 size_t train_mfma_workspace_bytes(uint32_t n, uint32_t d, uint32_t h);
+struct TrainSlots {  // the compact rows to densify the forward's planes from first (a step after an update)
+    const int32_t* up_off;
+    const int16_t* up_idx;
+    const float* up_val;
+    const int32_t* down_off;
+    const int16_t* down_idx;
+    const float* down_val;
+};
 hipError_t launch_train_forward(const float* x, const void* up_planes, const int32_t* up_exp, const float* b_up, const void* down_planes,
                                 const int32_t* down_exp, const float* b_down, void* workspace, float* x_t, float* act, float* z, float* y,
-                                uint32_t n, uint32_t d, uint32_t h, uint32_t ld, hipStream_t stream);
+                                uint32_t n, uint32_t d, uint32_t h, uint32_t ld, hipStream_t stream, const TrainSlots* slots = nullptr);
 hipError_t launch_train_backward(const float* gy, const float* z, const void* down_t_planes, const int32_t* down_t_exp,
                                  const void* up_t_planes, const int32_t* up_t_exp, void* workspace, float* gz, float* gx, uint32_t n,
                                  uint32_t d, uint32_t h, uint32_t ld, hipStream_t stream);

@@ -338,7 +338,8 @@ __device__ __forceinline__ void densify(DensTile<PARTS>& lds, const DensSide& si
     static_assert(kDensThreads / kWave == kDensRows, "a wave per row");
     const uint32_t tid = threadIdx.x, lane = tid % kWave, row = uniform(tid / kWave);
     const uint32_t groups = (side.rows_pad + kDensRows - 1) / kDensRows, chunk = block / groups;
-    const uint32_t r0 = block % groups * kDensRows, n = r0 + row, c0 = chunk * kDensChunk;
+    const uint32_t group = side.pos != nullptr ? xcd_order(block % groups, groups) : block % groups;  // values by position: neighbours share lines
+    const uint32_t r0 = group * kDensRows, n = r0 + row, c0 = chunk * kDensChunk;
     const uint32_t width = min(kDensChunk, side.k - c0), pieces = width / 8;  // width: a multiple of 32
     const bool real = n < side.rows;
     RowSlots<V> slots(side.idx, static_cast<const V*>(side.val), side.pos, real ? side.off[n] : 0, real ? side.off[n + 1] : 0, side.off[side.rows],
@@ -380,7 +381,7 @@ __global__ __launch_bounds__(kDensThreads, kDensOccupancy) void densify_kernel(D
 // What a call that densifies its own planes (launch_prefill) needs before its first GEMM, in one launch: the planes of
 // both sides from the compact rows and the input planes of x. The first split_blocks split x, kSplitGroups groups of 8
 // rows a block, the next trans_blocks transpose it (training), the next up_blocks densify W_up, the others W_down (the
-// split, a block's longest work, first: last it was the launch's tail, 46 us instead of PREPT at 1999 tokens on 2048 x 8192).
+// split, a block's longest work, first: last it was the launch's tail, 46 us instead of 34.5 at 1999 tokens on 2048 x 8192).
 // MI355X: 7.8 us on 512 x 2048 at 20 % (float32, 128 tokens), 17 on 1024 x 4096 at 10 % with uneven rows, 28 on 2048 x
 // 8192 at 20 % (bfloat16, 128 tokens; 72 with single slots a lane in place of 8, 38 in blocks of 1024 threads, two per CU).
 // A block is a chain of four round trips (offsets, slots, LDS, stores): many small blocks cover one another.
@@ -824,7 +825,7 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
     constexpr int W = kDmaWaves, MI = BM == kDmaBM ? 2 : 1, NI = BM == 64 ? 1 : 2, BN = kDmaBN, S = dma_stages(BM);
     constexpr uint32_t kT = 64 * W, kWaveRows = 32 * MI, kWaveCols = 32 * NI, kWavesN = BN / kWaveCols;
     static_assert(kWaveRows * (W / kWavesN) == BM, "the waves cover the block's rows");
-    static_assert(BM == kDmaBM || (CHAIN > 0 && LIVE == BM), "narrower row tiles: whole ones, in chains");
+    static_assert(BM == kDmaBM || (LIVE == BM && (CHAIN > 0 || EPI == Epi::UpSplit)), "narrower row tiles: whole ones, in chains or split products");
     constexpr bool FOLD = CHAIN > 0;
     static_assert(!FOLD || EPI != Epi::Down || CHAIN == static_cast<int>(kKtPerActBlock), "a down chain has one power of two per row");
     static_assert(LIVE == BM || LIVE == 128 || LIVE == 64, "live rows: the whole tile, its first half or first quarter");
@@ -859,7 +860,7 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
     const uint32_t wm = wave / kWavesN, wn = wave % kWavesN;
     // wave-uniform: this wave's rows hold tokens (a constant for a full tile)
     const bool live = LIVE == BM || wm * kWaveRows < static_cast<uint32_t>(LIVE);
-    const uint32_t tiles_m = (M + BM - 1) / BM, tiles_n = Ncol / BN;
+    const uint32_t tiles_m = BM == kDmaBM ? rows_pad / BM : (M + BM - 1) / BM, tiles_n = Ncol / BN;
     // the first tiles_m * whole_n blocks: column tiles 0 .. whole_n - 1 over all of K (one round of long blocks first);
     // the others: the remaining column tiles, K split `splits` ways (whole_n 0: every tile split alike)
     const uint32_t whole_blocks = tiles_m * whole_n;
@@ -925,7 +926,13 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
     for (int s = 0; s < S; ++s)
         if (static_cast<uint32_t>(s) < steps) issue(k_begin + s, s);
     // stage k_begin has landed (later stages may be in flight), and with it the binades; then the block meets
-    wait_stages<S - 1, kLoads>(steps - 1);
+    if constexpr (S == 3) {
+        if (steps >= 3) wait_loads<2 * kLoads>();
+        else if (steps == 2) wait_loads<kLoads>();
+        else wait_loads<0>();
+    } else {
+        wait_stages<S - 1, kLoads>(steps - 1);
+    }
     block_barrier();
 
     floatx16 acc[MI][NI], sum[FOLD ? MI : 1][FOLD ? NI : 1];
@@ -1084,7 +1091,13 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
         load(f1, slot, 1);
         __builtin_amdgcn_sched_barrier(0);
         multiply(f0);
-        wait_stages<S - 2, kLoads>(k_end - kt - 2);  // stage kt + 1 has landed, the S - 2 after it may be in flight
+        // stage kt + 1 has landed, the S - 2 after it may be in flight
+        if constexpr (S == 3) {
+            if (kt + 2 < k_end) wait_loads<kLoads>();
+            else wait_loads<0>();
+        } else {
+            wait_stages<S - 2, kLoads>(k_end - kt - 2);
+        }
         wait_loads<63>();  // the same LDS wait on every path, where the compiler's wait tracking sees it
         block_barrier();
         load(f0, (it + 1) % S, 0);
@@ -1117,7 +1130,7 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
         for (int j = 0; j < NI; ++j) {
             const uint32_t c = wn * kWaveCols + j * 32 + lane % 32;
             const int ce = b_exp[n0 + c];
-            const float cb = n0 + c < cols ? bias[n0 + c] : 0.0f;  // a padding neuron: gelu(0) = 0
+            const float cb = FOLD && n0 + c >= cols ? 0.0f : bias[n0 + c];  // a padding neuron (chained calls only): gelu(0) = 0
 #pragma unroll
             for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -1192,7 +1205,7 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
         // y (whole k range) or this split's partial: [splits, M, Ncol], or with whole_n > 0 [splits, M, Ncol - whole_n BN]
         // over the split column tiles only
         // (y: the real columns only; partials: the padded ones as well)
-        const bool apart = nsplit > 1 && whole_n > 0, is_y = EPI == Epi::Down && nsplit == 1;
+        const bool apart = nsplit > 1 && whole_n > 0, is_y = FOLD && EPI == Epi::Down && nsplit == 1;  // (padded: chained calls only)
         const uint32_t ld = apart ? Ncol - whole_n * BN : is_y ? cols : Ncol, c0 = n0 - (apart ? whole_n * BN : 0);
         float* target = nsplit == 1 ? out : (whole_n > 0 ? part : out) + static_cast<size_t>(tile.split) * M * ld;
         const uint32_t c_end = is_y ? cols - min(cols, n0) : BN;
@@ -1200,7 +1213,7 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
         for (uint32_t q = tid; q < BM * (BN / 4); q += kT) {
             const uint32_t m = q / (BN / 4), c = (q % (BN / 4)) * 4;
             if (m0 + m >= M) break;  // rows ascend with q
-            if (c >= c_end) continue;
+            if (FOLD && c >= c_end) continue;
             float4 v = *reinterpret_cast<const float4*>(tile_v + m * kLd + c);
             if (add_bias) {
                 const float4 b = *reinterpret_cast<const float4*>(bias + n0 + c);
@@ -1633,7 +1646,7 @@ hipError_t launch_dma(const _Float16* a_planes, const int32_t* a_exp, const _Flo
     return hipGetLastError();
 }
 
-// The chained GEMMs: row tiles of bm (64, 128 or 256) tokens, K split `splits` ways.
+// The chained GEMMs: row tiles of bm (64, 128 or 256) tokens, K split `splits` ways (CHAIN 0: one chain, bm 128).
 template <Epi EPI, bool LO_B, int CHAIN>
 hipError_t launch_chained(uint32_t bm, const _Float16* a_planes, const int32_t* a_exp, const _Float16* b_planes, const int32_t* b_exp,
                           const float* bias, float* out, _Float16* out_planes, int32_t* out_exp, uint32_t M, uint32_t Ncol, uint32_t K,
@@ -1643,7 +1656,8 @@ hipError_t launch_chained(uint32_t bm, const _Float16* a_planes, const int32_t* 
 #define HFFN_CHAINED(BM)                                                                                                          \
     hipLaunchKernelGGL((gemm_dma_kernel<EPI, LO_B, BM, CHAIN, BM>), grid, dim3(64 * kDmaWaves), 0, stream, a_planes, a_exp, b_planes, \
                        b_exp, bias, out, out_planes, out_exp, M, rows_pad, Ncol, K, splits, 0u, static_cast<float*>(nullptr), cols)
-    if (bm == 64) HFFN_CHAINED(64);
+    if constexpr (CHAIN == 0) HFFN_CHAINED(128);
+    else if (bm == 64) HFFN_CHAINED(64);
     else if (bm == 128) HFFN_CHAINED(128);
     else HFFN_CHAINED(256);
 #undef HFFN_CHAINED
@@ -2020,8 +2034,13 @@ hipError_t launch_grad_dense(const float* row, const float* mat, const int32_t* 
     hipLaunchKernelGGL(split_pair_kernel, dim3((rows + cols) / kSplitBlockRows), dim3(kThreads), 0, stream, row, rows, a_planes, a_exp, mat, cols,
                        b_planes, b_exp, l.k_pad, ld, n);
     if (hipError_t status = hipGetLastError(); status != hipSuccess) return status;
-    if (hipError_t status = launch_dma<Epi::UpSplit, true>(a_planes, a_exp, b_planes, b_exp, nullptr, partials, nullptr, nullptr, rows,
-                                                           cols, l.k_pad, l.splits, stream);
+    // row tiles of 128 where 256 leave CUs idle (an output's products and their order are the same): 1024 x 4096 at 2048
+    // tokens, 128 blocks -> 256, 64.5 -> 50.5 us; at 512 tokens 23.3 -> 18.3 us
+    const bool narrow = dma_tiles(rows, cols) * l.splits <= kCus / 2;
+    if (hipError_t status = narrow ? launch_chained<Epi::UpSplit, true, 0>(128, a_planes, a_exp, b_planes, b_exp, nullptr, partials, nullptr,
+                                                                           nullptr, rows, cols, l.k_pad, l.splits, cols, stream)
+                                   : launch_dma<Epi::UpSplit, true>(a_planes, a_exp, b_planes, b_exp, nullptr, partials, nullptr, nullptr,
+                                                                    rows, cols, l.k_pad, l.splits, stream);
         status != hipSuccess)
         return status;
     hipLaunchKernelGGL(gather_dense_kernel, dim3(ceil_div(rows, kThreads / kWave)), dim3(kThreads), 0, stream, partials, l.splits, row,
@@ -2031,23 +2050,45 @@ hipError_t launch_grad_dense(const float* row, const float* mat, const int32_t* 
 
 size_t train_mfma_workspace_bytes(uint32_t n, uint32_t d, uint32_t h) { return workspace_layout(n, d, h, true).bytes; }
 
+namespace {
+// x [n, d] split into planes and transposed, and the two sides densified (up_blocks, down_blocks; 0: neither).
+hipError_t launch_train_prep(const DensSide& up, const DensSide& down, uint32_t up_blocks, uint32_t down_blocks, const float* x, float* x_t,
+                             uint32_t n, uint32_t d, uint32_t ld, _Float16* x_planes, int32_t* x_exp, hipStream_t stream) {
+    const uint32_t split_blocks = rows_live(n) / kSplitBlockRows / kSplitGroups, tiles_c = d / kTransCols;
+    const uint32_t trans_blocks = ceil_div(tiles_c * ceil_div(n, kTransRows), kSplitGroups);
+    hipLaunchKernelGGL(prefill_prep_kernel<float>, dim3(up_blocks + down_blocks + split_blocks + trans_blocks), dim3(kDensThreads), 0, stream, up,
+                       down, up_blocks, split_blocks, trans_blocks, x, n, rows_padded(n), d, d, x_planes, x_exp, x_t, ld, tiles_c,
+                       transpose_vectors(x, x_t, d, ld));
+    return hipGetLastError();
+}
+}  // namespace
+
 // Training forward on the planes (fp32 weights): x split into planes, the up projection as a split product (partials
 // at every split count) whose epilogue (train_planes_kernel<Forward>) writes z, act (hidden-major) and the activation
 // planes, then the inference down GEMM: y. x_t = x transposed for the sampled product of g_up. The workspace is laid
 // out as the MFMA workspace with the training partials (train_mfma_workspace_bytes).
 hipError_t launch_train_forward(const float* x, const void* up_planes, const int32_t* up_exp, const float* b_up, const void* down_planes,
                                 const int32_t* down_exp, const float* b_down, void* workspace, float* x_t, float* act, float* z, float* y,
-                                uint32_t n, uint32_t d, uint32_t h, uint32_t ld, hipStream_t stream) {
+                                uint32_t n, uint32_t d, uint32_t h, uint32_t ld, hipStream_t stream, const TrainSlots* slots) {
     const Workspace w = workspace_layout(n, d, h, true);
     int32_t* words = static_cast<int32_t*>(workspace);
     char* bytes = static_cast<char*>(workspace);
     auto* x_planes = reinterpret_cast<_Float16*>(bytes + w.x_planes);
     auto* act_planes = reinterpret_cast<_Float16*>(bytes + w.act_planes);
     float* partials = reinterpret_cast<float*>(bytes + w.partials);
-    if (hipError_t status = launch_transpose(x, x_t, n, d, d, ld, stream); status != hipSuccess) return status;
-    hipLaunchKernelGGL(split_rows_kernel, dim3(rows_live(n) / kSplitBlockRows), dim3(kThreads), 0, stream, x, n, rows_padded(n), d, d,
-                       d, x_planes, words + w.x_binades);
-    if (hipError_t status = hipGetLastError(); status != hipSuccess) return status;
+    // x split and transposed, and (slots) the planes densified from the values again: one launch
+    const auto planes = [](const void* p) { return static_cast<_Float16*>(const_cast<void*>(p)); };
+    DensSide up{}, down{};
+    if (slots != nullptr) {
+        up = {slots->up_off, slots->up_idx, slots->up_val, nullptr, h, h, d, kNoChains, slots_aligned(slots->up_idx, slots->up_val),
+              planes(up_planes), const_cast<int32_t*>(up_exp)};
+        down = {slots->down_off, slots->down_idx, slots->down_val, nullptr, d, d, h, kNoChains, slots_aligned(slots->down_idx, slots->down_val),
+                planes(down_planes), const_cast<int32_t*>(down_exp)};
+    }
+    const uint32_t up_blocks = slots ? dens_blocks(h, d, 2) : 0, down_blocks = slots ? dens_blocks(d, h, 2) : 0;
+    if (hipError_t status = launch_train_prep(up, down, up_blocks, down_blocks, x, x_t, n, d, ld, x_planes, words + w.x_binades, stream);
+        status != hipSuccess)
+        return status;
     const uint32_t splits = max(1u, dma_up_splits(n, h, d));
     if (hipError_t status = launch_dma<Epi::UpSplit, true>(x_planes, words + w.x_binades, static_cast<const _Float16*>(up_planes), up_exp,
                                                            nullptr, partials, nullptr, nullptr, n, h, d, splits, stream);
@@ -2142,13 +2183,11 @@ hipError_t launch_train_planes_backward(const TrainBackward& c, hipStream_t stre
     };
     if (hipError_t status = values(down_t, c.hid_pos, c.out_val, c.hid_val, c.nnz_down); status != hipSuccess) return status;
     if (hipError_t status = values(up_t, c.in_pos, c.up_val, c.in_val, c.nnz_up); status != hipSuccess) return status;
-    const uint32_t up_blocks = dens_blocks(c.h, c.d, 2), down_blocks = dens_blocks(c.d, c.h, 2), rows = rows_padded(c.n);
-    const uint32_t split_blocks = rows_live(c.n) / kSplitBlockRows / kSplitGroups, tiles_c = c.d / kTransCols;
-    const uint32_t trans_blocks = ceil_div(tiles_c * ceil_div(c.n, kTransRows), kSplitGroups);
-    hipLaunchKernelGGL(prefill_prep_kernel<float>, dim3(up_blocks + down_blocks + split_blocks + trans_blocks), dim3(kDensThreads), 0, stream,
-                       down_t, up_t, up_blocks, split_blocks, trans_blocks, c.gy, c.n, rows, c.d, c.d, halves(l.x_planes), words(l.x_exp),
-                       c.gy_t, c.ld, tiles_c, transpose_vectors(c.gy, c.gy_t, c.d, c.ld));
-    if (hipError_t status = hipGetLastError(); status != hipSuccess) return status;
+    if (hipError_t status = launch_train_prep(down_t, up_t, dens_blocks(c.h, c.d, 2), dens_blocks(c.d, c.h, 2), c.gy, c.gy_t, c.n, c.d, c.ld,
+                                              halves(l.x_planes), words(l.x_exp), stream);
+        status != hipSuccess)
+        return status;
+    const uint32_t rows = rows_padded(c.n);
     float* partials = reinterpret_cast<float*>(w + l.partials);
     const uint32_t splits = max(1u, dma_up_splits(c.n, c.h, c.d));
     if (hipError_t status = launch_dma<Epi::UpSplit, true>(halves(l.x_planes), words(l.x_exp), down_t.planes, down_t.exps, nullptr, partials,

@@ -242,14 +242,6 @@ class HFFNTrainRuntime:
             mode = self._modes["train", n] = "mfma" if self._mfma_possible(n) else "gather"
         return mode
 
-    def _runtime_planes(self, index: int) -> dict:
-        """The runtime's planes of layer ``index``, rebuilt first if an update made them stale."""
-        runtime = self.runtime
-        if index in runtime._stale:
-            runtime._densify(runtime._tensors[index], runtime._planes[index])
-            runtime._stale.discard(index)
-        return runtime._planes[index]
-
     def _tokens_of(self, t: torch.Tensor, name: str) -> int:
         if not (t.dim() == 2 and t.shape[1] == self.d_model and t.dtype == torch.float32 and t.device == self.runtime._y.device
                 and t.is_contiguous()):
@@ -285,13 +277,17 @@ class HFFNTrainRuntime:
         self.reserve(n)
         x_t, act, y_t, y = runtime._work
         if self.train_mode(n) == "mfma":
-            planes, tensors, x = self._runtime_planes(index), runtime._tensors[index], _aligned(x)
-            _lib.check(self._lib.hffn_forward_mfma_z(x.data_ptr(), planes["up"].data_ptr(), planes["up_binades"].data_ptr(),
-                                                     tensors["b_up"].data_ptr(), planes["down"].data_ptr(),
-                                                     planes["down_binades"].data_ptr(), tensors["b_down"].data_ptr(),
-                                                     self._mfma_work.data_ptr(), self._mfma_work.numel(), x_t, act, z.data_ptr(),
-                                                     y, self.d_model, self.d_ff, n, ld, _stream(runtime.device)),
-                       "forward with z (mfma)")
+            planes, tensors, x = runtime._planes[index], runtime._tensors[index], _aligned(x)
+            held = [planes[name].data_ptr() for name in ("up", "up_binades", "down", "down_binades")]
+            work = (self._mfma_work.data_ptr(), self._mfma_work.numel(), x_t, act, z.data_ptr(), y, self.d_model, self.d_ff, n, ld,
+                    _stream(runtime.device))
+            if index in runtime._stale:  # an update made the planes stale: rebuilt in the forward's first launch
+                _, *model = runtime._args[index]
+                _lib.check(self._lib.hffn_forward_mfma_z_refresh(x.data_ptr(), *model, *held, *work), "forward with z (mfma)")
+                runtime._stale.discard(index)
+            else:
+                b_up, b_down = tensors["b_up"].data_ptr(), tensors["b_down"].data_ptr()
+                _lib.check(self._lib.hffn_forward_mfma_z(x.data_ptr(), *held[:2], b_up, *held[2:], b_down, *work), "forward with z (mfma)")
             self.calls["mfma", "mfma"] += 1
         else:
             up, down = self.modes(n)

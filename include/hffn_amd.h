@@ -329,6 +329,14 @@ int hffn_backward_mfma(const float* gy, const float* z, const void* down_t_plane
                        const int32_t* up_t_binades, void* workspace, uint64_t workspace_bytes, float* gz, float* gx, uint32_t d_model,
                        uint32_t d_ff, uint32_t n, uint32_t ld, void* stream);
 
+/* hffn_forward_mfma_z after the planes are densified again from the compact rows (hffn_densify of both sides, the same
+ * planes), in the launch that splits x. */
+int hffn_forward_mfma_z_refresh(const float* x, const int32_t* up_offsets, const int16_t* up_idx, const float* up_val, const float* b_up,
+                                const int32_t* out_offsets, const int16_t* out_hidden, const float* out_val, const float* b_down,
+                                void* up_planes, int32_t* up_binades, void* down_planes, int32_t* down_binades, void* workspace,
+                                uint64_t workspace_bytes, float* x_t, float* act, float* z, float* y, uint32_t d_model, uint32_t d_ff,
+                                uint32_t n, uint32_t ld, void* stream);
+
 /* hffn_backward_mfma with its planes densified for the call, the same bits; it also writes gy_t (gy transposed, [d_model,
  * ld]). The planes come from the transposed supports, whose slot s holds out_val[hid_pos[s]] or up_val[in_pos[s]]
  * (hid_val and in_val: buffers of nnz_down and nnz_up floats for them). The workspace (hffn_train_planes_workspace bytes,
