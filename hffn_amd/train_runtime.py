@@ -40,6 +40,7 @@ from . import _lib
 from .runtime import MAX_TOKENS, PAIR_MODES, HFFNRuntime, _aligned, down_mode, edges_supported, leading_dim, mfma_streamed, up_mode
 
 PARAMETERS = ("up_val", "b_up", "out_val", "b_down")
+_POINTERS, _COUNTS = ctypes.c_void_p * len(PARAMETERS), ctypes.c_uint32 * len(PARAMETERS)
 SUPPORTS = ("in_offsets", "in_pos", "in_hidden", "hid_offsets", "hid_pos", "hid_output")
 GRAD_TILE = 256              # tokens per tile of the gather sampled products
 PARTIAL_MAX_TOKENS = 2048    # tokens the tile partials are sized for at construction
@@ -86,7 +87,6 @@ class _LayerState:
     supports: dict
     values: dict          # in_val, hid_val: the compact values in the transposed orders
     columns: tuple        # g_down [0, c1), gb_down [c1, c2), g_up [c2, c3), gb_up [c3, width) of the partials
-    adamw: tuple          # hffn_adamw_arrays' arrays: values, gradients, first and second moments, counts
 
 
 class HFFNTrainRuntime:
@@ -134,13 +134,9 @@ class HFFNTrainRuntime:
         c3 = c2 + arrays["up_val"].numel()
         grads = {name: torch.zeros_like(arrays[name]) for name in PARAMETERS}
         moments = {name: (torch.zeros_like(arrays[name]), torch.zeros_like(arrays[name])) for name in PARAMETERS}
-        pointers = ctypes.c_void_p * len(PARAMETERS)
-        of = lambda tensors: pointers(*(tensors(name).data_ptr() for name in PARAMETERS))  # noqa: E731
-        adamw = (of(arrays.__getitem__), of(grads.__getitem__), of(lambda name: moments[name][0]), of(lambda name: moments[name][1]),
-                 (ctypes.c_uint32 * len(PARAMETERS))(*(arrays[name].numel() for name in PARAMETERS)))
         return _LayerState(grads=grads, moments=moments, supports=supports,
                            values={"in_val": torch.empty_like(arrays["up_val"]), "hid_val": torch.empty_like(arrays["out_val"])},
-                           columns=(c1, c2, c3, c3 + self.d_ff), adamw=adamw)
+                           columns=(c1, c2, c3, c3 + self.d_ff))
 
     # -- buffers ---------------------------------------------------------------------------------------------------
     def reserve(self, n: int) -> None:
@@ -374,9 +370,13 @@ class HFFNTrainRuntime:
         beta1, beta2 = self.betas
         scalars = (self.lr * self.weight_decay, beta1, 1.0 - beta1, beta2, 1.0 - beta2, self.lr / (1.0 - beta1 ** k),
                    math.sqrt(1.0 - beta2 ** k), self.eps)
-        values, grads, first, second, counts = self._layers[index].adamw
-        _lib.check(self._lib.hffn_adamw_arrays(len(PARAMETERS), values, grads, first, second, counts, *scalars, _stream(self.runtime.device)),
-                   "AdamW")
+        arrays, state = self.runtime._tensors[index], self._layers[index]
+        # Addresses of this call: gradients() and moments() hand out the dictionaries, whose tensors a caller may replace.
+        values, pairs = [arrays[name] for name in PARAMETERS], [state.moments[name] for name in PARAMETERS]
+        pointers = [_POINTERS(*(t.data_ptr() for t in tensors)) for tensors in
+                    (values, [state.grads[name] for name in PARAMETERS], [first for first, _ in pairs], [second for _, second in pairs])]
+        _lib.check(self._lib.hffn_adamw_arrays(len(PARAMETERS), *pointers, _COUNTS(*(t.numel() for t in values)), *scalars,
+                                               _stream(self.runtime.device)), "AdamW")
         self.runtime.invalidate_planes(index)
 
     def step(self, index: int, x: torch.Tensor, gy: torch.Tensor) -> torch.Tensor:
