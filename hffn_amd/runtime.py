@@ -86,9 +86,9 @@ ROWS_CALL_US, ROWS_SLOT_US = 30.0, 0.148e-6
 # 2560 x 10240, 10-30 % density, both value types) at 65-3000 tokens, each within 15 %. Against it the lane-per-token
 # kernels are priced at ROWS_SHARE of rows_us (which the same layers' timings stay below by about that), and at least at
 # their walk: ROWS_WALK_US plus ROWS_WALK_SLOT_US per slot of the longest row of either side (one wave walks a row).
-# Measured, µs (compact store's kernels, planes of the call): 512 x 2048 at 20 % float32, 128 tokens: 36.6, 30.3; 768 x
-# 3072 at 10 %, 128 and 512 tokens: 34.8, 39.9 and 55.8, 48.4; 1024 x 4096 at 10 % with outputs of up to 4096 slots, 128
-# tokens: 186, 46; 2048 x 8192 at 20 % bfloat16, 128 and 1999 tokens: 98, 80 and 1415, 318.
+# Measured, µs (compact store's kernels, planes of the call): 512 x 2048 at 20 % float32, 128 tokens: 35.8, 26.6; 768 x
+# 3072 at 10 %, 512 tokens: 51.5, 39.8; 1024 x 4096 at 10 % with outputs of up to 4096 slots, 128
+# tokens: 186, 46; 2048 x 8192 at 20 % bfloat16, 128 and 1999 tokens: 98, 80 and 1416, 304.
 PREFILL_CALL_US, PREFILL_PLANE_US, PREFILL_MAC_US, PREFILL_ROW_US = 22.5, 2.5e-6, 3.05e-9, 1.45e-6
 ROWS_SHARE, ROWS_WALK_US, ROWS_WALK_SLOT_US = 0.9, 10.0, 0.045
 MAX_TOKENS = 1 << 18      # runtime/gpu/nvidia/common/kernels/hffn_cuda/runtime.py:26
