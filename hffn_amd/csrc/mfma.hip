@@ -34,6 +34,8 @@
 // those tiles share). A down projection with very few output tiles splits K over 2 blocks per tile; the block that
 // finishes a tile last (an integer counter per tile) adds the partials in split order, so the result does not depend
 // on which block ends first.
+#include <type_traits>
+
 #include "common.hpp"
 #include "launch.hpp"
 
@@ -120,10 +122,12 @@ __device__ __forceinline__ size_t plane_at(uint32_t rows, uint32_t row, uint32_t
 constexpr uint32_t kSplitBlockRows = 8;
 constexpr uint32_t kSplitChunk = 256;  // k per chunk: 4 steps of 64
 constexpr uint32_t kSplitWaves = kThreads / kWave;
+constexpr uint32_t kTinyRow = static_cast<uint32_t>(127 - kBinadeClamp) << 23;  // bits of 2^-kBinadeClamp
 // The work of kThreads threads (tid) on row group `group`; part: their maxima in LDS. Every thread of the block calls it.
 __device__ __forceinline__ void split_rows(uint32_t (&part)[kSplitWaves][kSplitBlockRows], uint32_t tid, uint32_t group,
                                            const float* __restrict__ x, uint32_t M, uint32_t rows_pad, uint32_t K, uint32_t ld,
-                                           uint32_t k_real, _Float16* __restrict__ planes, int32_t* __restrict__ e) {
+                                           uint32_t k_real, _Float16* __restrict__ planes, int32_t* __restrict__ e,
+                                           bool mark = false) {
     constexpr uint32_t kWaves = kSplitWaves;
     const uint32_t lane = tid % kWave, wave = uniform(tid / kWave);
     const uint32_t r = lane % kSplitBlockRows, piece = lane / kSplitBlockRows;
@@ -174,7 +178,8 @@ __device__ __forceinline__ void split_rows(uint32_t (&part)[kSplitWaves][kSplitB
     for (uint32_t w = 1; w < kWaves; ++w) mx = max(mx, part[w][r]);
     const int be = binade_of_bits(mx);
     if (wave == 0 && piece == 0) e[row] = be;
-    const float scale = ldexpf(1.0f, -be);
+    // mark: a row of only tiny entries, which the planes hold with fewer bits, becomes NaN (irregular_row takes it)
+    const float scale = mark && mx != 0 && mx < kTinyRow ? __uint_as_float(0x7fc00000u) : ldexpf(1.0f, -be);
     for (uint32_t k0 = k_begin; k0 < k_end; k0 += kSplitChunk) {
         if (span > kSplitChunk) load_chunk(k0);  // one chunk: still in registers
 #pragma unroll
@@ -400,7 +405,7 @@ __global__ __launch_bounds__(kDensThreads, kDensOccupancy) void prefill_prep_ker
     uint32_t block = blockIdx.x;
     if (block < split_blocks) {
         using Parts = uint32_t[kSplitGroups][kSplitWaves][kSplitBlockRows];
-        split_rows(reinterpret_cast<Parts&>(lds)[g], threadIdx.x % kThreads, block * kSplitGroups + g, x, M, rows_pad, K, ld, ld, planes, e);
+        split_rows(reinterpret_cast<Parts&>(lds)[g], threadIdx.x % kThreads, block * kSplitGroups + g, x, M, rows_pad, K, ld, ld, planes, e, x_t == nullptr);
         return;
     }
     block -= split_blocks;
@@ -415,6 +420,68 @@ __global__ __launch_bounds__(kDensThreads, kDensOccupancy) void prefill_prep_ker
     block -= trans_blocks;
     if (block < up_blocks) densify<V, kParts>(lds, up, block);
     else densify<V, kParts>(lds, down, block - up_blocks);
+}
+
+// ------------------------------------------------------------------------------------ irregular results
+// What the planes of a call cannot hold is computed again as the lane-per-token kernels compute it: from the float32
+// operands in stored slot order, the same bits. A token's planes turn an infinity, a NaN, a magnitude beyond fp16's range
+// past the clamp of its power of two (2^104) and (mark above) a row of only tiny entries into NaN, and the zeros of the
+// dense planes carry that to every output of the token; a weight beyond the clamp does so to its output or, through its
+// neuron's activation, to the token's every output. So the kernel that writes y sees it: an output that is not finite. Its
+// block (the split reduction: its wave) then walks that token's outputs in its columns. Where every output is finite a
+// call is 0.2 us longer (512 x 2048 at 20 %, 128 tokens: 26.6 -> 26.8 us; 2048 x 8192 at 20 % bfloat16, 1999 tokens: 304.3 ->
+// 306.5); a launch of its own that looked at the tokens cost 2.2 and 5.6 us.
+struct Walk {
+    const float* x;  // [M, d]
+    const int32_t* up_off;
+    const int16_t* up_idx;
+    const void* up_val;
+    const float* b_up;
+    const int32_t* down_off;
+    const int16_t* down_idx;
+    const void* down_val;
+    const float* b_down;
+    uint32_t d, h;
+};
+__device__ __forceinline__ bool finite(float v) { return abs_bits(v) < 0x7f800000u; }
+__device__ __forceinline__ bool finite(const float4& v) { return finite(v.x) && finite(v.y) && finite(v.z) && finite(v.w); }
+// y[row, o] for o in [o0, o_end), at most THREADS of them, by THREADS threads (a block, or a wave): the token's activations
+// CHUNK neurons at a time in `act` (LDS, free for it), thread i the slots of output o0 + i among them (ascending within a
+// row, so the chunks in turn are the stored order). Every one of the threads calls it.
+template <typename V, uint32_t THREADS, uint32_t CHUNK>
+__device__ __forceinline__ void irregular_row(const Walk& a, float* act, uint32_t row, uint32_t o0, uint32_t o_end, float* y) {
+    const auto meet = [] {
+        if constexpr (THREADS == kWave) {  // a wave's LDS accesses keep their order: only the compiler has to
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+            __builtin_amdgcn_wave_barrier();
+        } else {
+            __syncthreads();
+        }
+    };
+    const float* x = a.x + static_cast<size_t>(row) * a.d;
+    const V *up_val = static_cast<const V*>(a.up_val), *down_val = static_cast<const V*>(a.down_val);
+    const uint32_t thread = threadIdx.x % THREADS, o = o0 + thread;
+    const bool mine = o < o_end;
+    int32_t slot = mine ? a.down_off[o] : 0;
+    const int32_t end = mine ? a.down_off[o + 1] : 0;
+    float out = 0.0f;
+    for (uint32_t c0 = 0; c0 < a.h; c0 += CHUNK) {
+        for (uint32_t r = c0 + thread; r < min(c0 + CHUNK, a.h); r += THREADS) {
+            float z = 0.0f;
+            const int32_t last = a.up_off[r + 1];
+#pragma unroll 4
+            for (int32_t s = a.up_off[r]; s < last; ++s) z = fmaf(widen(up_val[s]), x[static_cast<uint16_t>(a.up_idx[s])], z);
+            act[r - c0] = gelu(a.b_up[r] + z);
+        }
+        meet();
+        for (; slot < end; ++slot) {
+            const uint32_t at = static_cast<uint16_t>(a.down_idx[slot]) - c0;
+            if (at >= CHUNK) break;
+            out = fmaf(widen(down_val[slot]), act[at], out);
+        }
+        meet();
+    }
+    if (mine) y[static_cast<size_t>(row) * a.d + o] = out + a.b_down[o];
 }
 
 // ------------------------------------------------------------------------------------------------ GEMM
@@ -820,7 +887,8 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
     uint32_t M, uint32_t rows_pad, uint32_t Ncol, uint32_t K, uint32_t splits,
     uint32_t whole_n,                       // Down: column tiles below whole_n take all of K and write y into `out`
     float* __restrict__ part,               // Down, whole_n > 0: the other column tiles' partials [splits, M, Ncol - whole_n BN]
-    uint32_t cols) {                        // real columns (<= Ncol, a multiple of 4): biases and y end there
+    uint32_t cols,                          // real columns (<= Ncol, a multiple of 4): biases and y end there
+    Walk walk) {                            // Down, chained, one split: what irregular outputs are computed again from
     // 256 rows: 8 waves in 4 x 2, 64 x 64 outputs each (two waves per SIMD)
     constexpr int W = kDmaWaves, MI = BM == kDmaBM ? 2 : 1, NI = BM == 64 ? 1 : 2, BN = kDmaBN, S = dma_stages(BM);
     constexpr uint32_t kT = 64 * W, kWaveRows = 32 * MI, kWaveCols = 32 * NI, kWavesN = BN / kWaveCols;
@@ -1210,6 +1278,8 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
         float* target = nsplit == 1 ? out : (whole_n > 0 ? part : out) + static_cast<size_t>(tile.split) * M * ld;
         const uint32_t c_end = is_y ? cols - min(cols, n0) : BN;
         const bool add_bias = EPI == Epi::Down && nsplit == 1 && bias != nullptr;  // no bias: the training gx product
+        uint32_t irregular = 0;  // bit i: in the thread's pass i (row kPassRows i + tid / (BN / 4))
+        constexpr uint32_t kPassRows = kT / (BN / 4);
         for (uint32_t q = tid; q < BM * (BN / 4); q += kT) {
             const uint32_t m = q / (BN / 4), c = (q % (BN / 4)) * 4;
             if (m0 + m >= M) break;  // rows ascend with q
@@ -1219,19 +1289,24 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
                 const float4 b = *reinterpret_cast<const float4*>(bias + n0 + c);
                 v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w;
             }
+            if constexpr (FOLD && EPI == Epi::Down) irregular |= static_cast<uint32_t>(!finite(v)) << (m / kPassRows);
             *reinterpret_cast<float4*>(target + static_cast<size_t>(m0 + m) * ld + c0 + c) = v;
+        }
+        if constexpr (FOLD && EPI == Epi::Down) {
+            constexpr uint32_t kWalkChunk = 8192;
+            static_assert(BM / kPassRows <= 32 && kWalkChunk * 4 <= S * kStage * 2, "a bit per pass; the walk's activations fit the ring");
+            if (nsplit > 1 || !__syncthreads_or(static_cast<int>(irregular))) return;  // block-uniform
+            for (uint32_t m = 0; m < BM; ++m)
+                if (__syncthreads_or(static_cast<int>(irregular >> (m / kPassRows) & 1u) & static_cast<int>(tid / (BN / 4) == m % kPassRows)))
+                    irregular_row<std::conditional_t<LO_B, float, uint16_t>, kT, kWalkChunk>(walk, tile_v, m0 + m, n0, min(n0 + BN, cols), out);
         }
     }
 }
 
-// y[m, c0 + c] = sum over splits (in split order) of partials[s, m, c] + bias[c0 + c] for the partials' width columns
-// below cols (y rows of cols); 4 columns per thread, kReduceRows rows x 256 columns per block.
-constexpr uint32_t kReduceRows = 4;
-__global__ __launch_bounds__(kThreads) void reduce_splits_kernel(const float* __restrict__ partials, const float* __restrict__ bias,
-                                                                float* __restrict__ y, uint32_t M, uint32_t splits, uint32_t width,
-                                                                uint32_t c0, uint32_t cols) {
-    const uint32_t m = blockIdx.x * kReduceRows + threadIdx.x / 64, quad = blockIdx.y * 64 + threadIdx.x % 64, c = c0 + quad * 4;
-    if (m >= M || quad * 4 >= width || c >= cols) return;
+// One thread's four columns; whether they are finite.
+__device__ __forceinline__ bool reduce_quad(const float* __restrict__ partials, const float* __restrict__ bias, float* __restrict__ y,
+                                            uint32_t M, uint32_t splits, uint32_t width, uint32_t cols, uint32_t m, uint32_t quad,
+                                            uint32_t c) {
     const size_t quads = static_cast<size_t>(M) * (width / 4), i = static_cast<size_t>(m) * (width / 4) + quad;
     const float4* p = reinterpret_cast<const float4*>(partials);
     float4 t = p[i];
@@ -1251,6 +1326,28 @@ __global__ __launch_bounds__(kThreads) void reduce_splits_kernel(const float* __
         t.x += b.x; t.y += b.y; t.z += b.z; t.w += b.w;
     }
     *reinterpret_cast<float4*>(y + static_cast<size_t>(m) * cols + c) = t;
+    return finite(t);
+}
+// y[m, c0 + c] = sum over splits (in split order) of partials[s, m, c] + bias[c0 + c] for the partials' width columns
+// below cols (y rows of cols); 4 columns per thread, kReduceRows rows x 256 columns per block.
+// V: float or uint16_t, the walk's values (irregular_row; the calls whose planes are densified per call), or void: none.
+constexpr uint32_t kReduceRows = 4;
+template <typename V>
+__global__ __launch_bounds__(kThreads) void reduce_splits_kernel(const float* __restrict__ partials, const float* __restrict__ bias,
+                                                                float* __restrict__ y, uint32_t M, uint32_t splits, uint32_t width,
+                                                                uint32_t c0, uint32_t cols, Walk walk) {
+    const uint32_t m = blockIdx.x * kReduceRows + threadIdx.x / 64, quad = blockIdx.y * 64 + threadIdx.x % 64, c = c0 + quad * 4;
+    const bool live = m < M && quad * 4 < width && c < cols;
+    const bool odd = live && !reduce_quad(partials, bias, y, M, splits, width, cols, m, quad, c);
+    if constexpr (!std::is_void_v<V>) {
+        constexpr uint32_t kChunk = 512;
+        __shared__ float act[kReduceRows][kChunk];
+        static_assert(kReduceRows * kWave == kThreads, "a wave per row");
+        if (__builtin_amdgcn_ballot_w64(odd) == 0) return;
+        const uint32_t o_end = min(c0 + blockIdx.y * 256 + 256, cols);
+        for (uint32_t o = c0 + blockIdx.y * 256; o < o_end; o += kWave)
+            irregular_row<V, kWave, kChunk>(walk, act[threadIdx.x / kWave], m, o, min(o + kWave, o_end), y);
+    }
 }
 
 // Activation planes from the up GEMM's k-split partial sums (Epi::UpSplit): v = gelu(sum over the splits, in split
@@ -1636,13 +1733,13 @@ hipError_t launch_dma(const _Float16* a_planes, const int32_t* a_exp, const _Flo
     const uint32_t rows_pad = rows_padded(M), live = rows_live(M);
     if (live == 64)
         hipLaunchKernelGGL((gemm_dma_kernel<EPI, LO_B, 64, 0>), grid, block, 0, stream, a_planes, a_exp, b_planes, b_exp, bias, out,
-                           out_planes, out_exp, M, rows_pad, Ncol, K, splits, whole_n, part, Ncol);
+                           out_planes, out_exp, M, rows_pad, Ncol, K, splits, whole_n, part, Ncol, Walk{});
     else if (live == 128)
         hipLaunchKernelGGL((gemm_dma_kernel<EPI, LO_B, 128, 0>), grid, block, 0, stream, a_planes, a_exp, b_planes, b_exp, bias, out,
-                           out_planes, out_exp, M, rows_pad, Ncol, K, splits, whole_n, part, Ncol);
+                           out_planes, out_exp, M, rows_pad, Ncol, K, splits, whole_n, part, Ncol, Walk{});
     else
         hipLaunchKernelGGL((gemm_dma_kernel<EPI, LO_B, kDmaBM, 0>), grid, block, 0, stream, a_planes, a_exp, b_planes, b_exp, bias, out,
-                           out_planes, out_exp, M, rows_pad, Ncol, K, splits, whole_n, part, Ncol);
+                           out_planes, out_exp, M, rows_pad, Ncol, K, splits, whole_n, part, Ncol, Walk{});
     return hipGetLastError();
 }
 
@@ -1650,12 +1747,12 @@ hipError_t launch_dma(const _Float16* a_planes, const int32_t* a_exp, const _Flo
 template <Epi EPI, bool LO_B, int CHAIN>
 hipError_t launch_chained(uint32_t bm, const _Float16* a_planes, const int32_t* a_exp, const _Float16* b_planes, const int32_t* b_exp,
                           const float* bias, float* out, _Float16* out_planes, int32_t* out_exp, uint32_t M, uint32_t Ncol, uint32_t K,
-                          uint32_t splits, uint32_t cols, hipStream_t stream) {
+                          uint32_t splits, uint32_t cols, hipStream_t stream, const Walk& walk = {}) {
     const dim3 grid(ceil_div(M, bm) * (Ncol / kDmaBN) * splits);
     const uint32_t rows_pad = rows_padded(M);
 #define HFFN_CHAINED(BM)                                                                                                          \
     hipLaunchKernelGGL((gemm_dma_kernel<EPI, LO_B, BM, CHAIN, BM>), grid, dim3(64 * kDmaWaves), 0, stream, a_planes, a_exp, b_planes, \
-                       b_exp, bias, out, out_planes, out_exp, M, rows_pad, Ncol, K, splits, 0u, static_cast<float*>(nullptr), cols)
+                       b_exp, bias, out, out_planes, out_exp, M, rows_pad, Ncol, K, splits, 0u, static_cast<float*>(nullptr), cols, walk)
     if constexpr (CHAIN == 0) HFFN_CHAINED(128);
     else if (bm == 64) HFFN_CHAINED(64);
     else if (bm == 128) HFFN_CHAINED(128);
@@ -1665,10 +1762,11 @@ hipError_t launch_chained(uint32_t bm, const _Float16* a_planes, const int32_t* 
 }
 
 // y = the split partials [splits, M, width] of columns c0 .. c0 + width - 1, added in split order, plus the bias.
+template <typename V = void>
 hipError_t launch_reduce_splits(const float* partials, const float* bias, float* y, uint32_t M, uint32_t splits, uint32_t width, uint32_t c0,
-                                uint32_t cols, hipStream_t stream) {
-    hipLaunchKernelGGL(reduce_splits_kernel, dim3(ceil_div(M, kReduceRows), ceil_div(width, 256)), dim3(kThreads), 0, stream, partials, bias, y,
-                       M, splits, width, c0, cols);
+                                uint32_t cols, hipStream_t stream, const Walk& walk = {}) {
+    hipLaunchKernelGGL(reduce_splits_kernel<V>, dim3(ceil_div(M, kReduceRows), ceil_div(width, 256)), dim3(kThreads), 0, stream, partials, bias, y,
+                       M, splits, width, c0, cols, walk);
     return hipGetLastError();
 }
 
@@ -1980,11 +2078,12 @@ hipError_t prefill(const PrefillCall& c, hipStream_t stream) {
             if (status = hipGetLastError(); status != hipSuccess) return status;
         }
         const bool parts = plan.down.splits > 1;
+        const Walk walk{x, c.up_off, c.up_idx, c.up_val, c.b_up, c.down_off, c.down_idx, c.down_val, c.b_down, c.d, c.h};
         status = launch_chained<Epi::Down, kLoB, kPrefillDownChain>(plan.down.bm, halves(l.act_planes), words(l.act_exp), down.planes,
                                                                     down.exps, c.b_down, parts ? partials : y, nullptr, nullptr, n, l.d, l.h,
-                                                                    plan.down.splits, c.d, stream);
+                                                                    plan.down.splits, c.d, stream, walk);
         if (status == hipSuccess && parts)
-            status = launch_reduce_splits(partials, c.b_down, y, n, plan.down.splits, l.d, 0, c.d, stream);
+            status = launch_reduce_splits<V>(partials, c.b_down, y, n, plan.down.splits, l.d, 0, c.d, stream, walk);
         if (status != hipSuccess) return status;
     }
     return hipSuccess;
