@@ -346,9 +346,8 @@ class HFFNRuntime:
         self._tiles_work = torch.empty(1, device=self.device)
         if self._tiles_eligible():
             self._tiles = [self._tiles_build(tensors) for tensors in self._tensors]
-            value_type = self._args[0][0]
-            words = max(_lib.query_bytes(self._lib.hffn_tiles_workspace, value_type, TILES_MAX_TOKENS, self.d_model, self.d_ff,
-                                         *nnz) for nnz in self._nnz) // 4
+            words = max(_lib.query_bytes(self._lib.hffn_tiles_workspace, args[0], TILES_MAX_TOKENS, self.d_model, self.d_ff,
+                                         *nnz) for args, nnz in zip(self._args, self._nnz)) // 4
             self._tiles_work = torch.empty(words, device=self.device)  # the per-chunk partial sums
         self._gemv_work = torch.empty(1, device=self.device)
         if (dense or (dense is None and self.density >= MFMA_MIN_DENSITY)) and self._mfma_eligible():
@@ -500,7 +499,8 @@ class HFFNRuntime:
         self._transient.clear()
         self._prefill_work = None
         if any(self._prefers_transient(m) for m in {n, *(1 << b for b in range(7, n.bit_length()))}):
-            words = _lib.query_bytes(self._lib.hffn_prefill_workspace, self._args[0][0], n, self.d_model, self.d_ff) // 4
+            words = max(_lib.query_bytes(self._lib.hffn_prefill_workspace, value_type, n, self.d_model, self.d_ff)
+                        for value_type in {args[0] for args in self._args}) // 4  # neither value type's is always the larger
             self._prefill_work = torch.empty(words, dtype=torch.int32, device=self.device)
         self._work = (self._x_t.data_ptr(), self._act.data_ptr(), self._y_t.data_ptr(), self._y.data_ptr())
 

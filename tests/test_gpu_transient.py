@@ -133,6 +133,21 @@ def test_policy_plans_and_capture(device):
     assert not never.transient(n) and never._prefill_work is None
 
 
+@pytest.mark.parametrize("d,h,density,tokens", [(256, 1024, 0.2, 600), (768, 3072, 0.1, 100), (2048, 8192, 0.1, 1100)])
+@pytest.mark.parametrize("first", [False, True], ids=["float32_first", "bf16_first"])
+def test_layers_of_both_value_types(d, h, density, tokens, first, device):
+    """A runtime of a bfloat16 and a float32 layer: the workspaces hold either layer's calls (above and below 64 tokens),
+    whichever comes first."""
+    compact = {bf16: _layer(d, h, density, bf16) for bf16 in (False, True)}
+    order = [first, not first]
+    runtime = HFFNRuntime([_device_layer(compact[bf16], bf16, device) for bf16 in order], device)
+    for n in (tokens, 48):
+        x = np.random.default_rng(n).standard_normal((n, d)).astype(np.float32)
+        for index, bf16 in enumerate(order):
+            expected = reference.forward_dense(compact[bf16], x, reference.dense_weights(compact[bf16]))
+            assert _relative(runtime.forward(index, torch.from_numpy(x).to(device)), expected) <= 1e-6, (n, bf16)
+
+
 def test_prefill_refusals(device):
     lib, size = _lib.load(), ctypes.c_uint64(0)
     p, odd = 256, 264  # never dereferenced: the calls are refused before any launch
