@@ -92,7 +92,7 @@ class PreparedRuntime(HFFNRuntime):
         if not 1 <= n <= MAX_TOKENS:
             raise ValueError("unsupported token count")
         if n > self._tokens:
-            self._reserve(n)
+            self._grow(n)
         key = (index, n)
         entry = self._plans.get(key)
         if entry is None:

@@ -496,13 +496,24 @@ class HFFNRuntime:
             words = (_lib.query_bytes(self._lib.hffn_mfma_workspace, n, self.d_model, self.d_ff) + 3) // 4
         # zero-filled once: the split-K counters it holds start at zero and every call leaves them at zero
         self._mfma_work = torch.zeros(words, dtype=torch.int32, device=self.device)
-        self._transient.clear()
-        self._prefill_work = None
-        if any(self._prefers_transient(m) for m in {n, *(1 << b for b in range(7, n.bit_length()))}):
-            words = max(_lib.query_bytes(self._lib.hffn_prefill_workspace, value_type, n, self.d_model, self.d_ff)
+        self._prefill_work = None  # allocated for calls that run on planes of the call (_grow, _prefill_buffer)
+        self._work = (self._x_t.data_ptr(), self._act.data_ptr(), self._y_t.data_ptr(), self._y.data_ptr())
+
+    def _grow(self, n: int) -> None:
+        """Buffers for calls of up to N tokens, with the prefill workspace where such a call may run on planes of the call:
+        one of the largest counts of every padded row count (the estimate's steps) is asked. The choice of a path never
+        depends on what is allocated: a call that finds no workspace gets it (``_prefill_buffer``)."""
+        self._reserve(n)
+        if any(self._prefers_transient(m) for m in (128, *range(256, n, 256), n) if m <= n):
+            self._prefill_buffer()
+
+    def _prefill_buffer(self) -> torch.Tensor:
+        """The workspace of the calls on planes of the call, of the size for the largest N reserved."""
+        if self._prefill_work is None:
+            words = max(_lib.query_bytes(self._lib.hffn_prefill_workspace, value_type, self._tokens, self.d_model, self.d_ff)
                         for value_type in {args[0] for args in self._args}) // 4  # neither value type's is always the larger
             self._prefill_work = torch.empty(words, dtype=torch.int32, device=self.device)
-        self._work = (self._x_t.data_ptr(), self._act.data_ptr(), self._y_t.data_ptr(), self._y.data_ptr())
+        return self._prefill_work
 
     def workspace_bytes(self) -> int:
         return 4 * (self._x_t.numel() + self._act.numel() + self._y_t.numel() + self._y.numel() + self._mfma_work.numel() +
@@ -559,13 +570,14 @@ class HFFNRuntime:
     def transient(self, n: int) -> bool:
         """Whether a call of N tokens runs on planes densified for the call (``hffn_forward_prefill``) in place of the
         compact store's path that ``modes`` names: unforced calls above 64 tokens of layers without resident planes
-        (``dense=False`` excludes them as well), where that is estimated faster. The planes live in the runtime's
-        workspace, one layer's at a time; ``calls`` counts the call under the path that ``modes`` names."""
+        (``dense=False`` excludes them as well), where that is estimated faster. It depends on N and the layers only, not
+        on the calls before. The planes live in the runtime's workspace, one layer's at a time; ``calls`` counts the call
+        under the path that ``modes`` names."""
         if self.forced_up is not None or self.forced_down is not None:
             return False
         chosen = self._transient.get(n)
         if chosen is None:
-            chosen = self._transient[n] = n <= self._tokens and self._prefill_work is not None and self._prefers_transient(n)
+            chosen = self._transient[n] = self._prefers_transient(n)
         return chosen
 
     def forward(self, index: int, x: torch.Tensor) -> torch.Tensor:
@@ -579,7 +591,7 @@ class HFFNRuntime:
         if not 1 <= n <= MAX_TOKENS:
             raise ValueError("unsupported token count")
         if n > self._tokens:
-            self._reserve(n)
+            self._grow(n)
         up, down = self.modes(n)
         self._launch(index, x, n, up, down)
         self.calls[up, down] += 1
@@ -614,9 +626,9 @@ class HFFNRuntime:
         x_t, act, y_t, y = self._work
         stream = torch.cuda.current_stream(self.device).cuda_stream
         if n > TILES_MAX_TOKENS and self.transient(n):
-            x = _aligned(x)  # read 16 bytes at a time
-            _lib.check(self._lib.hffn_forward_prefill(value_type, x.data_ptr(), *model, self._prefill_work.data_ptr(),
-                                                      4 * self._prefill_work.numel(), y, self.d_model, self.d_ff, n, stream),
+            x, work = _aligned(x), self._prefill_buffer()  # x is read 16 bytes at a time
+            _lib.check(self._lib.hffn_forward_prefill(value_type, x.data_ptr(), *model, work.data_ptr(), 4 * work.numel(), y,
+                                                      self.d_model, self.d_ff, n, stream),
                        f"forward ({up}, {down}) on planes of the call")
             return
         if up == "tiles":

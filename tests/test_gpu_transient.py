@@ -18,6 +18,7 @@ from hffn_amd import _lib, synth
 from hffn_amd.ffn import hip_layer
 from hffn_amd.prepared_runtime import PreparedRuntime
 from hffn_amd.runtime import HFFNLayer, HFFNRuntime
+from hffn_amd.train_runtime import HFFNTrainRuntime
 from oracle import reference
 
 pytestmark = pytest.mark.gpu
@@ -146,6 +147,34 @@ def test_layers_of_both_value_types(d, h, density, tokens, first, device):
         for index, bf16 in enumerate(order):
             expected = reference.forward_dense(compact[bf16], x, reference.dense_weights(compact[bf16]))
             assert _relative(runtime.forward(index, torch.from_numpy(x).to(device)), expected) <= 1e-6, (n, bf16)
+
+
+def _even_layer(d, h, slots):
+    rng = np.random.default_rng([slots, d, h])
+    offsets = np.arange(0, (h + 1) * slots, slots, dtype=np.int32)
+    sides = [(offsets, np.concatenate([np.sort(rng.choice(d, slots, replace=False)) for _ in range(h)]).astype(np.int16),
+              (rng.standard_normal(h * slots) * 0.02).astype(np.float32)) for _ in range(2)]
+    b_up, b_down = ((rng.standard_normal(k) * 0.01).astype(np.float32) for k in (h, d))
+    return synth.CompactLayer(d, h, synth._groups(h), *sides[0], b_up, *sides[1], b_down)
+
+
+def test_results_do_not_depend_on_earlier_calls(device):
+    """The same input gives the same bits whatever larger call came before (counts on either side of a step of the
+    estimates), with HFFNRuntime and PreparedRuntime; a training runtime holds no prefill workspace until a call needs it."""
+    layer = hip_layer(_even_layer(512, 2048, 26))
+    policy = HFFNRuntime([layer], device)
+    below = next(n for n in range(700, 2100) if policy.transient(n) and not policy.transient(n + 1))
+    counts = (100, below, below + 1)
+    inputs = {n: torch.from_numpy(np.random.default_rng(n).standard_normal((n, 512)).astype(np.float32)).to(device) for n in counts}
+    alone = {n: HFFNRuntime([layer], device).forward(0, inputs[n]).clone() for n in counts}
+    for kind in (HFFNRuntime, PreparedRuntime):
+        runtime = kind([layer], device)
+        for n in (*counts, below, 100):
+            assert torch.equal(runtime.forward(0, inputs[n]), alone[n]), (kind, n)
+    runtime = HFFNRuntime([layer], device)
+    HFFNTrainRuntime(runtime, max_tokens=below).reserve(below)
+    assert runtime._prefill_work is None
+    assert torch.equal(runtime.forward(0, inputs[below]), alone[below]) and runtime._prefill_work is not None
 
 
 def test_prefill_refusals(device):
