@@ -116,7 +116,7 @@ def time_kernels(runtime, x: torch.Tensor, steps: int, copies: int) -> dict:
     lib = _lib.load()
     n = x.shape[0]
     ld = leading_dim(n)
-    up, down = runtime.modes(n)
+    up, down = runtime.path(n)
     x_t, act, y_t, y = runtime._work
     stream = torch.cuda.current_stream().cuda_stream
     recorded = []  # the steps run back to back; the events are read after the last one
@@ -142,7 +142,7 @@ def time_kernels(runtime, x: torch.Tensor, steps: int, copies: int) -> dict:
             events[3].record()
             recorded.append(events)
         return _kernel_seconds(recorded, names, steps)
-    if up in ("gemv", "tiles"):  # both projections in one ABI call, timed as one
+    if up in ("gemv", "tiles", "prefill"):  # both projections in one ABI call, timed as one
         work, work_bytes = runtime._gemv_work.data_ptr(), 4 * runtime._gemv_work.numel()
         for step in range(steps):
             index = step % copies
@@ -151,6 +151,8 @@ def time_kernels(runtime, x: torch.Tensor, steps: int, copies: int) -> dict:
             events[0].record()
             if up == "tiles":
                 runtime._tiles_forward(index, x, n, stream)
+            elif up == "prefill":
+                runtime._launch(index, x, n, up, down)
             else:
                 planes, tensors = runtime._planes[index], runtime._tensors[index]
                 _lib.check(lib.hffn_forward_gemv(value_type, x.data_ptr(), planes["up"].data_ptr(), planes["up_binades"].data_ptr(),
@@ -265,7 +267,7 @@ def decode_entry(runtime, workload, compact, n: int, copies: int, rotations: int
     x = torch.from_numpy(synth.make_input(workload, n)).to(device)
     us = call_us(runtime, x, copies, rotations)
     moved = layer_costs(compact, n)["step_bytes"]  # the compact store, x read, y written
-    entry = {"tokens": n, "modes": list(runtime.modes(n)), "us_per_call": round(us, 2), "tokens_per_s": round(n / us * 1e6, 1),
+    entry = {"tokens": n, "modes": list(runtime.path(n)), "us_per_call": round(us, 2), "tokens_per_s": round(n / us * 1e6, 1),
              "hbm_fraction": round(moved / (us * 1e-6) / HBM_PEAK, 4)}
     if floor:  # the call's time against a plain read of its stores in two launches
         entry["of_read_floor"] = round(floor["two_launches_us"] / us, 3)
@@ -403,21 +405,21 @@ def main() -> int:
     torch.cuda.synchronize()
     wall = time.perf_counter() - wall
     seconds = start.elapsed_time(end) * 1e-3
-    up, down = runtime.modes(n)
+    up, down = runtime.path(n)
 
     kernels = time_kernels(runtime, x, max(20, min(args.steps, 200)), copies)
     decode = None if args.no_decode else decode_record(runtime, base, device, args.decode_rotations, 50)
-    dominant = max((k for k in kernels if k in ("up", "down", "gemv", "tiles")), key=kernels.get)
-    cost = costs["gemv" if dominant == "tiles" else dominant]
+    dominant = max((k for k in kernels if k in ("up", "down", "gemv", "tiles", "prefill")), key=kernels.get)
+    cost = costs["gemv" if dominant in ("tiles", "prefill") else dominant]
     seconds_kernel = kernels[dominant]
     density = {"up": costs["density_up"], "down": costs["density_down"]}.get(dominant, costs["density"])
-    if up == "mfma" and dominant in ("up", "down"):
+    if up == "mfma" and dominant in ("up", "down") or dominant == "prefill":
         # The tile-densified MFMA path: its useful flops against the dense fp16 MFMA peak scaled by the useful/dense
         # flop ratio of the side (its support density); beside it, the same flops against the fp32 peak, and what the
         # MFMA units issue (the dense products of the planes: 3 fp16 MFMAs per product for fp32 values, 2 for bf16).
         achieved = cost["flops"] / seconds_kernel
         peak = FP16_MFMA_PEAK * density
-        products = 2 if base.value_dtype == "bf16" else 3
+        products = (2 if base.value_dtype == "bf16" else 3) * (2 if dominant == "prefill" else 1)  # both sides in one call
         roofline = {"bound": "mfma", "achieved": round(achieved / 1e12, 3), "peak": round(peak / 1e12, 1), "unit": "TFLOP/s",
                     "frac": round(achieved / peak, 4),
                     "peak_rule": "dense fp16 MFMA 2.5 PFLOP/s x useful/dense flops (the side's support density)",
@@ -437,7 +439,7 @@ def main() -> int:
             planes = held + costs["step_bytes"] - costs["model_bytes"]
             roofline["planes_bytes"] = int(planes)
             roofline["frac_on_planes_bytes"] = round(planes / seconds_kernel / HBM_PEAK, 4)
-    names = {"gemv": "up+down (gemv)", "tiles": "up+down (tiles)"}
+    names = {"gemv": "up+down (gemv)", "tiles": "up+down (tiles)", "prefill": "densify+up+down (prefill)"}
     roofline["kernel"] = names.get(dominant, f"{dominant} ({up if dominant == 'up' else down})")
     roofline["traffic"] = measured_traffic(workload.name, n, roofline["kernel"])
     roofline["traffic_source"] = ("rocprofv3 FETCH_SIZE + WRITE_SIZE of this command, per launch, scaled by the copy-kernel "

@@ -89,7 +89,7 @@ def measure(runtime: PreparedRuntime, compacts: list[synth.CompactLayer], batch:
         bitwise &= all(torch.equal(a, b) for a, b in zip(eager, replayed))
     graph_us = timed(graph.replay)
     step_bytes = sum(compact_bytes(layer) for layer in compacts)
-    return {"batch": batch, "layers": layers, "modes": list(runtime.modes(batch)),
+    return {"batch": batch, "layers": layers, "modes": list(runtime.path(batch)),
             "calls_us_per_step": round(calls_us, 1), "calls_graph_us_per_step": round(calls_graph_us, 1),
             "calls_us_per_layer": round(calls_us / layers, 2), "ffn_bytes_per_step": step_bytes,
             "hbm_fraction": round(step_bytes / (min(calls_us, calls_graph_us) * 1e-6) / HBM_PEAK, 4),

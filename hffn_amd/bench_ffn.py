@@ -101,7 +101,7 @@ class LayerCell:
             "dense": lambda p=dense[0]: F.linear(F.gelu(F.linear(x, p[0], p[1]), approximate="none"), p[2], p[3]),
             "dense_copy": lambda p=dense[1]: F.linear(F.gelu(F.linear(x, p[0], p[1]), approximate="none"), p[2], p[3]),
         }
-        self.record = {"layer": name, "n": n, "modes": list(self.runtimes[0].modes(n)),
+        self.record = {"layer": name, "n": n, "modes": list(self.runtimes[0].path(n)),
                        "model_bytes": self.runtimes[0].layers[0].model_bytes(),
                        "workspace_bytes": self.runtimes[0].workspace_bytes(),
                        "dense_weight_bytes": 4 * 2 * layer.d_model * layer.d_ff}

@@ -55,9 +55,7 @@ class PreparedRuntime(HFFNRuntime):
 
     def _plan(self, index: int, n: int):
         """(handle, up, down) for a gather-mode or decode-GEMV call, or False for a call that takes the control's path."""
-        up, down = self.modes(n)
-        if self.transient(n):
-            return False  # planes densified for the call: the control's launch
+        up, down = self.path(n)  # (planes of the call: no plan, the control's launch)
         value_type, *model = self._args[index]
         x_t, act, y_t, y = self._work
         handle = ctypes.c_uint64(0)

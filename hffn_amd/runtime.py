@@ -13,7 +13,7 @@ Kernel shapes (the build's own policy, ``up_mode``/``down_mode``):
   rows through a table of row bounds (default) or from a tiled copy (``tiled=True``: the compact slots regrouped at
   load by 16-row tile and 512-wide sub-chunk of K, interleaved 16-bit fields), densified per block in LDS and
   multiplied on 16x16x32 MFMAs.
-* planes of the call (``transient``) - both sides densified into the workspace, then split-fp16 MFMA GEMMs in short
+* ``prefill`` - planes of the call (``transient``): both sides densified into the workspace, then split-fp16 MFMA GEMMs in short
   chains; N > 64 on layers without resident planes, where estimated faster than the two compact-store paths above 64.
 * ``rows``  - lanes over tokens (1, 2 or 4 per lane), slots walked in order; large N on layers without the MFMA path.
 * ``mfma``  - tile-densified split-fp16 MFMA GEMMs over dense planes (up and down together) on high-density layers
@@ -53,6 +53,7 @@ UP_MODES = ("edges", "rows", "mfma", "gemv", "tiles")
 DOWN_MODES = ("edges", "rows", "mfma", "gemv", "tiles")
 PAIR_MODES = ("mfma", "gemv", "tiles")  # up and down run together (token-major activations of their own)
 PLANES_MODES = ("mfma", "gemv")         # the paths over densified planes
+PREFILL = ("prefill", "prefill")        # planes densified for the call: the policy's only, never forced
 GEMV_MAX_TOKENS = 64      # the planes GEMVs' largest call
 TILES_MAX_TOKENS = 64     # the compact-store MFMA path's largest call
 EDGES_MAX_TOKENS = 32     # the policy's last N for the lane-per-slot shapes
@@ -523,7 +524,8 @@ class HFFNRuntime:
     def modes(self, n: int) -> tuple[str, str]:
         """The (up, down) shapes over the resident stores a call of N tokens takes (forced ones first). The policy's choice
         depends on N and the layers only, so it is worked out once per N (the library queries behind it are ctypes
-        calls). An unforced call above 64 tokens may run on planes densified for the call instead (``transient``)."""
+        calls). An unforced call above 64 tokens may run on planes densified for the call instead: ``path`` says what
+        runs."""
         chosen = self._policy.get(n) if self.forced_up is None and self.forced_down is None else None
         if chosen is None:
             chosen = self._modes(n)
@@ -571,14 +573,18 @@ class HFFNRuntime:
         """Whether a call of N tokens runs on planes densified for the call (``hffn_forward_prefill``) in place of the
         compact store's path that ``modes`` names: unforced calls above 64 tokens of layers without resident planes
         (``dense=False`` excludes them as well), where that is estimated faster. It depends on N and the layers only, not
-        on the calls before. The planes live in the runtime's workspace, one layer's at a time; ``calls`` counts the call
-        under the path that ``modes`` names."""
+        on the calls before. The planes live in the runtime's workspace, one layer's at a time."""
         if self.forced_up is not None or self.forced_down is not None:
             return False
         chosen = self._transient.get(n)
         if chosen is None:
             chosen = self._transient[n] = self._prefers_transient(n)
         return chosen
+
+    def path(self, n: int) -> tuple[str, str]:
+        """The (up, down) kernels a call of N tokens runs, as ``calls`` counts them: ``modes``, or ``prefill`` for both where
+        the call runs on planes of its own (``transient``)."""
+        return PREFILL if n > TILES_MAX_TOKENS and self.transient(n) else self.modes(n)
 
     def forward(self, index: int, x: torch.Tensor) -> torch.Tensor:
         """y[N, d_model] of layer ``index`` for x[N, d_model] (contiguous float32 on the device).
@@ -592,7 +598,7 @@ class HFFNRuntime:
             raise ValueError("unsupported token count")
         if n > self._tokens:
             self._grow(n)
-        up, down = self.modes(n)
+        up, down = self.path(n)
         self._launch(index, x, n, up, down)
         self.calls[up, down] += 1
         return self._y[:n]
@@ -625,11 +631,11 @@ class HFFNRuntime:
         value_type, *model = self._args[index]
         x_t, act, y_t, y = self._work
         stream = torch.cuda.current_stream(self.device).cuda_stream
-        if n > TILES_MAX_TOKENS and self.transient(n):
+        if up == "prefill":
             x, work = _aligned(x), self._prefill_buffer()  # x is read 16 bytes at a time
             _lib.check(self._lib.hffn_forward_prefill(value_type, x.data_ptr(), *model, work.data_ptr(), 4 * work.numel(), y,
                                                       self.d_model, self.d_ff, n, stream),
-                       f"forward ({up}, {down}) on planes of the call")
+                       "forward (prefill, prefill)")
             return
         if up == "tiles":
             x = _aligned(x)  # read 16 bytes at a time

@@ -177,6 +177,36 @@ def test_results_do_not_depend_on_earlier_calls(device):
     assert torch.equal(runtime.forward(0, inputs[below]), alone[below]) and runtime._prefill_work is not None
 
 
+def test_path_and_calls_name_what_runs(device):
+    """``path`` and ``calls`` name the planes of the call where they run, ``modes`` otherwise: the small and the large
+    workload layers, forced pairs, prepared calls."""
+    for name, counts in (("pythia70m_d20", (64, 65, 128, 2048)), ("pythia1p4b_d20_bf16", (64, 65, 300, 2048))):
+        layer = hip_layer(synth.make_workload_layer(name))
+        for kind in (HFFNRuntime, PreparedRuntime):
+            runtime = kind([layer], device)
+            for n in counts:
+                x = torch.randn(n, runtime.d_model, device=device)
+                expected = ("prefill", "prefill") if runtime.transient(n) else runtime.modes(n)
+                runtime.calls.clear()
+                runtime.forward(0, x)
+                assert runtime.path(n) == expected and dict(runtime.calls) == {expected: 1}, (name, n)
+            assert runtime.path(counts[-1]) == ("prefill", "prefill") and runtime.path(64) == ("tiles", "tiles")
+            runtime.force("rows", "rows")
+            runtime.calls.clear()
+            runtime.forward(0, x)
+            assert runtime.path(counts[-1]) == ("rows", "rows") and dict(runtime.calls) == {("rows", "rows"): 1}
+
+
+def test_bench_times_the_path_that_runs(device):
+    """bench.py's kernel record of a call on planes of the call is that call, not the compact store's kernels."""
+    import bench
+    runtime = HFFNRuntime([hip_layer(_layer(400, 1608, 0.3, False))], device)
+    x = torch.randn(300, 400, device=device)
+    runtime.forward(0, x)
+    runtime.calls.clear()
+    assert runtime.transient(300) and list(bench.time_kernels(runtime, x, 3, 1)) == ["prefill"]
+
+
 def test_prefill_refusals(device):
     lib, size = _lib.load(), ctypes.c_uint64(0)
     p, odd = 256, 264  # never dereferenced: the calls are refused before any launch
