@@ -371,8 +371,8 @@ int hffn_grad_hidden(const float* gy, const float* gy_t, const float* z, const i
                      const float* down_val, float* gz, uint32_t d_model, uint32_t d_ff, uint32_t nnz_down, uint32_t n, uint32_t ld,
                      void* stream);
 
-/* gx[t, i] = sum over the input-major up slots of i of in_val * gz[in_hidden, t] (above 8 tokens through gx_t,
- * feature-major). Replaces grad_x (kernels_train.py:201-231). */
+/* gx[t, i] = sum over the input-major up slots of i of in_val * gz[in_hidden, t] (from n d_model =
+ * 3 << 18 entries on through gx_t, feature-major). Replaces grad_x (kernels_train.py:201-231). */
 int hffn_grad_x(const float* gz, const int32_t* in_offsets, const int16_t* in_hidden, const float* in_val, float* gx_t, float* gx,
                 uint32_t d_model, uint32_t d_ff, uint32_t nnz_up, uint32_t n, uint32_t ld, void* stream);
 
