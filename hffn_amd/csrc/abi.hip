@@ -719,8 +719,9 @@ int hffn_grad_dense_workspace(uint32_t rows, uint32_t cols, uint32_t n, uint64_t
     return HFFN_OK;
 }
 
-int hffn_grad_dense(const float* row, const float* mat, const int32_t* offsets, const int16_t* index, float* g, float* gb,
-                    uint32_t rows, uint32_t cols, uint32_t n, uint32_t ld, void* workspace, uint64_t workspace_bytes, void* stream) {
+namespace {
+int grad_dense(const float* row, const float* mat, const int32_t* offsets, const int16_t* index, float* g, float* gb, uint32_t rows,
+               uint32_t cols, uint32_t n, uint32_t ld, void* workspace, uint64_t workspace_bytes, bool narrow, void* stream) {
     uint64_t needed = 0;
     if (int status = hffn_grad_dense_workspace(rows, cols, n, &needed)) return status;
     if (ld < n || ld % 4 != 0) return fail(HFFN_ERROR_ARGUMENT, "grad_dense: ld=%u must be a multiple of 4 and at least n=%u", ld, n);
@@ -731,8 +732,19 @@ int hffn_grad_dense(const float* row, const float* mat, const int32_t* offsets, 
     if (workspace_bytes < needed)
         return fail(HFFN_ERROR_ARGUMENT, "grad_dense: workspace of %llu bytes, %llu needed", static_cast<unsigned long long>(workspace_bytes),
                     static_cast<unsigned long long>(needed));
-    return launched(hffn::launch_grad_dense(row, mat, offsets, index, g, gb, rows, cols, n, ld, workspace, static_cast<hipStream_t>(stream)),
+    return launched(hffn::launch_grad_dense(row, mat, offsets, index, g, gb, rows, cols, n, ld, workspace, narrow, static_cast<hipStream_t>(stream)),
                     "grad_dense");
+}
+}  // namespace
+
+int hffn_grad_dense(const float* row, const float* mat, const int32_t* offsets, const int16_t* index, float* g, float* gb,
+                    uint32_t rows, uint32_t cols, uint32_t n, uint32_t ld, void* workspace, uint64_t workspace_bytes, void* stream) {
+    return grad_dense(row, mat, offsets, index, g, gb, rows, cols, n, ld, workspace, workspace_bytes, false, stream);
+}
+
+int hffn_grad_dense_planes(const float* row, const float* mat, const int32_t* offsets, const int16_t* index, float* g, float* gb,
+                           uint32_t rows, uint32_t cols, uint32_t n, uint32_t ld, void* workspace, uint64_t workspace_bytes, void* stream) {
+    return grad_dense(row, mat, offsets, index, g, gb, rows, cols, n, ld, workspace, workspace_bytes, true, stream);
 }
 
 int hffn_train_mfma_workspace(uint32_t n, uint32_t d_model, uint32_t d_ff, uint64_t* bytes) {

@@ -132,8 +132,9 @@ hipError_t launch_prefill(int vt, const PrefillCall& call, hipStream_t stream);
 // then the support's entries and the bias gradient (A [rows, ld], B [cols, ld] row-major, n real columns).
 // grad_dense_workspace_bytes is 0 for shapes the streamed GEMM does not take.
 size_t grad_dense_workspace_bytes(uint32_t rows, uint32_t cols, uint32_t n);
+// narrow: row tiles of 128 where 256 leave CUs idle.
 hipError_t launch_grad_dense(const float* row, const float* mat, const int32_t* off, const int16_t* idx, float* g, float* gb,
-                             uint32_t rows, uint32_t cols, uint32_t n, uint32_t ld, void* workspace, hipStream_t stream);
+                             uint32_t rows, uint32_t cols, uint32_t n, uint32_t ld, void* workspace, bool narrow, hipStream_t stream);
 
 // The training forward (z, act hidden-major; y) and the backward products gz (hidden-major) and gx on the planes
 // (mfma.hip; fp32 weights): the up-shaped products as split products with the training epilogues, the down-shaped ones

@@ -2122,7 +2122,7 @@ size_t grad_dense_workspace_bytes(uint32_t rows, uint32_t cols, uint32_t n) {
 }
 
 hipError_t launch_grad_dense(const float* row, const float* mat, const int32_t* off, const int16_t* idx, float* g, float* gb,
-                             uint32_t rows, uint32_t cols, uint32_t n, uint32_t ld, void* workspace, hipStream_t stream) {
+                             uint32_t rows, uint32_t cols, uint32_t n, uint32_t ld, void* workspace, bool narrow, hipStream_t stream) {
     const GradDenseLayout l = grad_dense_layout(rows, cols, n);
     char* w = static_cast<char*>(workspace);
     auto* a_planes = reinterpret_cast<_Float16*>(w + l.a_planes);
@@ -2133,9 +2133,12 @@ hipError_t launch_grad_dense(const float* row, const float* mat, const int32_t* 
     hipLaunchKernelGGL(split_pair_kernel, dim3((rows + cols) / kSplitBlockRows), dim3(kThreads), 0, stream, row, rows, a_planes, a_exp, mat, cols,
                        b_planes, b_exp, l.k_pad, ld, n);
     if (hipError_t status = hipGetLastError(); status != hipSuccess) return status;
-    // row tiles of 128 where 256 leave CUs idle (an output's products and their order are the same): 1024 x 4096 at 2048
-    // tokens, 128 blocks -> 256, 64.5 -> 50.5 us; at 512 tokens 23.3 -> 18.3 us
-    const bool narrow = dma_tiles(rows, cols) * l.splits <= kCus / 2;
+    // narrow, in steps whose other products run on planes: row tiles of 128 where 256 leave CUs idle (an output's products and
+    // their order are the same): 1024 x 4096 at 512 tokens, 128 blocks -> 256, 23.3 -> 18.3 us, a step at 50 % 275 -> 266 us; at
+    // 2048 tokens 64.5 -> 50.5 us, the step 556 -> 529. Not beside the lane-per-token gathers: matrix units busy on all 256 CUs
+    // take a card at its power limit to a lower clock, at which the gathers, most of such a step, take 136 us in place of 128:
+    // steps at 10 % 725 -> 751 us (2048 tokens), 227 -> 231 (512), at 30 % 458 -> 483 (512); on a card below its limit 722 -> 695.
+    narrow = narrow && dma_tiles(rows, cols) * l.splits <= kCus / 2;
     if (hipError_t status = narrow ? launch_chained<Epi::UpSplit, true, 0>(128, a_planes, a_exp, b_planes, b_exp, nullptr, partials, nullptr,
                                                                            nullptr, rows, cols, l.k_pad, l.splits, cols, stream)
                                    : launch_dma<Epi::UpSplit, true>(a_planes, a_exp, b_planes, b_exp, nullptr, partials, nullptr, nullptr,

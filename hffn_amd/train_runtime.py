@@ -339,8 +339,9 @@ class HFFNTrainRuntime:
 
         def sampled(row, mat, owner_offsets, owner_index, g, gb, rows, cols, what):
             if dense:
-                _lib.check(lib.hffn_grad_dense(row, mat, owner_offsets, owner_index, g, gb, rows, cols, n, ld,
-                                               self._dense_work.data_ptr(), self._dense_work.numel(), stream), f"{what} (dense)")
+                entry = lib.hffn_grad_dense_planes if planes_mode else lib.hffn_grad_dense
+                _lib.check(entry(row, mat, owner_offsets, owner_index, g, gb, rows, cols, n, ld,
+                                 self._dense_work.data_ptr(), self._dense_work.numel(), stream), f"{what} (dense)")
             else:
                 _lib.check(lib.hffn_grad_sddmm(row, mat, owner_offsets, owner_index, g, gb, rows, n, ld, stride, stream), what)
 

@@ -27,7 +27,7 @@
 extern "C" {
 #endif
 
-#define HFFN_ABI_VERSION 19
+#define HFFN_ABI_VERSION 20
 
 #define HFFN_OK 0
 #define HFFN_ERROR_ARGUMENT (-1) /* invalid shape, mode, pointer or workspace */
@@ -308,8 +308,12 @@ int hffn_forward_z(int up_mode, int down_mode, const float* x, const int32_t* up
  * counterpart (the reference's sampled products are gathers, kernels_train.py:115-184); for high density and many
  * tokens, where a gather reads nnz * n * 4 bytes of activations per product. */
 int hffn_grad_dense_workspace(uint32_t rows, uint32_t cols, uint32_t n, uint64_t* bytes);
+/* hffn_grad_dense_planes: the same bits, on tiles of half the rows where those of 256 leave CUs idle; for a step whose other
+ * products run on planes too. */
 int hffn_grad_dense(const float* row, const float* mat, const int32_t* offsets, const int16_t* index, float* g, float* gb,
                     uint32_t rows, uint32_t cols, uint32_t n, uint32_t ld, void* workspace, uint64_t workspace_bytes, void* stream);
+int hffn_grad_dense_planes(const float* row, const float* mat, const int32_t* offsets, const int16_t* index, float* g, float* gb,
+                           uint32_t rows, uint32_t cols, uint32_t n, uint32_t ld, void* workspace, uint64_t workspace_bytes, void* stream);
 
 /* The training step's dense products on the planes (fp32 values; layers whose planes the runtime holds), for the
  * token counts the streamed GEMM takes (hffn_train_mfma_workspace refuses the others). hffn_forward_mfma_z: the forward

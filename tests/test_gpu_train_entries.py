@@ -1,4 +1,5 @@
-"""The training step's entry points where one path stands in for another: both stores of gx."""
+"""The training step's entry points where one stands in for another: both stores of gx and both tile heights of the dense
+sampled products."""
 from __future__ import annotations
 
 import pytest
@@ -38,3 +39,27 @@ def test_grad_x_on_both_sides_of_its_rule(d, h, n, device):
     expected, size = (dense @ rows).T, (dense.abs() @ rows.abs()).T
     assert bool(((gx[:n].double() - expected).abs() <= slots * 2.0 ** -24 * size + 1e-30).all()) and bool(gx[n].isnan().all())
     assert bool(gx_t.isnan().all()) == (n * d < 3 << 18)
+
+
+@pytest.mark.parametrize("rows,cols,n", [(1024, 4096, 512), (4096, 1024, 515), (1024, 4096, 2048), (512, 2048, 300)])
+def test_dense_sampled_products_on_either_tile_height(rows, cols, n, device):
+    """hffn_grad_dense and hffn_grad_dense_planes: the same bits, and the sampled product within the split operands' error
+    (2^-21 of the sum of the products' magnitudes)."""
+    lib, ld, slots = _lib.load(), leading_dim(n), 40
+    offsets, index, _ = _support(rows, cols, slots, device)
+    drawn = torch.Generator(device=device).manual_seed(2)
+    row, mat = (torch.randn(count * ld, generator=drawn, device=device) for count in (rows, cols))
+    need = _lib.query_bytes(lib.hffn_grad_dense_workspace, rows, cols, n)
+    results = []
+    for entry in (lib.hffn_grad_dense, lib.hffn_grad_dense_planes):
+        work = torch.empty(need, dtype=torch.uint8, device=device)
+        g, gb = torch.full((rows * slots,), float("nan"), device=device), torch.full((rows,), float("nan"), device=device)
+        _lib.check(entry(row.data_ptr(), mat.data_ptr(), offsets.data_ptr(), index.data_ptr(), g.data_ptr(), gb.data_ptr(), rows, cols, n,
+                         ld, work.data_ptr(), need, _stream()), "sampled product")
+        results.append((g, gb))
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+    a, b = row.view(rows, ld)[:, :n].double(), mat.view(cols, ld)[:, :n].double()
+    owner, column = torch.arange(rows, device=device).repeat_interleave(slots), index.long()
+    expected, size = (a @ b.T)[owner, column], (a.abs() @ b.abs().T)[owner, column]
+    assert bool(((results[0][0].double() - expected).abs() <= 2.0 ** -21 * size).all())
+    assert bool(((results[0][1].double() - a.sum(1)).abs() <= n * 2.0 ** -24 * a.abs().sum(1)).all())
