@@ -119,7 +119,7 @@ __global__ __launch_bounds__(kBlock) void reduce_tiles_kernel(const float* __res
 // Compact AdamW in the order of PyTorch's AdamW (kernels_train.py:233-247): decoupled decay, then the moments, then
 // the bias-corrected step; the step-dependent scalars come from the host (float64 there). A thread takes four
 // consecutive entries with 16-byte loads and stores (the first `quads` threads, when all four arrays are 16-byte
-// aligned), one entry otherwise (the rest); the same arithmetic per entry either way.
+// aligned), one entry otherwise (the rest); the same arithmetic per entry, contracted differently (a rounding apart).
 __device__ __forceinline__ void adamw_entry(float& p, float g, float& m, float& v, const AdamScalars& a) {
     p -= a.lr_decay * p;
     m = a.beta1 * m + a.one_minus_beta1 * g;
