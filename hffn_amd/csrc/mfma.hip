@@ -1209,7 +1209,7 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
                 }
         }
         __syncthreads();
-        // H threads per block row (2 with 256 rows, 4 with fewer: lanes h of a row are adjacent), each a BN / H-wide part
+        // H threads per block row (2, 4 or 8 with 256, 128 or 64 rows: lanes h of a row are adjacent), each a BN / H-wide part
         constexpr uint32_t H = kT / BM;
         const uint32_t row = tid / H, part = tid % H;
         const float* row_v = tile_v + row * kLd;

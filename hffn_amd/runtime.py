@@ -15,6 +15,8 @@ Kernel shapes (the build's own policy, ``up_mode``/``down_mode``):
   multiplied on 16x16x32 MFMAs.
 * ``prefill`` - planes of the call (``transient``): both sides densified into the workspace, then split-fp16 MFMA GEMMs in short
   chains; N > 64 on layers without resident planes, where estimated faster than the two compact-store paths above 64.
+  Its k splits follow the 256-token class of N, so a token's bits may differ between counts above 64 (as on ``mfma``;
+  the compact-store paths give a token the same bits at any N).
 * ``rows``  - lanes over tokens (1, 2 or 4 per lane), slots walked in order; large N on layers without the MFMA path.
 * ``mfma``  - tile-densified split-fp16 MFMA GEMMs over dense planes (up and down together) on high-density layers
   (density at least ``MFMA_MIN_DENSITY``, ``d_model`` and ``d_ff`` multiples of 256), above 64 tokens.
@@ -22,11 +24,11 @@ Kernel shapes (the build's own policy, ``up_mode``/``down_mode``):
   large token counts), run when forced.
 
 The policy reads the compact store up to 64 tokens: ``edges`` (up to 32 tokens) or ``tiles``, whichever has the least
-estimated time (``decode_mode``); above 64 tokens the MFMA path where the layer has planes, else ``tiles`` in pieces of
-64 tokens or ``rows``, whichever has the least estimated time (``pieces_us``, ``rows_us``: the tiles path reads the
-store once per piece, the lane-per-token kernels read an input row per slot and token, so the tiles path takes the
-larger layers, e.g. the 1.4B layer at 20 %, 59 against 213 us at 65 tokens and 1.32 against 2.00 ms at 2048, and the
-lane-per-token kernels the smallest, e.g. the 70M layer at 20 % from 65 tokens on, 38.9 against 44.0 us). The dense
+estimated time (``decode_mode``); above 64 tokens the MFMA path where the layer has planes, else ``prefill``, ``tiles``
+in pieces of 64 tokens or ``rows``, whichever has the least estimated time (``prefill_us``, ``pieces_us``, ``rows_us``: the
+tiles path reads the store once per piece, the lane-per-token kernels read an input row per slot and token, planes of the
+call cost the densification whatever N is: 1.4B layer at 20 %: tiles 59, rows 213 us at 65 tokens, prefill 304 against
+1416 us on tiles at 1999; 70M layer at 20 %: prefill 26.8, rows 35.8 us at 128 tokens). ``path`` says which. The dense
 planes (4 bytes per weight for float32 values, 2 for bfloat16) are built only for layers of at least
 ``MFMA_MIN_DENSITY`` unless asked for (``dense=True``). Per call on the Pythia-410M layer at 50 % (12 rotating
 copies, MI355X, HFFNRuntime.forward, forced pairs, compact rows): N = 1: edges 12.9 us, tiles 17.8; N = 4: edges

@@ -105,7 +105,7 @@ class HFFNTrainRuntime:
         self.forced_train: str | None = None   # diagnostic: the forward with z, gz and gx on gathers or planes
         self._mfma_work: torch.Tensor | None = None    # forward on the runtime's planes
         self._planes_work: torch.Tensor | None = None  # the backward's planes and buffers
-        self._modes: dict = {}                  # (what, N, forced) -> mode
+        self._modes: dict = {}                  # (what, N) -> mode
         self._tokens = 0                        # N the dense buffers hold
         self._tiles = 1                         # token tiles the partials hold (none allocated for 1)
         self._partials: torch.Tensor | None = None

@@ -275,7 +275,7 @@ int hffn_plan_tiles_compact(int value_type, const int16_t* up_idx, const void* u
 /* A whole forward above the decode sizes on a layer without planes of its own: both sides' planes are densified from
  * the compact rows into the call's workspace (hffn_prefill_workspace bytes for calls of up to n tokens, any content,
  * 256-byte aligned), and the projections run on them as split-fp16 MFMA products, their float32 sums in chains of 128
- * k. d_model a multiple of 16, d_ff of 8, distinct ascending indices per row; x, y and the biases 16-byte aligned.
+ * k (64 in the float32 up projection). d_model a multiple of 16, d_ff of 8, distinct ascending indices per row; x, y and the biases 16-byte aligned.
  * Widths need not be multiples of 256 (the planes are padded). Calls above 16384 tokens run in pieces of that size
  * over the same planes. Outputs that the planes lose (infinities, NaN, magnitudes of 2^104 and above, tokens whose every
  * entry is below 2^-100) are computed again from the compact rows: hffn_forward's results on the rows kernels. No counterpart (the reference's large-N kernels are gathers, kernels.py:87-191). */

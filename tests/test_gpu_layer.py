@@ -670,10 +670,11 @@ def test_gemv_wide_calls(name, tokens, device):
 
 
 def test_default_policy_reads_the_compact_store(device):
-    """With the default construction, dense planes exist only for layers of at least 50 % density: the 1.4B/20 % bf16
-    layer has none and its calls take the compact-store MFMA path (tiles; above 64 tokens in pieces of 64) at every
-    size; the 70M/20 % layer takes the lane-per-token kernels from 128 tokens on; the 410M/50 % layer keeps its planes
-    for the MFMA path above 64 tokens and takes the compact store below."""
+    """With the default construction, dense planes exist only for layers of at least 50 % density: of the compact store's
+    kernels (``modes``) the 1.4B/20 % bf16 layer takes the MFMA path (tiles; above 64 tokens in pieces of 64) at every
+    size, the 70M/20 % layer the lane-per-token kernels from 128 tokens on; but the calls themselves (``path``) densify
+    planes of their own at 2048 tokens on both and at 128 on the 70M layer. The 410M/50 % layer keeps its planes for the
+    MFMA path above 64 tokens and takes the compact store below."""
     from hffn_amd.runtime import MFMA_MIN_DENSITY
     sparse = HFFNRuntime([hip_layer(_cached("pythia1p4b_d20_bf16"))], device)
     assert sparse.density < MFMA_MIN_DENSITY and sparse.dense_bytes() == 0 and not sparse.mfma_available
@@ -681,7 +682,11 @@ def test_default_policy_reads_the_compact_store(device):
     assert sparse.modes(65) == ("tiles", "tiles") and sparse.modes(2048) == ("tiles", "tiles")
     small = HFFNRuntime([hip_layer(_cached("pythia70m_d20"))], device)
     assert small.modes(128) == ("rows", "rows") and small.modes(2048) == ("rows", "rows")
+    assert sparse.path(64) == ("tiles", "tiles") and sparse.path(65) == ("tiles", "tiles")
+    assert sparse.path(2048) == ("prefill", "prefill")
+    assert small.path(128) == ("prefill", "prefill") and small.path(2048) == ("prefill", "prefill")
     dense = HFFNRuntime([hip_layer(_cached("pythia410m_d50"))], device)
     assert dense.density >= MFMA_MIN_DENSITY and dense.dense_bytes() > 0
     assert dense.modes(16) == ("tiles", "tiles") and dense.modes(2048) == ("mfma", "mfma")
+    assert dense.path(2048) == ("mfma", "mfma") and dense.path(16) == ("tiles", "tiles")
     assert dense.modes(1)[0] == "edges"
