@@ -428,9 +428,9 @@ __global__ __launch_bounds__(kDensThreads, kDensOccupancy) void prefill_prep_ker
 // past the clamp of its power of two (2^104) and (mark above) a row of only tiny entries into NaN, and the zeros of the
 // dense planes carry that to every output of the token; a weight beyond the clamp does so to its output or, through its
 // neuron's activation, to the token's every output. So the kernel that writes y sees it: an output that is not finite. Its
-// block (the split reduction: its wave) then walks that token's outputs in its columns. Where every output is finite a
-// call is 0.2 us longer (512 x 2048 at 20 %, 128 tokens: 26.6 -> 26.8 us; 2048 x 8192 at 20 % bfloat16, 1999 tokens: 304.3 ->
-// 306.5); a launch of its own that looked at the tokens cost 2.2 and 5.6 us.
+// block (the split reduction: its wave) then walks that token's outputs in its columns. Calls whose outputs are finite take
+// the same time as without it (512 x 2048 at 20 %, 128 tokens: 26.6 us; 2048 x 8192 at 20 % bfloat16, 1999 tokens: 304.5);
+// a launch of its own that looked at the tokens cost 2.2 and 5.6 us.
 struct Walk {
     const float* x;  // [M, d]
     const int32_t* up_off;
@@ -874,7 +874,10 @@ __device__ __forceinline__ void wait_stages(uint32_t later) {
 // 512 tokens: up projection 18.2 + 6.4 us in 3 splits of 256 rows and their activation pass, 17.6 us with 64 rows (no
 // split); down 18.7 -> 14.6 us.
 constexpr int dma_stages(int bm) { return bm == 64 ? 6 : bm == 128 ? 4 : kDmaStages; }
-template <Epi EPI, bool LO_B, int LIVE, int CHAIN, int BM = kDmaBM>
+//
+// WALK (a chained down GEMM of one split, which writes y): irregular outputs are walked (irregular_row). An instance of its
+// own: in the one that writes partials the code costs 1-3 us of 127 without being reached.
+template <Epi EPI, bool LO_B, int LIVE, int CHAIN, int BM = kDmaBM, bool WALK = false>
 __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
     const _Float16* __restrict__ a_planes,  // [K / 32][8][rows_pad][8]
     const int32_t* __restrict__ a_exp,      // Up: [rows_pad]; Down: [K / kActBlock, rows_pad] (act_exp_at)
@@ -888,7 +891,7 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
     uint32_t whole_n,                       // Down: column tiles below whole_n take all of K and write y into `out`
     float* __restrict__ part,               // Down, whole_n > 0: the other column tiles' partials [splits, M, Ncol - whole_n BN]
     uint32_t cols,                          // real columns (<= Ncol, a multiple of 4): biases and y end there
-    Walk walk) {                            // Down, chained, one split: what irregular outputs are computed again from
+    Walk walk) {                            // WALK: what irregular outputs are computed again from
     // 256 rows: 8 waves in 4 x 2, 64 x 64 outputs each (two waves per SIMD)
     constexpr int W = kDmaWaves, MI = BM == kDmaBM ? 2 : 1, NI = BM == 64 ? 1 : 2, BN = kDmaBN, S = dma_stages(BM);
     constexpr uint32_t kT = 64 * W, kWaveRows = 32 * MI, kWaveCols = 32 * NI, kWavesN = BN / kWaveCols;
@@ -1289,13 +1292,13 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
                 const float4 b = *reinterpret_cast<const float4*>(bias + n0 + c);
                 v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w;
             }
-            if constexpr (FOLD && EPI == Epi::Down) irregular |= static_cast<uint32_t>(!finite(v)) << (m / kPassRows);
+            if constexpr (WALK) irregular |= static_cast<uint32_t>(!finite(v)) << (m / kPassRows);
             *reinterpret_cast<float4*>(target + static_cast<size_t>(m0 + m) * ld + c0 + c) = v;
         }
-        if constexpr (FOLD && EPI == Epi::Down) {
+        if constexpr (WALK) {
             constexpr uint32_t kWalkChunk = 8192;
-            static_assert(BM / kPassRows <= 32 && kWalkChunk * 4 <= S * kStage * 2, "a bit per pass; the walk's activations fit the ring");
-            if (nsplit > 1 || !__syncthreads_or(static_cast<int>(irregular))) return;  // block-uniform
+            static_assert(FOLD && EPI == Epi::Down && BM / kPassRows <= 32 && kWalkChunk * 4 <= S * kStage * 2, "a bit per pass; the walk's activations fit the ring");
+            if (!__syncthreads_or(static_cast<int>(irregular))) return;  // block-uniform
             for (uint32_t m = 0; m < BM; ++m)
                 if (__syncthreads_or(static_cast<int>(irregular >> (m / kPassRows) & 1u) & static_cast<int>(tid / (BN / 4) == m % kPassRows)))
                     irregular_row<std::conditional_t<LO_B, float, uint16_t>, kT, kWalkChunk>(walk, tile_v, m0 + m, n0, min(n0 + BN, cols), out);
@@ -1743,15 +1746,16 @@ hipError_t launch_dma(const _Float16* a_planes, const int32_t* a_exp, const _Flo
     return hipGetLastError();
 }
 
-// The chained GEMMs: row tiles of bm (64, 128 or 256) tokens, K split `splits` ways (CHAIN 0: one chain, bm 128).
-template <Epi EPI, bool LO_B, int CHAIN>
+// The chained GEMMs: row tiles of bm (64, 128 or 256) tokens, K split `splits` ways (CHAIN 0: one chain, bm 128; WALK: one
+// split).
+template <Epi EPI, bool LO_B, int CHAIN, bool WALK = false>
 hipError_t launch_chained(uint32_t bm, const _Float16* a_planes, const int32_t* a_exp, const _Float16* b_planes, const int32_t* b_exp,
                           const float* bias, float* out, _Float16* out_planes, int32_t* out_exp, uint32_t M, uint32_t Ncol, uint32_t K,
                           uint32_t splits, uint32_t cols, hipStream_t stream, const Walk& walk = {}) {
     const dim3 grid(ceil_div(M, bm) * (Ncol / kDmaBN) * splits);
     const uint32_t rows_pad = rows_padded(M);
 #define HFFN_CHAINED(BM)                                                                                                          \
-    hipLaunchKernelGGL((gemm_dma_kernel<EPI, LO_B, BM, CHAIN, BM>), grid, dim3(64 * kDmaWaves), 0, stream, a_planes, a_exp, b_planes, \
+    hipLaunchKernelGGL((gemm_dma_kernel<EPI, LO_B, BM, CHAIN, BM, WALK>), grid, dim3(64 * kDmaWaves), 0, stream, a_planes, a_exp, b_planes, \
                        b_exp, bias, out, out_planes, out_exp, M, rows_pad, Ncol, K, splits, 0u, static_cast<float*>(nullptr), cols, walk)
     if constexpr (CHAIN == 0) HFFN_CHAINED(128);
     else if (bm == 64) HFFN_CHAINED(64);
@@ -2077,13 +2081,19 @@ hipError_t prefill(const PrefillCall& c, hipStream_t stream) {
                                l.h, c.h);
             if (status = hipGetLastError(); status != hipSuccess) return status;
         }
-        const bool parts = plan.down.splits > 1;
         const Walk walk{x, c.up_off, c.up_idx, c.up_val, c.b_up, c.down_off, c.down_idx, c.down_val, c.b_down, c.d, c.h};
-        status = launch_chained<Epi::Down, kLoB, kPrefillDownChain>(plan.down.bm, halves(l.act_planes), words(l.act_exp), down.planes,
-                                                                    down.exps, c.b_down, parts ? partials : y, nullptr, nullptr, n, l.d, l.h,
-                                                                    plan.down.splits, c.d, stream, walk);
-        if (status == hipSuccess && parts)
-            status = launch_reduce_splits<V>(partials, c.b_down, y, n, plan.down.splits, l.d, 0, c.d, stream, walk);
+        const auto down_gemm = [&](auto walks, float* out) {
+            return launch_chained<Epi::Down, kLoB, kPrefillDownChain, decltype(walks)::value>(
+                plan.down.bm, halves(l.act_planes), words(l.act_exp), down.planes, down.exps, c.b_down, out, nullptr, nullptr, n, l.d, l.h,
+                plan.down.splits, c.d, stream, walk);
+        };
+        if (plan.down.splits == 1) {
+            status = down_gemm(std::true_type{}, y);
+        } else {
+            status = down_gemm(std::false_type{}, partials);
+            if (status == hipSuccess)
+                status = launch_reduce_splits<V>(partials, c.b_down, y, n, plan.down.splits, l.d, 0, c.d, stream, walk);
+        }
         if (status != hipSuccess) return status;
     }
     return hipSuccess;

@@ -17,13 +17,16 @@ from hffn_amd.runtime import HFFNRuntime
 from oracle import reference
 
 pytestmark = pytest.mark.gpu
-SHAPES = [("pythia70m_d20", 128), ("pythia70m_d20", 300), ("pythia1p4b_d20_bf16", 300)]
+WIDE = {w.name: w for w in (synth.Workload("wide", 2048, 1024, 205, 7), synth.Workload("wide_bf16", 2048, 1024, 205, 7, value_dtype="bf16"))}
+# a split down GEMM and its reduction; one split on row tiles of 64, 128 and 256 (y written by the GEMM); bfloat16
+SHAPES = [("pythia70m_d20", 128), ("pythia70m_d20", 300), ("pythia70m_d20", 3000), ("pythia70m_d20", 6000), ("pythia1p4b_d20_bf16", 300),
+          ("wide", 2560), ("wide_bf16", 2560)]
 IDS = [f"{name}_{n}" for name, n in SHAPES]
 
 
 @functools.lru_cache(maxsize=None)
 def _compact(name):
-    return synth.make_workload_layer(name)
+    return synth.make_workload_layer(WIDE.get(name, name))
 
 
 def _pair(name, device):
