@@ -428,9 +428,10 @@ __global__ __launch_bounds__(kDensThreads, kDensOccupancy) void prefill_prep_ker
 // past the clamp of its power of two (2^104) and (mark above) a row of only tiny entries into NaN, and the zeros of the
 // dense planes carry that to every output of the token; a weight beyond the clamp does so to its output or, through its
 // neuron's activation, to the token's every output. So the kernel that writes y sees it: an output that is not finite. Its
-// block (the split reduction: its wave) then walks that token's outputs in its columns. Calls whose outputs are finite take
-// the same time as without it (512 x 2048 at 20 %, 128 tokens: 26.6 us; 2048 x 8192 at 20 % bfloat16, 1999 tokens: 304.5);
-// a launch of its own that looked at the tokens cost 2.2 and 5.6 us.
+// wave then walks that token's outputs in its columns. Calls whose outputs are finite take
+// the same time as without it where K is split (512 x 2048 at 20 %, 128 tokens: 26.6 us; 2048 x 8192 at 20 % bfloat16, 1999
+// tokens: 304.5) and on row tiles of 64 (512 x 2048, 3000 tokens: 69.2 and 69.0), 2 us more on row tiles of 128 in one split
+// (6000 tokens: 109.5 -> 112.4); a launch of its own that looked at the tokens cost 2.2-5.6 us, a check by the whole block 1-2.
 struct Walk {
     const float* x;  // [M, d]
     const int32_t* up_off;
@@ -1281,8 +1282,7 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
         float* target = nsplit == 1 ? out : (whole_n > 0 ? part : out) + static_cast<size_t>(tile.split) * M * ld;
         const uint32_t c_end = is_y ? cols - min(cols, n0) : BN;
         const bool add_bias = EPI == Epi::Down && nsplit == 1 && bias != nullptr;  // no bias: the training gx product
-        uint32_t irregular = 0;  // bit i: in the thread's pass i (row kPassRows i + tid / (BN / 4))
-        constexpr uint32_t kPassRows = kT / (BN / 4);
+        float irregular = 0.0f;  // WALK: 0 while every output of the thread is finite, else NaN
         for (uint32_t q = tid; q < BM * (BN / 4); q += kT) {
             const uint32_t m = q / (BN / 4), c = (q % (BN / 4)) * 4;
             if (m0 + m >= M) break;  // rows ascend with q
@@ -1292,16 +1292,25 @@ __global__ __launch_bounds__(64 * kDmaWaves) void gemm_dma_kernel(
                 const float4 b = *reinterpret_cast<const float4*>(bias + n0 + c);
                 v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w;
             }
-            if constexpr (WALK) irregular |= static_cast<uint32_t>(!finite(v)) << (m / kPassRows);
+            if constexpr (WALK) irregular = fmaf(v.x, 0.0f, fmaf(v.y, 0.0f, fmaf(v.z, 0.0f, fmaf(v.w, 0.0f, irregular))));
             *reinterpret_cast<float4*>(target + static_cast<size_t>(m0 + m) * ld + c0 + c) = v;
         }
         if constexpr (WALK) {
-            constexpr uint32_t kWalkChunk = 8192;
-            static_assert(FOLD && EPI == Epi::Down && BM / kPassRows <= 32 && kWalkChunk * 4 <= S * kStage * 2, "a bit per pass; the walk's activations fit the ring");
-            if (!__syncthreads_or(static_cast<int>(irregular))) return;  // block-uniform
-            for (uint32_t m = 0; m < BM; ++m)
-                if (__syncthreads_or(static_cast<int>(irregular >> (m / kPassRows) & 1u) & static_cast<int>(tid / (BN / 4) == m % kPassRows)))
-                    irregular_row<std::conditional_t<LO_B, float, uint16_t>, kT, kWalkChunk>(walk, tile_v, m0 + m, n0, min(n0 + BN, cols), out);
+            // by the wave that stored them, beside the tile (other waves may still read it)
+            constexpr uint32_t kWalkChunk = 256, kBeside = BM * kLd, kPassRows = kT / (BN / 4), kWaveRowsStored = kWave / (BN / 4);
+            static_assert(FOLD && EPI == Epi::Down && (kBeside + W * kWalkChunk) * 4 <= S * kStage * 2, "the activations fit the ring");
+            if (__builtin_amdgcn_ballot_w64(irregular != 0.0f) == 0) return;
+            for (uint32_t i = 0; i < BM / kPassRows; ++i) {
+                const uint32_t m = m0 + i * kPassRows + tid / (BN / 4), c = tid % (BN / 4) * 4;
+                const bool odd = m < M && c < c_end && !finite(*reinterpret_cast<const float4*>(out + static_cast<size_t>(m) * cols + n0 + c));
+                for (uint32_t r = 0; r < kWaveRowsStored; ++r) {
+                    if (__builtin_amdgcn_ballot_w64(odd && lane / (BN / 4) == r) == 0) continue;
+                    for (uint32_t o = n0; o < min(n0 + BN, cols); o += kWave)
+                        irregular_row<std::conditional_t<LO_B, float, uint16_t>, kWave, kWalkChunk>(
+                            walk, tile_v + kBeside + wave * kWalkChunk, m0 + i * kPassRows + wave * kWaveRowsStored + r, o,
+                            min(min(o + kWave, n0 + BN), cols), out);
+                }
+            }
         }
     }
 }
