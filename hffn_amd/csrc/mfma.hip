@@ -2055,6 +2055,10 @@ PrefillLayout prefill_layout(bool bf16, uint32_t n, uint32_t d, uint32_t h) {
 uint64_t prefill_workspace_bytes(int vt, uint32_t n, uint32_t d, uint32_t h) { return prefill_layout(vt == kBF16, n, d, h).bytes; }
 
 namespace {
+__global__ __launch_bounds__(kThreads) void copy_kernel(const float4* __restrict__ from, float4* __restrict__ to, uint32_t quads) {
+    const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
+    if (i < quads) to[i] = from[i];
+}
 template <typename V>
 hipError_t prefill(const PrefillCall& c, hipStream_t stream) {
     constexpr bool kLoB = sizeof(V) == 4;
@@ -2090,7 +2094,18 @@ hipError_t prefill(const PrefillCall& c, hipStream_t stream) {
                                l.h, c.h);
             if (status = hipGetLastError(); status != hipSuccess) return status;
         }
-        const Walk walk{x, c.up_off, c.up_idx, c.up_val, c.b_up, c.down_off, c.down_idx, c.down_val, c.b_down, c.d, c.h};
+        // x may be the memory of y (a call on the output of the one before): the walk reads it after y is written, so it is
+        // kept where x's planes were, which nothing reads any more
+        const float* kept = x;
+        const uintptr_t x0 = reinterpret_cast<uintptr_t>(x), y0 = reinterpret_cast<uintptr_t>(y), size = static_cast<uintptr_t>(n) * c.d * 4;
+        if (x0 < y0 + size && y0 < x0 + size) {
+            float4* copy = reinterpret_cast<float4*>(w + l.x_planes);
+            const uint32_t quads = static_cast<uint32_t>(size / 16);
+            hipLaunchKernelGGL(copy_kernel, dim3(ceil_div(quads, kThreads)), dim3(kThreads), 0, stream, reinterpret_cast<const float4*>(x), copy, quads);
+            if (status = hipGetLastError(); status != hipSuccess) return status;
+            kept = reinterpret_cast<const float*>(copy);
+        }
+        const Walk walk{kept, c.up_off, c.up_idx, c.up_val, c.b_up, c.down_off, c.down_idx, c.down_val, c.b_down, c.d, c.h};
         const auto down_gemm = [&](auto walks, float* out) {
             return launch_chained<Epi::Down, kLoB, kPrefillDownChain, decltype(walks)::value>(
                 plan.down.bm, halves(l.act_planes), words(l.act_exp), down.planes, down.exps, c.b_down, out, nullptr, nullptr, n, l.d, l.h,

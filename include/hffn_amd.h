@@ -278,7 +278,8 @@ int hffn_plan_tiles_compact(int value_type, const int16_t* up_idx, const void* u
  * k (64 in the float32 up projection). d_model a multiple of 16, d_ff of 8, distinct ascending indices per row; x, y and the biases 16-byte aligned.
  * Widths need not be multiples of 256 (the planes are padded). Calls above 16384 tokens run in pieces of that size
  * over the same planes. Outputs that the planes lose (infinities, NaN, magnitudes of 2^104 and above, tokens whose every
- * entry is below 2^-100) are computed again from the compact rows: hffn_forward's results on the rows kernels. No counterpart (the reference's large-N kernels are gathers, kernels.py:87-191). */
+ * entry is below 2^-100) are computed again from the compact rows: hffn_forward's results on the rows kernels (x may overlap y:
+ * it is then copied first). No counterpart (the reference's large-N kernels are gathers, kernels.py:87-191). */
 int hffn_prefill_workspace(int value_type, uint32_t n, uint32_t d_model, uint32_t d_ff, uint64_t* bytes);
 int hffn_forward_prefill(int value_type, const float* x, const int32_t* up_offsets, const int16_t* up_idx, const void* up_val,
                          const float* b_up, const int32_t* out_offsets, const int16_t* out_hidden, const void* out_val,

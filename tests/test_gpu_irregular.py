@@ -85,6 +85,23 @@ def test_irregular_weights(name, n, side, value, device):
     torch.testing.assert_close(y[regular], expected[regular], rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("name,n", [("pythia70m_d20", 128), ("pythia70m_d20", 3000), ("pythia1p4b_d20_bf16", 300)])
+def test_irregular_tokens_of_a_call_on_its_own_output(name, n, device):
+    """x may be (a part of) the output of the call before, which the call overwrites: the results of a call on a copy."""
+    policy, rows = _pair(name, device)
+    x = _input(n + 7, policy.d_model, device)
+    for skip in (0, 7):
+        policy.forward(0, x)
+        own = policy._y[skip:skip + n]
+        own[1, 3], own[n // 2, 7], own[n - 2, 1] = float("inf"), float("nan"), 3e38
+        copy = own.clone()
+        y = policy.forward(0, own).clone()
+        assert policy.transient(n) and own.data_ptr() == policy._y.data_ptr() + 4 * skip * policy.d_model
+        assert _same(y, policy.forward(0, copy))
+        odd = [1, n // 2, n - 2]
+        assert _same(y[odd], rows.forward(0, copy)[odd])
+
+
 def test_activations_beyond_the_planes(device):
     """A pre-activation whose GELU is not finite from finite operands: only the outputs that read that neuron are lost."""
     policy, rows = _pair("pythia70m_d20", device)
