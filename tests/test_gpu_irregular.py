@@ -1,7 +1,7 @@
 """Tokens and weights that the fp16 planes of a call cannot hold (infinities, NaN, magnitudes beyond the clamp of a plane's
 power of two, tokens of only tiny entries) on calls of the policy that densify planes: they are the lane-per-token kernels'
 results (the same bits, float32 in stored slot order), and the other tokens keep theirs. Inputs with outlier columns are
-held to the float64 oracle output by output."""
+held to the float64 oracle."""
 from __future__ import annotations
 
 import functools
@@ -121,8 +121,8 @@ def test_activations_beyond_the_planes(device):
 @pytest.mark.parametrize("scale", [1e2, 1e4])
 def test_outlier_columns(name, n, scale, device):
     """A few input columns of large magnitude in every token, as deep transformer layers have them. Every operand of the
-    planes is hi + lo of at least 21 bits down to 2^-15 of its row's largest, so an output that reads no outlier keeps its
-    own precision: 1e-5 of the deviation of the tokens' outputs without outliers (the lane-per-token kernels: the same bound)."""
+    planes is hi + lo of at least 21 bits down to 2^-15 of its row's largest, so the relative error keeps its bound of 6e-7
+    (2-norm; sums in chains of at most 24 products and at most 32 chains), and is no worse than the lane-per-token kernels'."""
     policy, rows = _pair(name, device)
     layer = _compact(name)
     x = _input(n, policy.d_model, device)
@@ -133,4 +133,4 @@ def test_outlier_columns(name, n, scale, device):
     assert policy.transient(n)
     print(name, scale, {label: (float(np.linalg.norm(e) / np.linalg.norm(expected)), float(e.max() / expected.std())) for label, e in error.items()})
     assert np.linalg.norm(error["planes"]) <= 6e-7 * np.linalg.norm(expected)
-    assert np.linalg.norm(error["planes"]) <= 1.5 * np.linalg.norm(error["rows"])
+    assert np.linalg.norm(error["planes"]) <= np.linalg.norm(error["rows"])
